@@ -1793,11 +1793,13 @@ int leo2d_dos(leo2d_handle* h, const double* mu, int32_t T, int32_t M, double a,
     return guarded(h, [&]() {
         if (!(a > 0.0)) throw ArgError("energy rescale must be positive");
         hipStream_t s = h->stream;
-        DevBuf dm, de, dr;
+        DevBuf dm, de, dr, dw;
         to_device(dm, mu, sizeof(double) * (size_t)T * M, s, "moments");
         dalloc(de, sizeof(double) * M, "energies");
         dalloc(dr, sizeof(double) * (size_t)T * M, "dos");
-        check(leo2d::launch_dos((const double*)dm.p, T, M, a, b, scale, (double*)de.p, (double*)dr.p, s), "dos");
+        dalloc(dw, leo2d::dos_workspace(T, M), "dos workspace");
+        check(leo2d::launch_dos((const double*)dm.p, T, M, a, b, scale, (double*)de.p, (double*)dr.p, (double*)dw.p, s),
+              "dos");
         check(hipMemcpyAsync(rho, dr.p, sizeof(double) * (size_t)T * M, hipMemcpyDeviceToHost, s), "dos");
         if (E) check(hipMemcpyAsync(E, de.p, sizeof(double) * M, hipMemcpyDeviceToHost, s), "dos");
         check(hipStreamSynchronize(s), "dos");

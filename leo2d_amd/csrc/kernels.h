@@ -189,9 +189,11 @@ struct DgemmArgs {
 };
 hipError_t launch_dgemm(const DgemmArgs& a, hipStream_t s);
 
-// Jackson-kernel DoS: rho[t][k] = DCT-III(g * mu[t]) / (pi sqrt(a^2 - (E_k - b)^2)) * scale
+// Jackson-kernel DoS: rho[t][k] = DCT-III(g * mu[t]) / (pi sqrt(a^2 - (E_k - b)^2)) * scale;
+// work: dos_workspace(T, M) bytes of device scratch
+size_t dos_workspace(int T, int M);
 hipError_t launch_dos(const double* mu, int T, int M, double a, double b, double scale, double* E, double* rho,
-                      hipStream_t s);
+                      double* work, hipStream_t s);
 
 // Static device workspace of the allocation-free KPM entry point (scratch.hip).
 // scratch_init(d) looks up device d's address of the array (d must be current);
