@@ -71,13 +71,15 @@ hipError_t pairs_write_staged(const GeomDev& g, const int64_t* pair_rp, int32_t*
 hipError_t job_positions(const GeomDev& g, const JobDev& j, double* i2pos, hipStream_t s);
 // each orbital's local twist from its nearest neighbour on positions i2pos
 hipError_t local_theta(const GeomDev& g, const double* i2pos, double* theta, hipStream_t s);
-hipError_t fill_slots(const GeomDev& g, const JobDev& j, const double* i2pos, const int64_t* pair_rp,
-                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, const int64_t* slot_rp,
-                      int32_t* scol, double* sval, uint8_t* skeep, double* sdx, double* sdy, const double* ltheta,
+// slots inside the couplings' support per row (and each row's diagonal where the reference
+// shifts it), and their exclusive scan out_rp
+hipError_t keep_count(const GeomDev& g, const JobDev& j, const double* i2pos, const int64_t* pair_rp,
+                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, int64_t* cnt, int64_t* out_rp,
                       hipStream_t s);
-hipError_t prune_count(int n, const int64_t* slot_rp, const uint8_t* skeep, int64_t* cnt, int64_t* out_rp,
-                       hipStream_t s);
-hipError_t prune_compact(int n, int is_complex, const int64_t* slot_rp, const uint8_t* skeep, const int32_t* scol,
-                         const double* sval, const int64_t* out_rp, int32_t* ocol, double* oval, hipStream_t s);
+// columns and values of every slot (pruned: of the supported ones), row i's from out_rp[i] on;
+// odx, ody: velocity values or both nullptr; ltheta: local twists or nullptr
+hipError_t fill_slots(const GeomDev& g, const JobDev& j, bool pruned, const double* i2pos, const int64_t* pair_rp,
+                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, const int64_t* out_rp,
+                      int32_t* ocol, double* oval, double* odx, double* ody, const double* ltheta, hipStream_t s);
 
 }  // namespace leo2d

@@ -12,13 +12,13 @@
 // Geometry arithmetic is compiled without FMA contraction and the rotation
 // cosines come from the host's libm, so every keep/reject decision and window
 // origin matches the reference bit for bit.  Two passes with a device scan in
-// between: the counts, one thread per row; then the lists, one wavefront per row
+// between: the counts, one wavefront per row; then the lists, one wavefront per row
 // with the row's lists staged in LDS and the per-image sorted runs merged there
 // (rows whose lists do not fit the LDS use the thread-per-row write pass, which
 // merges through a scratch copy in global memory).
 //
-// Fill: one thread per row walks its pairs in the reference order and
-// accumulates duplicate (row, col) pairs into one slot exactly as
+// Fill: one wavefront per row, a lane per slot, duplicate (row, col) pairs
+// accumulated into their slot in the reference order exactly as
 // generateRealH / generateCpxH do (locality.cpp:3967-4316, 4664-5153):
 // intralayer values from the hopping table, interlayer values from the
 // coupling model at the job's positions, diagonal shift, rescale, Peierls and
@@ -290,17 +290,6 @@ __device__ void search_inter(const GeomDev& g, int kh, PairSink& out)
         }
 }
 
-__global__ __launch_bounds__(kThreads) void pair_count_kernel(GeomDev g, int32_t* cnt_intra, int64_t* cnt_total)
-{
-    const int kh = blockIdx.x * kThreads + threadIdx.x;
-    if (kh >= g.n) return;
-    PairSink a = {nullptr, nullptr, 0, 0}, b = {nullptr, nullptr, 0, 0};
-    search_intra(g, kh, a);
-    search_inter(g, kh, b);
-    cnt_intra[kh] = a.count;
-    cnt_total[kh] = (int64_t)a.count + b.count;
-}
-
 __device__ void sort_by_col(int32_t* col, int32_t* sc, int64_t n)
 {
     // stable insertion sort == the reference's bubble sort permutation
@@ -446,12 +435,13 @@ struct WindowWalk {
     }
 };
 
-// kept candidates of one chunk appended to a list at cnt, and counted
+// kept candidates of one chunk appended to a list at cnt, and counted (STORE = false: only counted)
+template <bool STORE>
 __device__ inline void wave_push(bool keep, int col, int dx, int dy, int lane, int32_t* lc, int32_t* ls, int cap,
                                  int& cnt)
 {
     const uint64_t m = __ballot(keep);
-    if (keep) {
+    if (STORE && keep) {
         const int pos = cnt + lanes_below(m, lane);
         if (pos < cap) {
             lc[pos] = col;
@@ -462,6 +452,7 @@ __device__ inline void wave_push(bool keep, int col, int dx, int dy, int lane, i
 }
 
 // the intralayer and interlayer candidates of row kh (search_intra, search_inter)
+template <bool STORE>
 __device__ void wave_search(const GeomDev& g, int kh, int lane, const WaveLists& L, int& n_intra, int& n_inter,
                             int& runs_intra, int& runs_inter)
 {
@@ -505,9 +496,9 @@ __device__ void wave_search(const GeomDev& g, int kh, int lane, const WaveLists&
                             col = k2 + sd.base;
                         }
                     }
-                    wave_push(keep, col, dx, dy, lane, L.col, L.sc, kPairCapIntra, cnt);
+                    wave_push<STORE>(keep, col, dx, dy, lane, L.col, L.sc, kPairCapIntra, cnt);
                 }
-                if (lane == 0 && nrun < kMaxRuns) L.run_end[nrun] = cnt;
+                if (STORE && lane == 0 && nrun < kMaxRuns) L.run_end[nrun] = cnt;
                 ++nrun;
             }
         n_intra = cnt;
@@ -564,11 +555,11 @@ __device__ void wave_search(const GeomDev& g, int kh, int lane, const WaveLists&
                                 col = (int)K;
                             }
                         }
-                        wave_push(keep, col, dx, dy, lane, L.col + kPairCapIntra, L.sc + kPairCapIntra,
+                        wave_push<STORE>(keep, col, dx, dy, lane, L.col + kPairCapIntra, L.sc + kPairCapIntra,
                                          kPairCapInter, cnt);
                     }
                 }
-                if (lane == 0 && nrun < kMaxRuns) L.run_end[kMaxRuns + 1 + nrun] = cnt;
+                if (STORE && lane == 0 && nrun < kMaxRuns) L.run_end[kMaxRuns + 1 + nrun] = cnt;
                 ++nrun;
             }
         n_inter = cnt;
@@ -630,6 +621,23 @@ __device__ int wave_place(const int32_t* lc, const int32_t* ls, const int32_t* r
     return slots;
 }
 
+// The counts: the same walk without the lists.  (One thread per orbital left a
+// small cell's search to a few wavefronts, each row's thousands of candidates in
+// sequence: 1341 us for the cells of 1-3 degrees, whatever their size.)
+__global__ __launch_bounds__(64 * kPairWaves) void pair_count_kernel(GeomDev g, int32_t* cnt_intra, int64_t* cnt_total)
+{
+    const int lane = threadIdx.x & 63;
+    const int kh = blockIdx.x * kPairWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (kh >= g.n) return;
+    WaveLists L = {nullptr, nullptr, nullptr};
+    int ni = 0, nx = 0, ri = 0, rx = 0;
+    wave_search<false>(g, kh, lane, L, ni, nx, ri, rx);
+    if (lane == 0) {
+        cnt_intra[kh] = ni;
+        cnt_total[kh] = (int64_t)ni + nx;
+    }
+}
+
 __global__ __launch_bounds__(64 * kPairWaves) void pair_write_wave_kernel(GeomDev g, const int64_t* pair_rp,
                                                                           int32_t* pcol, int32_t* psc, int64_t* nslots)
 {
@@ -642,7 +650,7 @@ __global__ __launch_bounds__(64 * kPairWaves) void pair_write_wave_kernel(GeomDe
     if (kh >= g.n) return;
     WaveLists L = {lcol[w], lsc[w], lrun[w]};
     int ni = 0, nx = 0, ri = 0, rx = 0;
-    wave_search(g, kh, lane, L, ni, nx, ri, rx);
+    wave_search<true>(g, kh, lane, L, ni, nx, ri, rx);
     const int64_t base = pair_rp[kh];
     const int sh = g.i2g[4 * (size_t)kh + 3];
     // the host runs this kernel only when every list fits and has at most kMaxRuns runs
@@ -760,164 +768,271 @@ __global__ __launch_bounds__(kThreads) void local_theta_kernel(GeomDev g, const 
     theta[k1] = th;
 }
 
-template <bool CPX>
-__global__ __launch_bounds__(kThreads) void fill_kernel(GeomDev g, JobDev j, const double* i2pos, const int64_t* pair_rp,
-                                                        const int32_t* cnt_intra, const int32_t* pcol,
-                                                        const int32_t* psc, const int64_t* slot_rp, int32_t* scol,
-                                                        double* sval, uint8_t* skeep, double* sdx, double* sdy,
-                                                        const double* ltheta)
-{
-    const int k_i = blockIdx.x * kThreads + threadIdx.x;
-    if (k_i >= g.n) return;
-    const int64_t q0 = pair_rp[k_i], q1 = pair_rp[k_i + 1];
-    const int64_t qi = q0 + cnt_intra[k_i];
-    int64_t slot = slot_rp[k_i];
-    const int s_i = g.i2g[4 * (size_t)k_i + 3];
-    const int mat = g.s[s_i].mat;
-    const int ih = g.i2g[4 * (size_t)k_i + 0], jh = g.i2g[4 * (size_t)k_i + 1], l0 = g.i2g[4 * (size_t)k_i + 2];
-    const double xi = i2pos[3 * (size_t)k_i], yi = i2pos[3 * (size_t)k_i + 1], zi = i2pos[3 * (size_t)k_i + 2];
-    const double resc = j.energy_rescale, eshift = j.energy_shift;
-    double ar = 0.0, ai = 0.0;
-    // velocity slots (sdx != nullptr): (x1 - x2) t and (y1 - y2) t, real or complex like H
-    double axr = 0.0, axi = 0.0, ayr = 0.0, ayi = 0.0;
-    bool keep = false;
-    for (int64_t q = q0; q < q1; ++q) {
-        const bool intra = q < qi;
-        const int new_k = pcol[q];
-        const int32_t scp = psc[q];
-        const int sc_i = (int)(int16_t)(scp & 0xffff), sc_j = (int)(int16_t)((uint32_t)scp >> 16);
+// What a row's pairs are evaluated with (the row's orbital and position)
+struct FillRow {
+    int k, s, mat, ih, jh, l0;
+    double x, y, z;
+    __device__ inline FillRow(const GeomDev& g, const double* i2pos, int k_) : k(k_)
+    {
+        const int* a = g.i2g + 4 * (size_t)k_;
+        ih = a[0];
+        jh = a[1];
+        l0 = a[2];
+        s = a[3];
+        mat = g.s[s].mat;
+        x = i2pos[3 * (size_t)k_];
+        y = i2pos[3 * (size_t)k_ + 1];
+        z = i2pos[3 * (size_t)k_ + 2];
+    }
+};
+
+// One pair's geometry: the row's image position (x1, y1, z1), the column's position
+struct PairGeom {
+    int sc_i, sc_j;
+    double x1, y1, z1, x2, y2, z2;
+    __device__ inline PairGeom(const GeomDev& g, const JobDev& j, const double* i2pos, const FillRow& r, int col,
+                               int32_t scp)
+    {
+        sc_i = (int)(int16_t)(scp & 0xffff);
+        sc_j = (int)(int16_t)((uint32_t)scp >> 16);
         double psx = 0.0, psy = 0.0;
         if (g.bc == 1) {
             psx = sc_i * j.sc[0][0] + sc_j * j.sc[1][0];
             psy = sc_i * j.sc[0][1] + sc_j * j.sc[1][1];
         }
-        const double x1 = xi + psx, y1 = yi + psy, z1 = zi;
-        const double x2 = i2pos[3 * (size_t)new_k], y2 = i2pos[3 * (size_t)new_k + 1], z2 = i2pos[3 * (size_t)new_k + 2];
-        double t;
-        bool support;
-        if (intra) {
-            const SheetDev& sd = g.s[s_i];
-            int gd0 = g.i2g[4 * (size_t)new_k + 0] - ih, gd1 = g.i2g[4 * (size_t)new_k + 1] - jh;
-            if (sd.bc == 1) {
-                gd0 = gd0 - sc_i * sd.st[0][0] - sc_j * sd.st[1][0];
-                gd1 = gd1 - sc_i * sd.st[0][1] - sc_j * sd.st[1][1];
-            }
-            double raw_t = intralayer(mat, l0, g.i2g[4 * (size_t)new_k + 2], gd0, gd1);
-            if (mat == MAT_STRAINED_GRAPHENE && (j.strain_type == 1 || j.strain_type == 6 || j.uniform_strain == 1)) {
-                // strained intralayer term (locality.cpp:4034-4160, 4744-4870): the hop's direction on
-                // the job's positions, the uniform strain (zero for the relaxation field), the sheet angle
-                double hx = x2 - x1, hy = y2 - y1;
-                const double hn = sqrt(hx * hx + hy * hy);
-                if (hn != 0) {
-                    hx = hx / hn;
-                    hy = hy / hn;
-                }
-                const double zero_u[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-                raw_t = strained_intra(l0, g.i2g[4 * (size_t)new_k + 2], gd0, gd1, hx, hy,
-                                       j.uniform_strain == 1 ? j.u : zero_u, sd.cneg, -sd.sneg);
-            }
-            if (mat == MAT_GRAPHENE_SIMPLE_STRAIN && raw_t != 0) {
-                const double dx = x2 - x1, dy = y2 - y1, dz = z2 - z1;
-                raw_t = raw_t * exp(-kStrainBeta * (sqrt(dx * dx + dy * dy + dz * dz) / kAcc - 1.0));
-            }
-            const bool diag = CPX ? (new_k == k_i && sc_i == 0 && sc_j == 0) : (new_k == k_i);
-            if (diag) {
-                if (j.elec_on == 1) t = (raw_t + eshift + z1 * j.E) / resc;
-                else t = (raw_t + eshift) / resc;
-            } else {
-                t = raw_t / resc;
-            }
-            support = raw_t != 0 || (diag && (eshift != 0 || j.elec_on == 1));
-        } else {
-            const int s2 = g.i2g[4 * (size_t)new_k + 3];
-            const double dx = x2 - x1, dy = y2 - y1, dz = z2 - z1;
-            // with a relaxation field, each orbital's local twist (locality.cpp:4261-4269, 5045-5052)
-            const double th1 = ltheta ? ltheta[k_i] : g.s[s_i].angle;
-            const double th2 = ltheta ? ltheta[new_k] : g.s[s2].angle;
-            t = interlayer(mat, l0, g.i2g[4 * (size_t)new_k + 2], dx, dy, dz, th1, th2) / resc;
-            support = inter_support(mat, dx, dy, dz);
+        x1 = r.x + psx;
+        y1 = r.y + psy;
+        z1 = r.z;
+        x2 = i2pos[3 * (size_t)col];
+        y2 = i2pos[3 * (size_t)col + 1];
+        z2 = i2pos[3 * (size_t)col + 2];
+    }
+};
+
+template <bool CPX>
+__device__ inline bool on_diagonal(const FillRow& r, int col, const PairGeom& p)
+{
+    return CPX ? (col == r.k && p.sc_i == 0 && p.sc_j == 0) : (col == r.k);
+}
+
+// unscaled intralayer hopping of a pair
+__device__ inline double intra_raw(const GeomDev& g, const JobDev& j, const FillRow& r, int col, const PairGeom& p)
+{
+    const SheetDev& sd = g.s[r.s];
+    const int* c = g.i2g + 4 * (size_t)col;
+    int gd0 = c[0] - r.ih, gd1 = c[1] - r.jh;
+    if (sd.bc == 1) {
+        gd0 = gd0 - p.sc_i * sd.st[0][0] - p.sc_j * sd.st[1][0];
+        gd1 = gd1 - p.sc_i * sd.st[0][1] - p.sc_j * sd.st[1][1];
+    }
+    double raw_t = intralayer(r.mat, r.l0, c[2], gd0, gd1);
+    if (r.mat == MAT_STRAINED_GRAPHENE && (j.strain_type == 1 || j.strain_type == 6 || j.uniform_strain == 1)) {
+        // strained intralayer term (locality.cpp:4034-4160, 4744-4870): the hop's direction on
+        // the job's positions, the uniform strain (zero for the relaxation field), the sheet angle
+        double hx = p.x2 - p.x1, hy = p.y2 - p.y1;
+        const double hn = sqrt(hx * hx + hy * hy);
+        if (hn != 0) {
+            hx = hx / hn;
+            hy = hy / hn;
         }
-        if (!CPX) {
-            if (t != 0) {
-                ar += t;
-                axr += (x1 - x2) * t;   // locality.cpp:4182-4183, 4299-4300
-                ayr += (y1 - y2) * t;
-            }
+        const double zero_u[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+        raw_t = strained_intra(r.l0, c[2], gd0, gd1, hx, hy, j.uniform_strain == 1 ? j.u : zero_u, sd.cneg, -sd.sneg);
+    }
+    if (r.mat == MAT_GRAPHENE_SIMPLE_STRAIN && raw_t != 0) {
+        const double dx = p.x2 - p.x1, dy = p.y2 - p.y1, dz = p.z2 - p.z1;
+        raw_t = raw_t * exp(-kStrainBeta * (sqrt(dx * dx + dy * dy + dz * dz) / kAcc - 1.0));
+    }
+    return raw_t;
+}
+
+// pruned pattern: the pair lies in its coupling's support (or shifts the diagonal)
+template <bool CPX>
+__device__ inline bool pair_support(const GeomDev& g, const JobDev& j, const double* i2pos, const FillRow& r, bool intra,
+                                    int col, int32_t scp)
+{
+    const PairGeom p(g, j, i2pos, r, col, scp);
+    if (!intra) return inter_support(r.mat, p.x2 - p.x1, p.y2 - p.y1, p.z2 - p.z1);
+    return intra_raw(g, j, r, col, p) != 0 ||
+           (on_diagonal<CPX>(r, col, p) && (j.energy_shift != 0 || j.elec_on == 1));
+}
+
+// a slot's sums: H and the velocity terms (x1 - x2) t, (y1 - y2) t, real or complex like H
+struct SlotSum {
+    double ar = 0.0, ai = 0.0, axr = 0.0, axi = 0.0, ayr = 0.0, ayi = 0.0;
+};
+
+template <bool CPX>
+__device__ inline void add_pair(const GeomDev& g, const JobDev& j, const double* i2pos, const double* ltheta,
+                                const FillRow& r, bool intra, int col, int32_t scp, SlotSum& a)
+{
+    const PairGeom p(g, j, i2pos, r, col, scp);
+    const double resc = j.energy_rescale, eshift = j.energy_shift;
+    double t;
+    if (intra) {
+        const double raw_t = intra_raw(g, j, r, col, p);
+        if (on_diagonal<CPX>(r, col, p)) {
+            if (j.elec_on == 1) t = (raw_t + eshift + p.z1 * j.E) / resc;
+            else t = (raw_t + eshift) / resc;
         } else {
-            // peierlsPhase (locality.cpp:7157-7161) and k.(r2 - r1) (locality.cpp:4896-4905)
-            double phase = 3.14e-5 * j.B * (x2 - x1) * (0.5) * (y1 + y2);
-            phase = phase + j.k[0] * (x2 - x1) + j.k[1] * (y2 - y1);
-            double sn, cs;
-            sincos(phase, &sn, &cs);
-            const double tr = t * cs, ti = t * sn;
-            if (tr != 0 || ti != 0) {
-                ar += tr;
-                ai += ti;
-                axr += (x1 - x2) * tr;   // locality.cpp:4939-4940, 5113-5114
-                axi += (x1 - x2) * ti;
-                ayr += (y1 - y2) * tr;
-                ayi += (y1 - y2) * ti;
-            }
+            t = raw_t / resc;
         }
-        keep = keep || support;
-        const bool last = (q + 1 == q1) || (q + 1 == qi) || pcol[q + 1] != new_k;
-        if (last) {
-            scol[slot] = new_k;
-            if (CPX) {
-                sval[2 * slot] = ar;
-                sval[2 * slot + 1] = ai;
-                if (sdx) {
-                    sdx[2 * slot] = axr;
-                    sdx[2 * slot + 1] = axi;
-                    sdy[2 * slot] = ayr;
-                    sdy[2 * slot + 1] = ayi;
-                }
-            } else {
-                sval[slot] = ar;
-                if (sdx) {
-                    sdx[slot] = axr;
-                    sdy[slot] = ayr;
-                }
-            }
-            skeep[slot] = keep ? 1 : 0;
-            ++slot;
-            ar = 0.0;
-            ai = 0.0;
-            axr = axi = ayr = ayi = 0.0;
-            keep = false;
+    } else {
+        const int* c = g.i2g + 4 * (size_t)col;
+        // with a relaxation field, each orbital's local twist (locality.cpp:4261-4269, 5045-5052)
+        const double th1 = ltheta ? ltheta[r.k] : g.s[r.s].angle;
+        const double th2 = ltheta ? ltheta[col] : g.s[c[3]].angle;
+        t = interlayer(r.mat, r.l0, c[2], p.x2 - p.x1, p.y2 - p.y1, p.z2 - p.z1, th1, th2) / resc;
+    }
+    if (!CPX) {
+        if (t != 0) {
+            a.ar += t;
+            a.axr += (p.x1 - p.x2) * t;   // locality.cpp:4182-4183, 4299-4300
+            a.ayr += (p.y1 - p.y2) * t;
+        }
+    } else {
+        // peierlsPhase (locality.cpp:7157-7161) and k.(r2 - r1) (locality.cpp:4896-4905)
+        double phase = 3.14e-5 * j.B * (p.x2 - p.x1) * (0.5) * (p.y1 + p.y2);
+        phase = phase + j.k[0] * (p.x2 - p.x1) + j.k[1] * (p.y2 - p.y1);
+        double sn, cs;
+        sincos(phase, &sn, &cs);
+        const double tr = t * cs, ti = t * sn;
+        if (tr != 0 || ti != 0) {
+            a.ar += tr;
+            a.ai += ti;
+            a.axr += (p.x1 - p.x2) * tr;   // locality.cpp:4939-4940, 5113-5114
+            a.axi += (p.x1 - p.x2) * ti;
+            a.ayr += (p.y1 - p.y2) * tr;
+            a.ayi += (p.y1 - p.y2) * ti;
         }
     }
 }
 
-__global__ __launch_bounds__(kThreads) void keep_count_kernel(int n, const int64_t* slot_rp, const uint8_t* skeep,
-                                                              int64_t* cnt)
+// The fill: one wavefront per row, a lane per slot.  A slot is a run of equal
+// columns inside the row's intralayer or its interlayer list; the lane at the
+// run's first pair adds the run in list order, so every slot is summed exactly
+// as the reference's walk does, and the slots are written 64 at a time, in
+// order.  The pruned pattern first counts each row's supported slots (support
+// needs comparisons only, no exponentials or phases), then evaluates only those:
+// the heads that stay are queued in LDS until 64 are there, so the lanes that
+// evaluate are full although one slot in ten stays on a bilayer of GrapheneSimple.
+//
+// What bounds it: for a small matrix the latency of a row's walk, for a large one
+// the FP64 exponentials and phases.  One thread per row (every slot evaluated and
+// written, then counted and compacted) took 986 us for the pruned Bloch matrix of
+// 8,128 orbitals and 31.1 ms for 762,112; the two passes here take 66 us and
+// 8.4 ms, and need no arrays for the dropped slots (231 million of them there).
+// The whole pattern of a 230-orbital flake: 706 us then, 18 us now.
+constexpr int kFillWaves = 4;   // rows (wavefronts) per workgroup
+
+// lane l looks at pair b + l of the row's list [q0, q1): the end of its run when it heads one, else 0
+struct RowLists {
+    int64_t q0, qi, q1;   // intralayer pairs [q0, qi), interlayer pairs [qi, q1)
+    const int32_t* pcol;
+    __device__ inline bool head(int64_t q) const
+    {
+        return q < q1 && (q == q0 || q == qi || pcol[q] != pcol[q - 1]);
+    }
+    // pairs of the run that starts at q: q .. end(q) - 1
+    __device__ inline bool more(int64_t q, int64_t p) const
+    {
+        return p < (q < qi ? qi : q1) && pcol[p] == pcol[q];
+    }
+};
+
+template <bool CPX>
+__device__ inline bool slot_support(const GeomDev& g, const JobDev& j, const double* i2pos, const FillRow& r,
+                                    const RowLists& L, const int32_t* psc, int64_t q)
 {
-    const int r = blockIdx.x * kThreads + threadIdx.x;
-    if (r >= n) return;
-    int64_t c = 0;
-    for (int64_t q = slot_rp[r]; q < slot_rp[r + 1]; ++q) c += skeep[q];
-    cnt[r] = c;
+    bool keep = false;
+    for (int64_t p = q; !keep && L.more(q, p); ++p)
+        keep = pair_support<CPX>(g, j, i2pos, r, q < L.qi, L.pcol[q], psc[p]);
+    return keep;
 }
 
 template <bool CPX>
-__global__ __launch_bounds__(kThreads) void compact_kernel(int n, const int64_t* slot_rp, const uint8_t* skeep,
-                                                           const int32_t* scol, const double* sval, const int64_t* out_rp,
-                                                           int32_t* ocol, double* oval)
+__global__ __launch_bounds__(64 * kFillWaves) void keep_count_kernel(GeomDev g, JobDev j, const double* i2pos,
+                                                                     const int64_t* pair_rp, const int32_t* cnt_intra,
+                                                                     const int32_t* pcol, const int32_t* psc,
+                                                                     int64_t* cnt)
 {
-    const int r = blockIdx.x * kThreads + threadIdx.x;
-    if (r >= n) return;
-    int64_t w = out_rp[r];
-    for (int64_t q = slot_rp[r]; q < slot_rp[r + 1]; ++q) {
-        if (!skeep[q]) continue;
-        ocol[w] = scol[q];
-        if (CPX) {
-            oval[2 * w] = sval[2 * q];
-            oval[2 * w + 1] = sval[2 * q + 1];
-        } else {
-            oval[w] = sval[q];
-        }
-        ++w;
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * kFillWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= g.n) return;
+    const FillRow r(g, i2pos, row);
+    RowLists L;
+    L.q0 = pair_rp[row];
+    L.qi = L.q0 + cnt_intra[row];
+    L.q1 = pair_rp[row + 1];
+    L.pcol = pcol;
+    int64_t c = 0;
+    for (int64_t b = L.q0; b < L.q1; b += 64) {
+        const int64_t q = b + lane;
+        const bool keep = L.head(q) && slot_support<CPX>(g, j, i2pos, r, L, psc, q);
+        c += __popcll(__ballot(keep));
     }
+    if (lane == 0) cnt[row] = c;
+}
+
+// PRUNED: only the supported slots; out_rp: first output slot of every row
+template <bool CPX, bool PRUNED>
+__global__ __launch_bounds__(64 * kFillWaves) void fill_kernel(GeomDev g, JobDev j, const double* i2pos,
+                                                               const int64_t* pair_rp, const int32_t* cnt_intra,
+                                                               const int32_t* pcol, const int32_t* psc,
+                                                               const int64_t* out_rp, int32_t* ocol, double* oval,
+                                                               double* odx, double* ody, const double* ltheta)
+{
+    __shared__ int32_t queue[kFillWaves][128];   // waiting heads, as offsets into the row's list
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = blockIdx.x * kFillWaves + wave;
+    if (row >= g.n) return;
+    int32_t* wq = queue[wave];
+    const FillRow r(g, i2pos, row);
+    RowLists L;
+    L.q0 = pair_rp[row];
+    L.qi = L.q0 + cnt_intra[row];
+    L.q1 = pair_rp[row + 1];
+    L.pcol = pcol;
+    int64_t w = out_rp[row];
+    auto emit = [&](int64_t q, int64_t slot) {
+        SlotSum a;
+        const int col = pcol[q];
+        for (int64_t p = q; L.more(q, p); ++p) add_pair<CPX>(g, j, i2pos, ltheta, r, q < L.qi, col, psc[p], a);
+        ocol[slot] = col;
+        if (CPX) {
+            reinterpret_cast<double2*>(oval)[slot] = make_double2(a.ar, a.ai);
+            if (odx) {
+                reinterpret_cast<double2*>(odx)[slot] = make_double2(a.axr, a.axi);
+                reinterpret_cast<double2*>(ody)[slot] = make_double2(a.ayr, a.ayi);
+            }
+        } else {
+            oval[slot] = a.ar;
+            if (odx) {
+                odx[slot] = a.axr;
+                ody[slot] = a.ayr;
+            }
+        }
+    };
+    int waiting = 0;
+    for (int64_t b = L.q0; b < L.q1; b += 64) {
+        const int64_t q = b + lane;
+        const bool keep = L.head(q) && (!PRUNED || slot_support<CPX>(g, j, i2pos, r, L, psc, q));
+        const uint64_t m = __ballot(keep);
+        // the queue is this wavefront's own: its LDS accesses stay in order
+        if (keep) wq[waiting + lanes_below(m, lane)] = (int32_t)(q - L.q0);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        waiting += __popcll(m);
+        if (waiting >= 64) {
+            emit(L.q0 + wq[lane], w + lane);
+            w += 64;
+            waiting -= 64;
+            const int32_t rest = wq[64 + lane];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (lane < waiting) wq[lane] = rest;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+    if (lane < waiting) emit(L.q0 + wq[lane], w + lane);
 }
 
 // exclusive scan of n int64 counts into out[0..n] (out[n] = total)
@@ -941,7 +1056,8 @@ hipError_t scan_exclusive_i64(const int64_t* cnt, int64_t* out, int n, hipStream
 
 hipError_t pairs_count(const GeomDev& g, int32_t* cnt_intra, int64_t* cnt_total, int64_t* pair_rp, hipStream_t s)
 {
-    hipLaunchKernelGGL(pair_count_kernel, rows_grid(g.n), dim3(kThreads), 0, s, g, cnt_intra, cnt_total);
+    hipLaunchKernelGGL(pair_count_kernel, dim3((unsigned)((g.n + kPairWaves - 1) / kPairWaves)), dim3(64 * kPairWaves),
+                       0, s, g, cnt_intra, cnt_total);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return scan_counts(cnt_total, pair_rp, g.n, s);
@@ -985,40 +1101,33 @@ hipError_t local_theta(const GeomDev& g, const double* i2pos, double* theta, hip
     return hipGetLastError();
 }
 
-hipError_t fill_slots(const GeomDev& g, const JobDev& j, const double* i2pos, const int64_t* pair_rp,
-                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, const int64_t* slot_rp,
-                      int32_t* scol, double* sval, uint8_t* skeep, double* sdx, double* sdy, const double* ltheta,
+hipError_t keep_count(const GeomDev& g, const JobDev& j, const double* i2pos, const int64_t* pair_rp,
+                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, int64_t* cnt, int64_t* out_rp,
                       hipStream_t s)
 {
-    if ((sdx == nullptr) != (sdy == nullptr)) return hipErrorInvalidValue;   // both velocity arrays or neither
-    if (j.complex_matrix) {
-        hipLaunchKernelGGL(fill_kernel<true>, rows_grid(g.n), dim3(kThreads), 0, s, g, j, i2pos, pair_rp, cnt_intra,
-                           pcol, psc, slot_rp, scol, sval, skeep, sdx, sdy, ltheta);
-    } else {
-        hipLaunchKernelGGL(fill_kernel<false>, rows_grid(g.n), dim3(kThreads), 0, s, g, j, i2pos, pair_rp, cnt_intra,
-                           pcol, psc, slot_rp, scol, sval, skeep, sdx, sdy, ltheta);
-    }
-    return hipGetLastError();
-}
-
-hipError_t prune_count(int n, const int64_t* slot_rp, const uint8_t* skeep, int64_t* cnt, int64_t* out_rp, hipStream_t s)
-{
-    hipLaunchKernelGGL(keep_count_kernel, rows_grid(n), dim3(kThreads), 0, s, n, slot_rp, skeep, cnt);
+    const dim3 grid((unsigned)((g.n + kFillWaves - 1) / kFillWaves)), block(64 * kFillWaves);
+    if (j.complex_matrix)
+        hipLaunchKernelGGL(keep_count_kernel<true>, grid, block, 0, s, g, j, i2pos, pair_rp, cnt_intra, pcol, psc, cnt);
+    else
+        hipLaunchKernelGGL(keep_count_kernel<false>, grid, block, 0, s, g, j, i2pos, pair_rp, cnt_intra, pcol, psc, cnt);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return scan_counts(cnt, out_rp, n, s);
+    return scan_counts(cnt, out_rp, g.n, s);
 }
 
-hipError_t prune_compact(int n, int is_complex, const int64_t* slot_rp, const uint8_t* skeep, const int32_t* scol,
-                         const double* sval, const int64_t* out_rp, int32_t* ocol, double* oval, hipStream_t s)
+hipError_t fill_slots(const GeomDev& g, const JobDev& j, bool pruned, const double* i2pos, const int64_t* pair_rp,
+                      const int32_t* cnt_intra, const int32_t* pcol, const int32_t* psc, const int64_t* out_rp,
+                      int32_t* ocol, double* oval, double* odx, double* ody, const double* ltheta, hipStream_t s)
 {
-    if (is_complex)
-        hipLaunchKernelGGL(compact_kernel<true>, rows_grid(n), dim3(kThreads), 0, s, n, slot_rp, skeep, scol, sval,
-                           out_rp, ocol, oval);
-    else
-        hipLaunchKernelGGL(compact_kernel<false>, rows_grid(n), dim3(kThreads), 0, s, n, slot_rp, skeep, scol, sval,
-                           out_rp, ocol, oval);
-    return hipGetLastError();
+    if ((odx == nullptr) != (ody == nullptr)) return hipErrorInvalidValue;   // both velocity arrays or neither
+    const dim3 grid((unsigned)((g.n + kFillWaves - 1) / kFillWaves)), block(64 * kFillWaves);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, g, j, i2pos, pair_rp, cnt_intra, pcol, psc, out_rp, ocol, oval,
+                           odx, ody, ltheta);
+        return hipGetLastError();
+    };
+    if (j.complex_matrix) return pruned ? launch(fill_kernel<true, true>) : launch(fill_kernel<true, false>);
+    return pruned ? launch(fill_kernel<false, true>) : launch(fill_kernel<false, false>);
 }
 
 }  // namespace leo2d

@@ -1157,74 +1157,41 @@ int assemble_impl(leo2d_handle* h, const leo2d_job* job, int32_t pattern, int64_
             check(leo2d::local_theta(h->gdev, (const double*)h->i2pos.p, (double*)h->ltheta.p, s), "local twist");
             lt = (const double*)h->ltheta.p;
         }
-        DevBuf scol, sval, skeep, sdx, sdy;
-        dalloc(scol, sizeof(int32_t) * (size_t)h->n_slots, "slot columns");
-        dalloc(sval, sizeof(double) * (cpx ? 2 : 1) * (size_t)h->n_slots, "slot values");
-        dalloc(skeep, (size_t)h->n_slots + 1, "slot flags");
-        if (velocity) {
-            dalloc(sdx, sizeof(double) * (cpx ? 2 : 1) * (size_t)h->n_slots, "x-velocity slots");
-            dalloc(sdy, sizeof(double) * (cpx ? 2 : 1) * (size_t)h->n_slots, "y-velocity slots");
-        }
-        check(leo2d::fill_slots(h->gdev, jd, (const double*)h->i2pos.p, (const int64_t*)h->pair_rp.p,
-                                (const int32_t*)h->cnt_intra.p, (const int32_t*)h->pcol.p, (const int32_t*)h->psc.p,
-                                (const int64_t*)h->slot_rp.p, (int32_t*)scol.p, (double*)sval.p, (uint8_t*)skeep.p,
-                                velocity ? (double*)sdx.p : nullptr, velocity ? (double*)sdy.p : nullptr, lt, s),
-              "hamiltonian fill");
-        h->rp.release();
-        h->col.release();
-        h->val.release();
-        h->val_dx.release();
-        h->val_dy.release();
-        if (pattern == LEO2D_PATTERN_REFERENCE) {
-            dalloc(h->rp, sizeof(int64_t) * (n + 1), "row pointers");
-            check(hipMemcpyAsync(h->rp.p, h->slot_rp.p, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s), "rp");
-            h->col = std::move(scol);
-            h->val = std::move(sval);
-            skeep.release();
-            set_csr_owned(h, n, h->n_slots, cpx);
-            if (velocity) {
-                h->val_dx = std::move(sdx);
-                h->val_dy = std::move(sdy);
-            }
-        } else {
+        DevBuf rp, col, val, dx, dy;   // the handle keeps its Hamiltonian until the new one is whole
+        dalloc(rp, sizeof(int64_t) * (n + 1), "row pointers");
+        int64_t nnz = h->n_slots;
+        const bool pruned = pattern == LEO2D_PATTERN_PRUNED;
+        if (pruned) {
             DevBuf cnt;
             dalloc(cnt, sizeof(int64_t) * n, "prune counts");
-            dalloc(h->rp, sizeof(int64_t) * (n + 1), "row pointers");
-            check(leo2d::prune_count(n, (const int64_t*)h->slot_rp.p, (const uint8_t*)skeep.p, (int64_t*)cnt.p,
-                                     (int64_t*)h->rp.p, s),
+            check(leo2d::keep_count(h->gdev, jd, (const double*)h->i2pos.p, (const int64_t*)h->pair_rp.p,
+                                    (const int32_t*)h->cnt_intra.p, (const int32_t*)h->pcol.p, (const int32_t*)h->psc.p,
+                                    (int64_t*)cnt.p, (int64_t*)rp.p, s),
                   "prune count");
-            int64_t kept = 0;
-            check(hipMemcpyAsync(&kept, (int64_t*)h->rp.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, s), "prune");
+            check(hipMemcpyAsync(&nnz, (int64_t*)rp.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, s), "prune");
             check(hipStreamSynchronize(s), "prune");
-            dalloc(h->col, sizeof(int32_t) * (size_t)kept, "columns");
-            dalloc(h->val, sizeof(double) * (cpx ? 2 : 1) * (size_t)kept, "values");
-            check(leo2d::prune_compact(n, cpx, (const int64_t*)h->slot_rp.p, (const uint8_t*)skeep.p,
-                                       (const int32_t*)scol.p, (const double*)sval.p, (const int64_t*)h->rp.p,
-                                       (int32_t*)h->col.p, (double*)h->val.p, s),
-                  "prune compact");
-            if (velocity) {
-                // the same compaction for the velocity slots (columns rewritten identically)
-                DevBuf* dst[2] = {&h->val_dx, &h->val_dy};
-                const DevBuf* src[2] = {&sdx, &sdy};
-                for (int c = 0; c < 2; ++c) {
-                    dalloc(*dst[c], sizeof(double) * (cpx ? 2 : 1) * (size_t)std::max<int64_t>(kept, 1),
-                           "velocity values");
-                    check(leo2d::prune_compact(n, cpx, (const int64_t*)h->slot_rp.p, (const uint8_t*)skeep.p,
-                                               (const int32_t*)scol.p, (const double*)src[c]->p,
-                                               (const int64_t*)h->rp.p, (int32_t*)h->col.p, (double*)dst[c]->p, s),
-                          "prune compact velocity");
-                }
-            }
-            check(hipStreamSynchronize(s), "prune compact");
-            cnt.release();
-            scol.release();
-            sval.release();
-            skeep.release();
-            sdx.release();
-            sdy.release();
-            set_csr_owned(h, n, kept, cpx);
+        } else {
+            check(hipMemcpyAsync(rp.p, h->slot_rp.p, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s), "rp");
         }
+        const size_t vbytes = sizeof(double) * (cpx ? 2 : 1) * (size_t)nnz;
+        dalloc(col, sizeof(int32_t) * (size_t)nnz, "columns");
+        dalloc(val, vbytes, "values");
+        if (velocity) {
+            dalloc(dx, vbytes, "x-velocity values");
+            dalloc(dy, vbytes, "y-velocity values");
+        }
+        check(leo2d::fill_slots(h->gdev, jd, pruned, (const double*)h->i2pos.p, (const int64_t*)h->pair_rp.p,
+                                (const int32_t*)h->cnt_intra.p, (const int32_t*)h->pcol.p, (const int32_t*)h->psc.p,
+                                (const int64_t*)rp.p, (int32_t*)col.p, (double*)val.p,
+                                velocity ? (double*)dx.p : nullptr, velocity ? (double*)dy.p : nullptr, lt, s),
+              "hamiltonian fill");
         check(hipStreamSynchronize(s), "assemble");
+        h->rp = std::move(rp);
+        h->col = std::move(col);
+        h->val = std::move(val);
+        h->val_dx = std::move(dx);
+        h->val_dy = std::move(dy);
+        set_csr_owned(h, n, nnz, cpx);
         h->csr_geom_order = true;
         h->has_dx = velocity;
         if (nnz_out) *nnz_out = h->nnz;
