@@ -16,7 +16,8 @@
 //
 // Two lane layouts for R < 64 vectors (both parity-tested):
 //   mode 0 ("row groups"):  64/R rows per wavefront, R lanes per row, entries
-//                           of a row walked sequentially by its lanes;
+//                           of a row walked sequentially by its lanes (4 and 8 FP64
+//                           vectors: a group of lanes per row);
 //   mode 1 ("entry slots"): one row per wavefront, 64/R entries of the row in
 //                           flight at once (lanes e, e+R, ...), folded with
 //                           cross-lane shuffles at the end of the row;
@@ -29,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.h"
 #include "kpm_common.h"
@@ -262,6 +264,93 @@ __global__ __launch_bounds__(kThreads) void batch_step_chunk_kernel(BatchStepArg
     }
 }
 
+// Mode 0 with 4 or 8 FP64 vectors: 16 lanes per matrix row (kpm_common.h), sixteen
+// wavefronts per tile, so a tile of 128 rows is two rounds of 64 rows; with a lane per
+// vector it was sixteen, each a chain of eight rounds of gathers (eight cells of 1-3
+// degrees, 4 real vectors: 13.7 -> 12.6 us a step).
+constexpr int kLaneWaves = 16;
+template <typename HT, typename XT, int R>
+__global__ __launch_bounds__(64 * kLaneWaves) void batch_step_lanes_kernel(BatchStepArgs a)
+{
+    using AT = typename acc_of<XT>::type;
+    constexpr int DUP = 16 / R;          // lanes that end with the same vector
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int l = lane & 15;
+    const int r = l / DUP;
+    const bool writer = l % DUP == 0;
+    const int G = gridDim.x;
+    const int b = blockIdx.x;
+    const int lb = (b & 7) * (G >> 3) + (b >> 3);
+
+    const HT* __restrict__ val = static_cast<const HT*>(a.val);
+    const int32_t* __restrict__ col = a.col;
+    const XT* __restrict__ cur = static_cast<const XT*>(a.cur);
+    XT* out = static_cast<XT*>(a.out);   // holds T_{j-1} on entry, T_{j+1} on exit
+    const bool beta = a.beta != 0;
+
+    __shared__ double red[kLaneWaves][R][2];
+
+    for (int t = lb; t < a.ntiles; t += G) {
+        const int row0 = a.tile_row0[t], row1 = a.tile_row0[t + 1];
+        double d1 = 0.0, d2 = 0.0;
+        for (int base = row0 + wave * 4; base < row1; base += kLaneWaves * 4) {
+            const int row = base + (lane >> 4);
+            const bool live = row < row1;
+            RowExtent e = {0, 0};
+            if (live) e = row_extent(a.row_ptr, row);
+            const size_t idx = (size_t)(live ? row : row0) * R + r;
+            const XT cv = cur[idx];
+            XT p;
+            zero(p);
+            if (beta && live) p = out[idx];
+            AT acc[R];
+#pragma unroll
+            for (int v = 0; v < R; ++v) zero(acc[v]);
+            for (int64_t q = e.q0 + kLaneEntries * l; q < e.q1; q += kLaneEntries * 16) {
+                // entries past the row's end are loaded with these and not used
+                const LaneCols lc = *reinterpret_cast<const LaneCols*>(col + q);
+                const LaneVals<HT> lv = *reinterpret_cast<const LaneVals<HT>*>(val + q);
+                const int m = (int)min((int64_t)kLaneEntries, e.q1 - q);
+                XT x[kLaneEntries][R];
+#pragma unroll
+                for (int k = 0; k < kLaneEntries; ++k)
+                    if (k < m) ld_vecs<XT, R>(x[k], cur + (size_t)lc.c[k] * R);
+#pragma unroll
+                for (int k = 0; k < kLaneEntries; ++k)
+                    if (k < m) {
+#pragma unroll
+                        for (int v = 0; v < R; ++v) mac(acc[v], lv.h[k], x[k][v]);
+                    }
+            }
+            const AT s = fold_row<16>(acc, lane);
+            if (live && writer) {
+                const XT o = comb(a.alpha, s, p);
+                out[idx] = o;
+                d1 += nrm2(cv);
+                d2 += redot(o, cv);
+            }
+        }
+        d1 += __shfl_xor(d1, 16);
+        d2 += __shfl_xor(d2, 16);
+        d1 += __shfl_xor(d1, 32);
+        d2 += __shfl_xor(d2, 32);
+        if (writer && lane < 16) {
+            red[wave][r][0] = d1;
+            red[wave][r][1] = d2;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2 * R) {
+            const int rr = threadIdx.x % R, k = threadIdx.x / R;
+            double s = red[0][rr][k];
+#pragma unroll
+            for (int w = 1; w < kLaneWaves; ++w) s += red[w][rr][k];
+            a.part[((size_t)t * R + rr) * 2 + k] = s;
+        }
+        __syncthreads();
+    }
+}
+
 // mu[p][r][.] from the tiles of job p (doubling identity from the first step):
 //   j = 0: mu_0 = <T0|T0>, mu_1 = <T1|T0>;  j >= 1: mu_2j = 2<Tj|Tj> - mu_0,
 //   mu_2j+1 = 2<Tj+1|Tj> - mu_1
@@ -269,11 +358,14 @@ __global__ __launch_bounds__(kThreads) void batch_step_chunk_kernel(BatchStepArg
 // the tiles tt = first + u + s*NS (u = t / 2R, NS = kReduceThreads / 2R) with
 // four running sums, so several loads are in flight; the strands are then
 // added in order u = 0, 1, ...  The order is fixed, so the moments are
-// deterministic.
+// deterministic.  blockIdx.y is the step: the partials of several steps are reduced
+// in one launch (a launch per step added 4-7 us to every step).
 constexpr int kReduceThreads = 256;
-__global__ __launch_bounds__(kReduceThreads) void batch_reduce_kernel(const double* part, const int32_t* job_tile0, int R,
-                                                                      int M, int j, double* mu)
+__global__ __launch_bounds__(kReduceThreads) void batch_reduce_kernel(const double* part, const int32_t* job_tile0,
+                                                                      int ntiles, int R, int M, int j0, double* mu)
 {
+    const int j = j0 + blockIdx.y;
+    part += (size_t)blockIdx.y * ntiles * R * 2;
     __shared__ double strand[kReduceThreads];
     const int p = blockIdx.x;
     const int t = threadIdx.x;
@@ -359,6 +451,12 @@ hipError_t launch_mode(const BatchStepArgs& a, hipStream_t s)
     } else {
         if (a.mode == 2) return hipErrorInvalidValue;
     }
+    if constexpr (R <= 8 && (std::is_same<XT, double>::value || std::is_same<XT, double2>::value)) {
+        if (a.mode == 0) {
+            hipLaunchKernelGGL((batch_step_lanes_kernel<HT, XT, R>), dim3(a.grid), dim3(64 * kLaneWaves), 0, s, a);
+            return hipGetLastError();
+        }
+    }
     if (a.mode == 1)
         hipLaunchKernelGGL((batch_step_kernel<HT, XT, R, 1>), dim3(a.grid), dim3(kThreads), 0, s, a);
     else
@@ -393,11 +491,12 @@ hipError_t launch_batch_step(int mat_type, int vec_type, const BatchStepArgs& a,
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_batch_reduce(const double* part, const int32_t* job_tile0, int P, int R, int M, int j, double* mu,
-                               hipStream_t s)
+hipError_t launch_batch_reduce(const double* part, const int32_t* job_tile0, int ntiles, int P, int R, int M, int j0,
+                               int steps, double* mu, hipStream_t s)
 {
-    if (P <= 0 || 2 * R > kReduceThreads) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(batch_reduce_kernel, dim3(P), dim3(kReduceThreads), 0, s, part, job_tile0, R, M, j, mu);
+    if (P <= 0 || 2 * R > kReduceThreads || steps < 1 || (j0 == 0 && steps != 1)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(batch_reduce_kernel, dim3(P, steps), dim3(kReduceThreads), 0, s, part, job_tile0, ntiles, R, M,
+                       j0, mu);
     return hipGetLastError();
 }
 

@@ -58,8 +58,9 @@ constexpr int kVariantSell = 20;
 // build for little: the vector-chunk kernel runs those.
 constexpr int kSellMinRows = 16384;
 
-// step kernel for a block of B vectors on n rows (LEO2D_KPM_VARIANT = 0, 1, 14,
-// 15 or 20 overrides the default).  In the spatial order: B = 16, 32 or 64 run
+// step kernel for a block of B vectors on n rows (LEO2D_KPM_VARIANT = 0, 1, 2, 14,
+// 15 or 20 overrides the default).  FP64 blocks of at most 8 vectors run a group of
+// lanes per row (2) in either order.  In the spatial order: B = 16, 32 or 64 run
 // the SELL-4-sigma step with LDS-staged row tiles (20) where its layout applies
 // (complex vectors) and n >= kSellMinRows, else B = 16 or 32 vector chunks split
 // over the XCDs (14).  In the natural order (or where neither applies): B >= 64
@@ -69,8 +70,9 @@ int kpm_variant(bool mixed, bool spatial, int B, int n)
 {
     if (const char* e = std::getenv("LEO2D_KPM_VARIANT")) {
         const int v = std::atoi(e);
-        if (v == 0 || v == 1 || v == 14 || v == 15 || v == kVariantSell) return v;
+        if (v == 0 || v == 1 || v == 2 || v == 14 || v == 15 || v == kVariantSell) return v;
     }
+    if (!mixed && B <= 8) return 2;
     if (spatial && (B == 16 || B == 32)) return n >= kSellMinRows ? kVariantSell : 14;
     if (spatial && B >= 64) return kVariantSell;
     return mixed && spatial ? 15 : 1;
@@ -259,9 +261,10 @@ hipEvent_t event_at(leo2d_handle* h, size_t i)
     return h->events[i];
 }
 
-void to_device(DevBuf& b, const void* src, size_t bytes, hipStream_t s, const char* what)
+// src copied to the device, with `pad` unset bytes after it
+void to_device(DevBuf& b, const void* src, size_t bytes, hipStream_t s, const char* what, size_t pad = 0)
 {
-    dalloc(b, bytes, what);
+    dalloc(b, bytes + pad, what);
     if (bytes) check(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, s), what);
 }
 
@@ -702,8 +705,8 @@ void batch_stack(leo2d_handle* h)
     const size_t vb = B.is_complex ? 16 : 8;
     DevBuf rp, col, val;
     dalloc(rp, sizeof(int64_t) * (size_t)(rows + 1), "batch row pointers");
-    dalloc(col, sizeof(int32_t) * (size_t)nnz, "batch columns");
-    dalloc(val, vb * (size_t)nnz, "batch values");
+    dalloc(col, sizeof(int32_t) * ((size_t)nnz + leo2d::kCsrPad), "batch columns");
+    dalloc(val, vb * ((size_t)nnz + leo2d::kCsrPad), "batch values");
     if (B.rows > 0) {
         check(hipMemcpyAsync(rp.p, B.rp.p, sizeof(int64_t) * (size_t)(B.rows + 1), hipMemcpyDeviceToDevice, s), "batch");
         check(hipMemcpyAsync(col.p, B.col.p, sizeof(int32_t) * (size_t)B.nnz, hipMemcpyDeviceToDevice, s), "batch");
@@ -1173,8 +1176,9 @@ int assemble_impl(leo2d_handle* h, const leo2d_job* job, int32_t pattern, int64_
         } else {
             check(hipMemcpyAsync(rp.p, h->slot_rp.p, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s), "rp");
         }
-        const size_t vbytes = sizeof(double) * (cpx ? 2 : 1) * (size_t)nnz;
-        dalloc(col, sizeof(int32_t) * (size_t)nnz, "columns");
+        const size_t padded = (size_t)nnz + leo2d::kCsrPad;
+        const size_t vbytes = sizeof(double) * (cpx ? 2 : 1) * padded;
+        dalloc(col, sizeof(int32_t) * padded, "columns");
         dalloc(val, vbytes, "values");
         if (velocity) {
             dalloc(dx, vbytes, "x-velocity values");
@@ -1277,8 +1281,8 @@ int leo2d_csr_upload(leo2d_handle* h, int32_t n, int64_t nnz, const int64_t* row
             if (!std::isfinite(val[q])) throw NanError("non-finite matrix value at entry " + std::to_string(q / w));
         hipStream_t s = h->stream;
         to_device(h->rp, row_ptr, sizeof(int64_t) * (n + 1), s, "row pointers");
-        to_device(h->col, col, sizeof(int32_t) * (size_t)nnz, s, "columns");
-        to_device(h->val, val, sizeof(double) * w * (size_t)nnz, s, "values");
+        to_device(h->col, col, sizeof(int32_t) * (size_t)nnz, s, "columns", sizeof(int32_t) * leo2d::kCsrPad);
+        to_device(h->val, val, sizeof(double) * w * (size_t)nnz, s, "values", sizeof(double) * w * leo2d::kCsrPad);
         check(hipStreamSynchronize(s), "upload");
         set_csr_owned(h, n, nnz, is_complex ? 1 : 0);
         h->csr_geom_order = false;
@@ -1343,15 +1347,22 @@ int leo2d_spectral_bounds(leo2d_handle* h, double* lo, double* hi)
 // ---- KPM --------------------------------------------------------------------
 namespace {
 
+// the lanes-per-row kernel takes a whole wavefront per row: the rows of a bilayer's pruned
+// pattern hold about 32 entries, those of the reference pattern 150 to 300
+bool long_rows(int n, int64_t nnz) { return nnz > 64 * (int64_t)n; }
+
 // workgroups of a step launch when the caller leaves the grid to the library.
 // R >= 64: four workgroups per CU (one wavefront per row); fewer rows in flight
 // keep each XCD's gathered rows in its L2 (measured best on the 1.05 deg 8x8
-// cell: 1.66 ms per FP64 step at 1024 vs 1.79 ms at 2048)
-int auto_grid(int n, int B)
+// cell: 1.66 ms per FP64 step at 1024 vs 1.79 ms at 2048).  The lanes-per-row
+// kernel (2): four wavefronts' rows per workgroup and iteration, up to four workgroups
+// per CU (95 k rows, 4 real vectors: 15.9 us at 1024, 17.6 at 2048, 21.6 at 512).
+int auto_grid(int variant, int n, int64_t nnz, int B)
 {
-    const int rows_per_iter = std::max(1, 256 / B);   // 4 wavefronts x 64/B rows
+    int rows_per_iter = std::max(1, 256 / B);   // 4 wavefronts x 64/B rows
+    if (variant == 2) rows_per_iter = long_rows(n, nnz) ? 4 : 16;
     const int want = (n + rows_per_iter - 1) / rows_per_iter;
-    return std::min(B >= 64 ? 1024 : 2048, std::max(8, (want + 7) / 8 * 8));
+    return std::min(B >= 64 || variant == 2 ? 1024 : 2048, std::max(8, (want + 7) / 8 * 8));
 }
 
 // moments of a spectrum inside [-1, 1] are finite and satisfy |mu_n| <= mu_0
@@ -1393,6 +1404,38 @@ void check_kpm_params(const leo2d_handle* h, const leo2d_kpm_params* p)
     const int B = p->block ? p->block : std::min(64, next_pow2(R));
     if (B < 1 || B > 128 || (B & (B - 1))) throw ArgError("block must be a power of two <= 128");
 }
+
+// Where the steps of a recursion leave their partial sums, and the launches that
+// reduce them: step 0 by itself (the later moments need mu_0 and mu_1), then every
+// `every` steps and after the last.  The partials of a step are overwritten only by
+// steps queued after their reduction.
+struct MomentSink {
+    int scheme, grid, R, M, every;
+    double* space;     // [every][grid][R][3]
+    double* mu;        // [R][M]
+    hipStream_t s;
+    int first = 0;     // first step not reduced yet
+
+    double* part(int j) const { return space + (size_t)(j - first) * grid * R * 3; }
+    // target starts of the reference scheme: T_j's target values are the moments j < M/2
+    double* tval(int j) const { return scheme == 0 ? mu + j : nullptr; }
+    void done(int j)
+    {
+        const int steps = j + 1 - first;
+        if (j != 0 && steps < every && j + 1 < M / 2) return;
+        leo2d::ReduceArgs ra{};
+        ra.part = space;
+        ra.grid = grid;
+        ra.R = R;
+        ra.M = M;
+        ra.j0 = first;
+        ra.steps = steps;
+        ra.scheme = scheme;
+        ra.mu = mu;
+        check(leo2d::launch_kpm_reduce(ra, s), "kpm reduce");
+        first = j + 1;
+    }
+};
 
 }  // namespace
 
@@ -1449,14 +1492,15 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
         if (p->scheme == LEO2D_SCHEME_DOUBLING) dev_scheme = 1;
         else dev_scheme = p->start == LEO2D_START_TARGETS ? 0 : 2;
         const bool keep_v = dev_scheme == 2;
-        const int G = p->grid > 0 ? p->grid : auto_grid(n, B);
+        const int wanted = kpm_variant(mixed, spatial, B, n);
+        const int G = p->grid > 0 ? p->grid : auto_grid(wanted, n, h->nnz, B);
         if (G % 8 != 0) throw ArgError("grid must be a multiple of 8");
         const size_t vb = leo2d::vec_bytes(vec_type);
         DevBuf A, Bf, V, part, dmu, dtg, host_v;
         dalloc(A, vb * (size_t)n * B, "vector block");
         dalloc(Bf, vb * (size_t)n * B, "vector block");
         if (keep_v) dalloc(V, vb * (size_t)n * B, "start vectors");
-        dalloc(part, sizeof(double) * 3 * (size_t)G * B, "partials");
+        dalloc(part, std::max(sizeof(double) * 3 * (size_t)G * B, leo2d::kPartialSpace), "partials");
         dalloc(dmu, sizeof(double) * (size_t)M * B, "moments");
         dalloc(dtg, sizeof(int32_t) * B, "targets");
         std::vector<double> hv;
@@ -1500,7 +1544,8 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
             sa.part = (double*)part.p;
             sa.grid = G;
             sa.v = keep_v ? V.p : nullptr;
-            sa.variant = kpm_variant(mixed, spatial, B, n);
+            sa.variant = wanted;
+            sa.long_rows = long_rows(n, h->nnz) ? 1 : 0;
             sa.xcd_rows = kpm_sched() == 1 ? (n + 7) / 8 : 0;
             leo2d::SellStepArgs ss{};
             const bool sell_alternate = env_int("LEO2D_SELL_ALTERNATE", 1) != 0;
@@ -1549,17 +1594,13 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
             }
             if (sa.variant == 14 && B != 16 && B != 32 && B != 64 && B != 128) sa.variant = 1;
             if (sa.variant == 15 && (!spatial || B != 64 || vec_type != leo2d::VEC_CPX_F32)) sa.variant = 1;
-            if (B < 64 && sa.variant != 14 && sa.variant != kVariantSell) sa.variant = 0;
+            if (sa.variant == 2 && (mixed || B > 8)) sa.variant = B >= 64 ? 1 : 0;
+            if (B < 64 && sa.variant != 2 && sa.variant != 14 && sa.variant != kVariantSell) sa.variant = 0;
             kernel_used = sa.variant == kVariantSell && ss.copy_wave ? kVariantSell + 1 : sa.variant;
-            leo2d::ReduceArgs ra{};
-            ra.part = (const double*)part.p;
-            ra.grid = sa.grid;
-            ra.R = B;
-            ra.M = M;
-            ra.scheme = dev_scheme;
-            ra.targets = (const int32_t*)dtg.p;
-            ra.vec_type = vec_type;
-            ra.mu = (double*)dmu.p;
+            const int every = leo2d::reduce_every(sizeof(double) * 3 * (size_t)sa.grid * B, part.bytes, M);
+            MomentSink sink{dev_scheme, sa.grid, B, M, every, (double*)part.p, (double*)dmu.p, s};
+            sa.targets = (const int32_t*)dtg.p;
+            sa.tstride = M;
             check(hipEventRecord(e0, s), "event");
             for (int j = 0; j < M / 2; ++j) {
                 void* cur = (j % 2 == 0) ? A.p : Bf.p;
@@ -1569,6 +1610,8 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                 sa.out = other;
                 sa.alpha = j == 0 ? 1.0 : 2.0;
                 sa.beta = j == 0 ? 0 : 1;
+                sa.part = sink.part(j);
+                sa.tval = sink.tval(j);
                 if (p->time_steps) check(hipEventRecord(event_at(h, 2 + 2 * (size_t)j), s), "event");
                 if (sa.variant == kVariantSell) {
                     ss.cur = sa.cur;
@@ -1576,16 +1619,17 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                     ss.out = sa.out;
                     ss.alpha = sa.alpha;
                     ss.beta = sa.beta;
+                    ss.part = sa.part;
                     ss.reverse = sell_alternate && (j & 1);
                     check(leo2d::launch_kpm_step_sell(mat_type, vec_type, ss, s), "kpm step");
+                    if (sa.tval)
+                        check(leo2d::launch_target_values(cur, vec_type, sa.targets, B, sa.tval, sa.tstride, s),
+                              "target values");
                 } else {
                     check(leo2d::launch_kpm_step(mat_type, vec_type, sa, s), "kpm step");
                 }
                 if (p->time_steps) check(hipEventRecord(event_at(h, 3 + 2 * (size_t)j), s), "event");
-                ra.j = j;
-                ra.cur = cur;
-                ra.out = other;
-                check(leo2d::launch_kpm_reduce(ra, s), "kpm reduce");
+                sink.done(j);
             }
             check(hipEventRecord(e1, s), "event");
             check(hipStreamSynchronize(s), "kpm recursion");
@@ -1635,10 +1679,17 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
         if (!base) throw StateError("static device scratch not initialised on this device");
         const int M = p->M, R = p->R, n = h->n;
         const int B = p->block ? p->block : std::min(64, next_pow2(R));
-        const int G = p->grid > 0 ? p->grid : auto_grid(n, B);
-        if (G % 8 != 0) throw ArgError("grid must be a multiple of 8");
+        // the kernel leo2d_kpm_moments picks for the reference row order in FP64
+        int variant = kpm_variant(false, false, B, n);
         const bool real_vec = !h->is_complex && (p->start == LEO2D_START_TARGETS ||
-                                                 (p->start == LEO2D_START_VECTORS && !p->vectors_complex));
+                                                   (p->start == LEO2D_START_VECTORS && !p->vectors_complex));
+        int G = p->grid > 0 ? p->grid : auto_grid(variant, n, h->nnz, B);
+        if (variant == kVariantSell) variant = B == 16 || B == 32 ? 14 : 1;
+        if (variant == 14 && B != 16 && B != 32 && B != 64 && B != 128) variant = 1;
+        if (variant == 15) variant = 1;
+        if (variant == 2 && B > 8) variant = B >= 64 ? 1 : 0;
+        if (B < 64 && variant != 2 && variant != 14) variant = 0;
+        if (G % 8 != 0) throw ArgError("grid must be a multiple of 8");
         if (real_vec && p->start == LEO2D_START_RANDOM_PHASE) throw ArgError("random phases need complex vectors");
         const int mat_type = h->is_complex ? leo2d::MAT_CPX_F64 : leo2d::MAT_REAL_F64;
         const int vec_type = real_vec ? leo2d::VEC_REAL_F64 : leo2d::VEC_CPX_F64;
@@ -1660,14 +1711,21 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
         const size_t oA = take(block_bytes), oB = take(block_bytes);
         const size_t oV = keep_v ? take(block_bytes) : 0;
         const size_t oStage = p->start == LEO2D_START_VECTORS ? take(sizeof(double) * (size_t)w * n * B) : 0;
-        const size_t oPart = take(sizeof(double) * 3 * (size_t)G * B);
         const size_t oMu = take(sizeof(double) * (size_t)M * B);
         const size_t oTg = take(sizeof(int32_t) * (size_t)B);
+        // a request that only just fits takes fewer workgroups (and partials) than leo2d_kpm_moments
+        // would, down to the eight of a small matrix's lane-per-vector launch
+        auto part_bytes = [&]() { return (sizeof(double) * 3 * (size_t)G * B + 255) / 256 * 256; };
+        while (p->grid == 0 && variant == 2 && G > 8 && off + part_bytes() > leo2d::kScratchBytes) G = G / 16 * 8;
+        const size_t part_step = sizeof(double) * 3 * (size_t)G * B;
+        const size_t oPart = take(part_step);
         if (off > leo2d::kScratchBytes)
             throw ArgError("leo2d_kpm_moments_noalloc needs " + std::to_string(off) + " bytes of workspace for n = " +
                            std::to_string(n) + ", block = " + std::to_string(B) + ", M = " + std::to_string(M) +
                            "; the static scratch holds " + std::to_string(leo2d::kScratchBytes) +
                            " (use leo2d_kpm_moments)");
+        // the partials of further steps take what is left
+        const int every = leo2d::reduce_every(part_step, part_step + (leo2d::kScratchBytes - off), M);
         void* A = base + oA;
         void* Bf = base + oB;
         void* V = keep_v ? base + oV : nullptr;
@@ -1675,13 +1733,6 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
         double* part = reinterpret_cast<double*>(base + oPart);
         double* dmu = reinterpret_cast<double*>(base + oMu);
         int32_t* dtg = reinterpret_cast<int32_t*>(base + oTg);
-
-        // the kernel leo2d_kpm_moments picks for the reference row order in FP64
-        int variant = kpm_variant(false, false, B, n);
-        if (variant == kVariantSell) variant = B == 16 || B == 32 ? 14 : 1;
-        if (variant == 14 && B != 16 && B != 32 && B != 64 && B != 128) variant = 1;
-        if (variant == 15) variant = 1;
-        if (B < 64 && variant != 14) variant = 0;
 
         hipStream_t s = h->stream;
         for (int b0 = 0; b0 < R; b0 += B) {
@@ -1714,16 +1765,11 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
             sa.grid = G;
             sa.v = V;
             sa.variant = variant;
+            sa.long_rows = long_rows(n, h->nnz) ? 1 : 0;
             sa.xcd_rows = kpm_sched() == 1 ? (n + 7) / 8 : 0;
-            leo2d::ReduceArgs ra{};
-            ra.part = part;
-            ra.grid = G;
-            ra.R = B;
-            ra.M = M;
-            ra.scheme = dev_scheme;
-            ra.targets = dtg;
-            ra.vec_type = vec_type;
-            ra.mu = dmu;
+            MomentSink sink{dev_scheme, G, B, M, every, part, dmu, s};
+            sa.targets = dtg;
+            sa.tstride = M;
             for (int j = 0; j < M / 2; ++j) {
                 void* cur = (j % 2 == 0) ? A : Bf;
                 void* other = (j % 2 == 0) ? Bf : A;
@@ -1732,11 +1778,10 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
                 sa.out = other;
                 sa.alpha = j == 0 ? 1.0 : 2.0;
                 sa.beta = j == 0 ? 0 : 1;
+                sa.part = sink.part(j);
+                sa.tval = sink.tval(j);
                 check(leo2d::launch_kpm_step(mat_type, vec_type, sa, s), "kpm step");
-                ra.j = j;
-                ra.cur = cur;
-                ra.out = other;
-                check(leo2d::launch_kpm_reduce(ra, s), "kpm reduce");
+                sink.done(j);
             }
             check(hipMemcpyAsync(mu + (size_t)M * b0, dmu, sizeof(double) * (size_t)M * Rb, hipMemcpyDeviceToHost, s),
                   "moments");
@@ -2104,7 +2149,10 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
         if (sell_ok) max_tiles = std::max<int64_t>(max_tiles, B.sell.ntiles);
         ensure(B.A, vbytes, "batch vectors");
         ensure(B.B, vbytes, "batch vectors");
-        ensure(B.part, sizeof(double) * 2 * (size_t)std::max<int64_t>(max_tiles, 1) * R, "batch partials");
+        // partials of one step under any tiling, or of as many steps as kBatchPartialSpace holds
+        const size_t part_max = sizeof(double) * 2 * (size_t)std::max<int64_t>(max_tiles, 1) * R;
+        const size_t part_space = part_max * (size_t)leo2d::reduce_every(part_max, leo2d::kBatchPartialSpace, M);
+        ensure(B.part, part_space, "batch partials");
         ensure(B.mu, sizeof(double) * (size_t)P * R * M, "batch moments");
 
         leo2d::BatchStepArgs sa{};
@@ -2257,12 +2305,21 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
         auto record = [&]() {
             check(leo2d::launch_batch_init(B.A.p, vec_type, (const int64_t*)B.drow0.p, P, B.rows, R, p->seed, dtargets, s),
                   "batch init");
+            // the partials of `every` steps are reduced together (step 0 by itself)
+            const int ntiles = sa.mode == LEO2D_BATCH_SELL ? ss.ntiles : sa.ntiles;
+            const size_t part_step = 2 * (size_t)ntiles * R;
+            const int every = leo2d::reduce_every(sizeof(double) * part_step, part_space, M);
+            int first = 0;
             for (int j = 0; j < M / 2; ++j) {
                 void* cur = (j % 2 == 0) ? B.A.p : B.B.p;
                 void* other = (j % 2 == 0) ? B.B.p : B.A.p;
+                sa.part = ss.part = (double*)B.part.p + (size_t)(j - first) * part_step;
                 step(cur, other, j);
-                check(leo2d::launch_batch_reduce((const double*)B.part.p, job_tiles, P, R, M, j, (double*)B.mu.p, s),
+                if (j != 0 && j + 1 - first < every && j + 1 < M / 2) continue;
+                check(leo2d::launch_batch_reduce((const double*)B.part.p, job_tiles, ntiles, P, R, M, first, j + 1 - first,
+                                                 (double*)B.mu.p, s),
                       "batch reduce");
+                first = j + 1;
             }
         };
         if (p->graph) {

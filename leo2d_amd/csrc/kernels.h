@@ -32,14 +32,20 @@ struct StepArgs {
     double alpha;
     int beta;
     double* part;   // [grid][R][3]
+    const int32_t* targets;   // with tval: the row of each vector's unit start vector
+    double* tval;             // tval[r tstride] <- Re cur[targets[r]][r] (nullptr: not wanted)
+    int tstride;
     int grid;       // number of workgroups (multiple of 8)
-    int variant;    // 0 = lane per vector (any R), 1 = wavefront per row (R >= 64), 14 = vector chunks split
+    int variant;    // 0 = lane per vector (any R), 1 = wavefront per row (R >= 64), 2 = group of lanes per row
+                    // (FP64, R <= 8), 14 = vector chunks split
                     // over the XCDs (R = 16, 32, 64, 128), 15 = two rows per wavefront, 16-byte FP32 gathers
                     // (complex FP32, R = 64)
+    int long_rows;  // variant 2: 1 = a wavefront per row (rows of more than 64 entries on average)
     int xcd_rows;   // variant 1: rows per XCD slice (0 = interleave rows over the grid)
 };
 
-// trailing (column 0, value 0) entries after nnz in the spatially ordered CSR
+// entries allocated after nnz in every device CSR, so kernels may load whole chunks of a row
+// (column 0 and value 0 in the spatially ordered CSR, unset elsewhere)
 constexpr int kCsrPad = 16;
 hipError_t launch_kpm_step(int mat_type, int vec_type, const StepArgs& a, hipStream_t s);
 
@@ -90,25 +96,40 @@ hipError_t launch_kpm_step_sell(int mat_type, int vec_type, const SellStepArgs& 
 hipError_t launch_sell_fill(const int64_t* map, const void* src, void* dst, int elem_bytes, int64_t count,
                             hipStream_t s);
 
-// Deterministic reduction of the partials of one step into moments.
-//   scheme 0 (reference, target starts): mu_j = Re cur[target_r][r] for
-//            2 <= j < M/2, dots used for j >= M/4 (locality.cpp:6002-6034)
+// Deterministic reduction of the partials of `steps` consecutive steps from j0 on
+// into moments (step 0 in a launch of its own: the others read its moments).
+//   scheme 0 (reference, target starts): mu_j = Re T_j[target_r][r] for j < M/2 is
+//            written by the steps themselves (tval = mu + j); dots for j >= M/4
+//            (locality.cpp:6002-6034)
 //   scheme 1 (doubling from j = 1): mu_{2j}, mu_{2j+1} from the dots
 //   scheme 2 (reference, vector starts): mu_j = part[..][2] for j < M/2
 struct ReduceArgs {
-    const double* part;
+    const double* part;      // [steps][grid][R][3]
     int grid;
     int R;
     int M;
-    int j;          // step index (0 = first product T1 = H T0)
+    int j0;                  // first step (step 0 = the product T1 = H T0)
+    int steps;
     int scheme;
-    const int32_t* targets;  // [R] (scheme 0)
-    const void* cur;         // T_j   (scheme 0, j >= 2)
-    const void* out;         // T_j+1 (scheme 0, j == 0)
-    int vec_type;
     double* mu;              // [R][M] device
 };
+// steps whose partials a recursion collects before it reduces them, for partials of step_bytes
+// a step in `space` bytes
+inline int reduce_every(size_t step_bytes, size_t space, int M)
+{
+    const size_t k = space / (step_bytes ? step_bytes : 1);
+    const size_t most = (size_t)(M / 2);
+    return (int)(k < 1 ? 1 : (k < most ? k : most));
+}
+// Partials kept before a reduction: 10 to 20 steps of a full grid, so a reduction's launch is a
+// small part of a step.  (32 MiB allocated and freed by every call cost as much as it saved.)
+constexpr size_t kPartialSpace = size_t(4) << 20;
+// The same for a batch, whose buffers stay with the handle between calls.
+constexpr size_t kBatchPartialSpace = size_t(32) << 20;
 hipError_t launch_kpm_reduce(const ReduceArgs& a, hipStream_t s);
+// tval[r tstride] <- Re cur[targets[r]][r], for steps that do not write it themselves (the SELL step)
+hipError_t launch_target_values(const void* cur, int vec_type, const int32_t* targets, int R, double* tval, int tstride,
+                                hipStream_t s);
 
 // ---- batched recursion over many stacked Hamiltonians (batch.hip) ----------
 // One step for every job of a block-diagonal stack: out = alpha*H*cur - (beta ?
@@ -130,9 +151,10 @@ struct BatchStepArgs {
     int mode;                  // 0 = row groups, 1 = entry slots, 2 = row chunks (R = 16, 32)
 };
 hipError_t launch_batch_step(int mat_type, int vec_type, const BatchStepArgs& a, hipStream_t s);
-// mu[p][r][M] of job p from its tiles [job_tile0[p], job_tile0[p+1]) (doubling identity)
-hipError_t launch_batch_reduce(const double* part, const int32_t* job_tile0, int P, int R, int M, int j, double* mu,
-                               hipStream_t s);
+// mu[p][r][M] of job p from its tiles [job_tile0[p], job_tile0[p+1]) (doubling identity), for `steps`
+// steps from j0 on with partials part[step][ntiles][R][2]; step 0 in a launch of its own
+hipError_t launch_batch_reduce(const double* part, const int32_t* job_tile0, int ntiles, int P, int R, int M, int j0,
+                               int steps, double* mu, hipStream_t s);
 // start vectors: random phases (vector r of job p = global vector p*R + r), or,
 // when targets != nullptr, the unit vector on orbital targets[p*R + r] of job p
 hipError_t launch_batch_init(void* x, int vec_type, const int64_t* job_row0, int P, int64_t nrows, int R, uint64_t seed,

@@ -112,6 +112,7 @@ __global__ __launch_bounds__(kThreads) void kpm_step_kernel(StepArgs a)
             else zero(p);
             const XT o = comb(alpha, acc[v], p);
             out[idx] = o;
+            if (a.tval && row == a.targets[r0 + v * LPR]) a.tval[(r0 + v * LPR) * a.tstride] = re(c);
             d1[v] += nrm2(c);
             d2[v] += redot(o, c);
             if (direct) d3[v] += redot(vin[idx], c);
@@ -282,6 +283,7 @@ __global__ __launch_bounds__(kThreads) void kpm_step_wave_kernel(StepArgs a)
             else zero(p);
             const XT o = comb(alpha, acc[v], p);
             out[idx] = o;
+            if (a.tval && row == a.targets[lane + 64 * v]) a.tval[(lane + 64 * v) * a.tstride] = re(c);
             d1[v] += nrm2(c);
             d2[v] += redot(o, c);
             if (direct) d3[v] += redot(vin[idx], c);
@@ -304,6 +306,104 @@ __global__ __launch_bounds__(kThreads) void kpm_step_wave_kernel(StepArgs a)
 #pragma unroll
         for (int w = 1; w < NW; ++w) s += red[w][r][k];
         a.part[((size_t)lb * R + r) * 3 + k] = s;
+    }
+}
+
+// ---- variant 2: a group of lanes per row, for blocks of at most 8 vectors ----------
+// The lane-per-vector kernel gives a row of B = 4 vectors four lanes, which walk its
+// entries four at a time: every load moves 32 bytes a row and the row's gathers come
+// one batch after another.  Here a group of LPR lanes takes a row, three entries a
+// lane (kpm_common.h), so a row's entries and then its gathers are in flight together.
+// A workgroup owns consecutive rows, the same at every step.
+// FP64 only: the fold is not the CSR order, which the FP32 recursion keeps.
+template <typename HT, typename XT, int B, int LPR>
+__global__ __launch_bounds__(kThreads) void kpm_step_lanes_kernel(StepArgs a)
+{
+    using AT = typename acc_of<XT>::type;
+    constexpr int SL = 64 / LPR;           // rows per wavefront
+    constexpr int RPI = SL * kWaves;       // rows per workgroup iteration
+    constexpr int DUP = 16 / B;            // lanes that end with the same vector
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int l = lane % LPR;
+    const int b = (lane & 15) / DUP;
+    const bool writer = (lane & 15) % DUP == 0 && l < 16;
+    const int G = gridDim.x;
+    const int blk = blockIdx.x;
+    const int lb = (blk & 7) * (G >> 3) + (blk >> 3);
+    const int iters = (a.n + RPI - 1) / RPI;
+    const int it0 = (int)((int64_t)iters * lb / G), it1 = (int)((int64_t)iters * (lb + 1) / G);
+
+    const HT* __restrict__ val = static_cast<const HT*>(a.val);
+    const int32_t* __restrict__ col = a.col;
+    const XT* __restrict__ cur = static_cast<const XT*>(a.cur);
+    const XT* prev = static_cast<const XT*>(a.prev);
+    XT* out = static_cast<XT*>(a.out);
+    const XT* __restrict__ vin = static_cast<const XT*>(a.v);
+    const bool beta = a.beta != 0;
+    const int target = a.tval ? a.targets[b] : -1;
+
+    double d1 = 0.0, d2 = 0.0, d3 = 0.0;
+    for (int it = it0; it < it1; ++it) {
+        const int row = it * RPI + wave * SL + lane / LPR;
+        const bool live = row < a.n;
+        RowExtent e = {0, 0};
+        if (live) e = row_extent(a.row_ptr, row);
+        const size_t idx = (size_t)(live ? row : 0) * B + b;
+        const XT c = cur[idx];
+        XT p;
+        zero(p);
+        if (beta && live) p = prev[idx];
+        AT acc[B];
+#pragma unroll
+        for (int v = 0; v < B; ++v) zero(acc[v]);
+        for (int64_t q = e.q0 + kLaneEntries * l; q < e.q1; q += kLaneEntries * LPR) {
+            // entries past the row's end are loaded with these and not used
+            const LaneCols lc = *reinterpret_cast<const LaneCols*>(col + q);
+            const LaneVals<HT> lv = *reinterpret_cast<const LaneVals<HT>*>(val + q);
+            const int m = (int)min((int64_t)kLaneEntries, e.q1 - q);
+            XT x[kLaneEntries][B];
+#pragma unroll
+            for (int k = 0; k < kLaneEntries; ++k)
+                if (k < m) ld_vecs<XT, B>(x[k], cur + (size_t)lc.c[k] * B);
+#pragma unroll
+            for (int k = 0; k < kLaneEntries; ++k)
+                if (k < m) {
+#pragma unroll
+                    for (int v = 0; v < B; ++v) mac(acc[v], lv.h[k], x[k][v]);
+                }
+        }
+        const AT t = fold_row<LPR>(acc, lane);
+        if (live && writer) {
+            const XT o = comb(a.alpha, t, p);
+            out[idx] = o;
+            if (row == target) a.tval[b * a.tstride] = re(c);
+            d1 += nrm2(c);
+            d2 += redot(o, c);
+            if (vin) d3 += redot(vin[idx], c);
+        }
+    }
+    if constexpr (LPR == 16) {
+        d1 += __shfl_xor(d1, 16);
+        d2 += __shfl_xor(d2, 16);
+        d3 += __shfl_xor(d3, 16);
+        d1 += __shfl_xor(d1, 32);
+        d2 += __shfl_xor(d2, 32);
+        d3 += __shfl_xor(d3, 32);
+    }
+    __shared__ double red[kWaves][B][3];
+    if (writer && lane < 16) {
+        red[wave][b][0] = d1;
+        red[wave][b][1] = d2;
+        red[wave][b][2] = d3;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 * B) {
+        const int r = threadIdx.x / 3, k = threadIdx.x % 3;
+        double s = red[0][r][k];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) s += red[w][r][k];
+        a.part[((size_t)lb * B + r) * 3 + k] = s;
     }
 }
 
@@ -433,6 +533,7 @@ __global__ __launch_bounds__(kThreads) void kpm_step_xchunk_kernel(StepArgs a)
             const XT c = own_c;
             const XT o = comb(alpha, acc, own_p);
             out[idx] = o;
+            if (a.tval && row == a.targets[voff]) a.tval[voff * a.tstride] = re(c);
             d1 += nrm2(c);
             d2 += redot(o, c);
             if (direct) d3 += redot(vin[idx], c);
@@ -509,7 +610,9 @@ __global__ __launch_bounds__(kThreads) void kpm_step_pair_kernel(const int64_t* 
                                                                  const float4* __restrict__ cur,
                                                                  float4* __restrict__ po,
                                                                  const float4* __restrict__ vin, int nrows,
-                                                                 double alpha, int beta, double* __restrict__ part)
+                                                                 double alpha, int beta, double* __restrict__ part,
+                                                                 const int32_t* __restrict__ targets, double* tval,
+                                                                 int tstride)
 {
     constexpr int R = 64;
     constexpr int RQ = R / 2;             // float4 per row
@@ -599,6 +702,10 @@ __global__ __launch_bounds__(kThreads) void kpm_step_pair_kernel(const int64_t* 
             o1.x = al * a1.x - op.z;
             o1.y = al * a1.y - op.w;
             po[own] = make_float4(o0.x, o0.y, o1.x, o1.y);
+            if (tval) {
+                if (row == targets[2 * hl]) tval[2 * hl * tstride] = c0.x;
+                if (row == targets[2 * hl + 1]) tval[(2 * hl + 1) * tstride] = c1.x;
+            }
             d1a += nrm2(c0);
             d1b += nrm2(c1);
             d2a += redot(o0, c0);
@@ -644,6 +751,17 @@ __global__ __launch_bounds__(kThreads) void kpm_step_pair_kernel(const int64_t* 
 template <typename HT, typename XT, int LPR, int VPL>
 hipError_t launch_typed(const StepArgs& a, hipStream_t s)
 {
+    if (a.variant == 2) {
+        if constexpr (LPR <= 8 && VPL == 1 &&
+                      (std::is_same<XT, double>::value || std::is_same<XT, double2>::value)) {
+            if (a.long_rows)
+                hipLaunchKernelGGL((kpm_step_lanes_kernel<HT, XT, LPR, 64>), dim3(a.grid), dim3(kThreads), 0, s, a);
+            else
+                hipLaunchKernelGGL((kpm_step_lanes_kernel<HT, XT, LPR, 16>), dim3(a.grid), dim3(kThreads), 0, s, a);
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
+    }
     if (a.variant == 14) return launch_xchunk<HT, XT>(a, s);
     if constexpr (std::is_same<XT, float2>::value && sizeof(HT) <= 8) {
         if (a.variant == 15) {
@@ -652,7 +770,7 @@ hipError_t launch_typed(const StepArgs& a, hipStream_t s)
             hipLaunchKernelGGL((kpm_step_pair_kernel<HT, 8>), dim3(a.grid), dim3(kThreads), 0, s, a.row_ptr, a.col,
                                static_cast<const HT*>(a.val), static_cast<const float4*>(a.cur),
                                static_cast<float4*>(a.out), static_cast<const float4*>(a.v), a.n, a.alpha, a.beta,
-                               a.part);
+                               a.part, a.targets, a.tval, a.tstride);
             return hipGetLastError();
         }
     }
@@ -680,14 +798,19 @@ hipError_t launch_by_r(const StepArgs& a, hipStream_t s)
 }
 
 // ---- reduction of partials into moments ----------------------------------
+// One workgroup per vector and step.  A recursion keeps the partials of many steps
+// and reduces them in one launch: a launch per step cost 4-5 us of every step, as
+// much as the step itself on a small matrix.  The sum over workgroups is the same
+// fixed tree whatever the number of steps.
 __global__ __launch_bounds__(kThreads) void kpm_reduce_kernel(ReduceArgs a)
 {
     const int r = blockIdx.x;
     const int R = a.R;
     __shared__ double s[3][kThreads];
+    const double* part = a.part + (size_t)blockIdx.y * a.grid * R * 3;
     double t0 = 0.0, t1 = 0.0, t2 = 0.0;
     for (int g = threadIdx.x; g < a.grid; g += kThreads) {
-        const double* p = a.part + ((size_t)g * R + r) * 3;
+        const double* p = part + ((size_t)g * R + r) * 3;
         t0 += p[0];
         t1 += p[1];
         t2 += p[2];
@@ -707,33 +830,41 @@ __global__ __launch_bounds__(kThreads) void kpm_reduce_kernel(ReduceArgs a)
     if (threadIdx.x != 0) return;
     const double d1 = s[0][0], d2 = s[1][0], d3 = s[2][0];
     double* mu = a.mu + (size_t)r * a.M;
-    const int j = a.j, M = a.M;
-    auto load_re = [&](const void* buf, int row) -> double {
-        const size_t idx = (size_t)row * R + r;
-        switch (a.vec_type) {
-        case VEC_REAL_F64: return static_cast<const double*>(buf)[idx];
-        case VEC_CPX_F64: return static_cast<const double2*>(buf)[idx].x;
-        case VEC_CPX_F32: return (double)static_cast<const float2*>(buf)[idx].x;
-        default: return (double)static_cast<const float*>(buf)[idx];
-        }
-    };
+    const int j = a.j0 + blockIdx.y, M = a.M;
     if (a.scheme == 1) {
         if (j == 0) { mu[0] = d1; mu[1] = d2; }
         else if (2 * j + 1 < M) { mu[2 * j] = 2.0 * d1 - mu[0]; mu[2 * j + 1] = 2.0 * d2 - mu[1]; }
         return;
     }
     if (j == 0) {
-        if (a.scheme == 0) { mu[0] = 1.0; mu[1] = load_re(a.out, a.targets[r]); }
-        else { mu[0] = d1; mu[1] = d2; }
+        if (a.scheme != 0) { mu[0] = d1; mu[1] = d2; }
         return;
     }
     if (j >= 2 && j < M / 2) {
-        mu[j] = a.scheme == 0 ? load_re(a.cur, a.targets[r]) : d3;
+        if (a.scheme != 0) mu[j] = d3;
         if (j >= M / 4) {
             mu[2 * j] = 2.0 * d1 - mu[0];
             mu[2 * j + 1] = 2.0 * d2 - mu[1];
         }
     }
+}
+
+// The SELL step's own epilogue has no registers to spare for the target test (1.5 %
+// of every 64-vector step), so its target starts read the values in a launch of their own.
+__global__ void target_values_kernel(const void* cur, int vec_type, const int32_t* targets, int R, double* tval,
+                                     int tstride)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= R) return;
+    const size_t idx = (size_t)targets[r] * R + r;
+    double v;
+    switch (vec_type) {
+    case VEC_REAL_F64: v = static_cast<const double*>(cur)[idx]; break;
+    case VEC_CPX_F64: v = static_cast<const double2*>(cur)[idx].x; break;
+    case VEC_CPX_F32: v = (double)static_cast<const float2*>(cur)[idx].x; break;
+    default: v = (double)static_cast<const float*>(cur)[idx]; break;
+    }
+    tval[(size_t)r * tstride] = v;
 }
 
 // ---- start vectors ---------------------------------------------------------
@@ -886,7 +1017,16 @@ hipError_t launch_kpm_step(int mat_type, int vec_type, const StepArgs& a, hipStr
 
 hipError_t launch_kpm_reduce(const ReduceArgs& a, hipStream_t s)
 {
-    hipLaunchKernelGGL(kpm_reduce_kernel, dim3(a.R), dim3(kThreads), 0, s, a);
+    if (a.steps < 1 || (a.j0 == 0 && a.steps != 1)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kpm_reduce_kernel, dim3(a.R, a.steps), dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_target_values(const void* cur, int vec_type, const int32_t* targets, int R, double* tval, int tstride,
+                                hipStream_t s)
+{
+    hipLaunchKernelGGL(target_values_kernel, dim3((R + 63) / 64), dim3(64), 0, s, cur, vec_type, targets, R, tval,
+                       tstride);
     return hipGetLastError();
 }
 

@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kernels.h"
+
 namespace leo2d {
 namespace {
 
@@ -123,6 +125,109 @@ template <int K>
 __device__ inline double2 bc16(double2 v) { return make_double2(bc16<K>(v.x), bc16<K>(v.y)); }
 template <int K>
 __device__ inline float2 bc16(float2 v) { return make_float2(bc16<K>(v.x), bc16<K>(v.y)); }
+
+// ---- one row's entries over a group of lanes ------------------------------------
+// Blocks of few vectors put 16 lanes (64 where rows are long) on a matrix row.  A lane
+// takes three neighbouring entries, columns and values each in one wide load, gathers
+// all B vectors of each, and the lanes' sums are folded with DPP.  A pruned bilayer
+// row of 32 entries is one round of 48.  What bounds it: up to 4 real vectors the
+// matrix (12 B an entry, 3-4 TB/s), beyond that the gathers, which a CU's data path
+// returns at about 16 bytes a clock whatever the lane layout (TD 71 % busy while the
+// L1 hits 91 %; neighbouring lanes on one entry, or the next row's entries loaded
+// ahead, measured the same).  Microseconds per step on 95 k rows of 32 entries, lane
+// per vector before and this now: 4 real vectors 19.5 -> 15.9; on
+// 230 rows of 154 entries 17.1 -> 4.2.
+constexpr int kLaneEntries = 3;
+// entries that may be loaded (and not used) past the end of a matrix's arrays
+static_assert(kLaneEntries <= kCsrPad, "padding of the CSR arrays");
+
+// B consecutive elements, in 16-byte loads where they are that wide
+template <typename XT, int B>
+__device__ inline void ld_vecs(XT (&x)[B], const XT* p)
+{
+    if constexpr (sizeof(XT) * B >= 16) {
+        typedef int i4v __attribute__((ext_vector_type(4)));
+        constexpr int per = 16 / (int)sizeof(XT);
+#pragma unroll
+        for (int b = 0; b < B; b += per) {
+            const i4v q = *reinterpret_cast<const i4v*>(p + b);
+            __builtin_memcpy(&x[b], &q, 16);
+        }
+    } else {
+#pragma unroll
+        for (int b = 0; b < B; ++b) x[b] = p[b];
+    }
+}
+
+// row extents in one load
+struct alignas(8) RowExtent {
+    int64_t q0, q1;
+};
+__device__ inline RowExtent row_extent(const int64_t* __restrict__ rp, int row)
+{
+    return *reinterpret_cast<const RowExtent*>(rp + row);
+}
+struct alignas(4) LaneCols {
+    int c[kLaneEntries];
+};
+template <typename HT>
+struct LaneVals {
+    HT h[kLaneEntries];
+};
+
+template <int CTRL>
+__device__ inline int dpp_mov(int v) { return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true); }
+template <int CTRL>
+__device__ inline double dpp_mov(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = dpp_mov<CTRL>((int)(b & 0xffffffffLL)), hi = dpp_mov<CTRL>((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <int CTRL>
+__device__ inline double2 dpp_mov(double2 v) { return make_double2(dpp_mov<CTRL>(v.x), dpp_mov<CTRL>(v.y)); }
+__device__ inline double add(double a, double b) { return a + b; }
+__device__ inline double2 add(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ inline double xor_lanes(double a, int off) { return __shfl_xor(a, off); }
+__device__ inline double2 xor_lanes(double2 a, int off) { return make_double2(__shfl_xor(a.x, off), __shfl_xor(a.y, off)); }
+
+// One exchange of the fold: the lane with its bit W set keeps the upper half of its
+// N sums, its partner the lower, each adding the other's; with one sum left both add.
+// The partners (a rotation by 8, the half-row mirror, quad swaps by 2 and 1) differ in bit W.
+template <int W, typename AT, int N>
+__device__ inline AT fold_lanes(AT (&a)[N], int lane)
+{
+    constexpr int CTRL = W == 8 ? 0x128 : (W == 4 ? 0x141 : (W == 2 ? 0x4E : 0xB1));
+    if constexpr (N > 1) {
+        AT k[N / 2];
+        const bool hi = (lane & W) != 0;
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const AT mine = hi ? a[i + N / 2] : a[i];
+            const AT sent = hi ? a[i] : a[i + N / 2];
+            k[i] = add(mine, dpp_mov<CTRL>(sent));
+        }
+        if constexpr (W > 1) return fold_lanes<W / 2>(k, lane);
+        else return k[0];
+    } else {
+        AT k[1] = {add(a[0], dpp_mov<CTRL>(a[0]))};
+        if constexpr (W > 1) return fold_lanes<W / 2>(k, lane);
+        else return k[0];
+    }
+}
+// Sum over the LPR lanes of a row; lane l of each 16 ends with vector l / (16 / B)
+// (B a power of two, at most 16).
+template <int LPR, typename AT, int B>
+__device__ inline AT fold_row(AT (&a)[B], int lane)
+{
+    static_assert(B >= 1 && B <= 16 && (LPR == 16 || LPR == 64), "at most one vector per lane");
+    AT t = fold_lanes<8>(a, lane);
+    if constexpr (LPR == 64) {
+        t = add(t, xor_lanes(t, 16));
+        t = add(t, xor_lanes(t, 32));
+    }
+    return t;
+}
 
 // gathers and multiply-adds for the 16 entries of one chunk held by a
 // 16-lane row (entry K in lane K); only the first m entries are live
