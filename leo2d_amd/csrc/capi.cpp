@@ -114,6 +114,7 @@ struct SellTiles {
 }  // namespace
 
 struct leo2d_handle {
+    leo2d::DevPool pool;   // first member: the buffers below go back to it
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
@@ -220,6 +221,7 @@ namespace {
 template <typename F>
 int guarded(leo2d_handle* h, F&& f)
 {
+    leo2d::DevPool::Use use(h ? &h->pool : nullptr);
     try {
         if (h) {
             check(hipSetDevice(h->device), "hipSetDevice");
@@ -1503,7 +1505,6 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
         dalloc(part, std::max(sizeof(double) * 3 * (size_t)G * B, leo2d::kPartialSpace), "partials");
         dalloc(dmu, sizeof(double) * (size_t)M * B, "moments");
         dalloc(dtg, sizeof(int32_t) * B, "targets");
-        std::vector<double> hv;
         double rec_ms = 0.0, step_ms = 0.0;
         int kernel_used = -1;
         int64_t steps = 0;
@@ -1524,11 +1525,12 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                 if (real_vec) throw ArgError("random phases need complex vectors");
                 check(leo2d::launch_init_random_phase_perm(A.p, vec_type, n, B, p->seed, b0, iperm, s), "init");
             } else {
-                const int w = p->vectors_complex ? 2 : 1;
-                hv.assign((size_t)w * n * B, 0.0);
-                std::memcpy(hv.data(), p->vectors + (size_t)w * n * b0, sizeof(double) * (size_t)w * n * Rb);
-                dalloc(host_v, sizeof(double) * hv.size(), "vector upload");
-                check(hipMemcpyAsync(host_v.p, hv.data(), sizeof(double) * hv.size(), hipMemcpyHostToDevice, s), "upload");
+                // the caller's vectors as they are, the block's further vectors zero
+                const size_t per = (size_t)(p->vectors_complex ? 2 : 1) * n;
+                dalloc(host_v, sizeof(double) * per * B, "vector upload");
+                check(hipMemcpyAsync(host_v.p, p->vectors + per * b0, sizeof(double) * per * Rb, hipMemcpyHostToDevice, s),
+                      "upload");
+                check(leo2d::launch_zero_f64((double*)host_v.p + per * Rb, (int64_t)(per * (B - Rb)), s), "upload");
                 check(leo2d::launch_init_from_host_layout_perm(A.p, vec_type, (const double*)host_v.p,
                                                                p->vectors_complex, n, B, iperm, s),
                       "init");

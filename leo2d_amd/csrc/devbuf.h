@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <map>
 #include <stdexcept>
 #include <string>
 
@@ -11,14 +12,74 @@
 
 namespace leo2d {
 
-// owning device allocation (freed on release() or destruction; movable, not copyable)
+// Device buffers a handle has given back, kept for its next allocations.  A call
+// allocates and frees a dozen small buffers, each some 10-30 us with the device-wide
+// wait of a free; on a 230-orbital deck that was half of the time.  Everything a
+// handle queues runs on its one stream, so a buffer taken again is written only by
+// work queued after its last use.  Bounded: buffers of at most kPoolMost bytes, at
+// most kPoolKeep in all; the rest are freed at once, and all of them when an
+// allocation fails and with the handle.  Not shared between handles (one thread each).
+class DevPool {
+public:
+    static constexpr size_t kPoolMost = size_t(64) << 20;
+    static constexpr size_t kPoolKeep = size_t(256) << 20;
+    DevPool() = default;
+    DevPool(const DevPool&) = delete;
+    DevPool& operator=(const DevPool&) = delete;
+    ~DevPool() { clear(); }
+    // a kept buffer of at least `bytes` (and less than twice that), or nullptr; cap: its size
+    void* take(size_t bytes, size_t& cap)
+    {
+        auto it = free_.lower_bound(bytes);
+        if (it == free_.end() || it->first / 2 > bytes) return nullptr;
+        void* p = it->second;
+        cap = it->first;
+        kept_ -= cap;
+        free_.erase(it);
+        return p;
+    }
+    void give(void* p, size_t cap)
+    {
+        if (cap > kPoolMost || kept_ + cap > kPoolKeep) {
+            (void)hipFree(p);
+            return;
+        }
+        kept_ += cap;
+        free_.emplace(cap, p);
+    }
+    void clear()
+    {
+        for (auto& f : free_) (void)hipFree(f.second);
+        free_.clear();
+        kept_ = 0;
+    }
+    // the pool of the handle whose entry point this thread is in
+    static DevPool*& current()
+    {
+        static thread_local DevPool* pool = nullptr;
+        return pool;
+    }
+    struct Use {   // makes `pool` current for a scope
+        DevPool* was;
+        explicit Use(DevPool* pool) : was(current()) { current() = pool; }
+        ~Use() { current() = was; }
+    };
+
+private:
+    std::multimap<size_t, void*> free_;   // by size
+    size_t kept_ = 0;
+};
+
+// owning device allocation (given back on release() or destruction; movable, not copyable)
 struct DevBuf {
     void* p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0;          // as asked for
+    size_t cap = 0;            // as allocated
+    DevPool* pool = nullptr;   // where it goes back to (nullptr: freed)
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes)
+    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), cap(o.cap), pool(o.pool)
     {
         o.p = nullptr;
         o.bytes = 0;
@@ -29,6 +90,8 @@ struct DevBuf {
             release();
             p = o.p;
             bytes = o.bytes;
+            cap = o.cap;
+            pool = o.pool;
             o.p = nullptr;
             o.bytes = 0;
         }
@@ -37,7 +100,10 @@ struct DevBuf {
     ~DevBuf() { release(); }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (pool) pool->give(p, cap);
+            else (void)hipFree(p);
+        }
         p = nullptr;
         bytes = 0;
     }
@@ -106,7 +172,30 @@ inline void dalloc(DevBuf& b, size_t bytes, const char* what)
 {
     b.release();
     if (bytes == 0) bytes = 16;
-    const hipError_t e = hipMalloc(&b.p, bytes);
+    DevPool* const pool = DevPool::current();
+    // a pooled buffer's size is rounded up (to an eighth of its power of two), so that calls on
+    // slightly different sizes find each other's buffers
+    size_t cap = bytes;
+    if (pool && bytes <= DevPool::kPoolMost) {
+        size_t step = 256;
+        while (step * 16 < bytes) step *= 2;
+        cap = (bytes + step - 1) / step * step;
+        size_t got = 0;
+        if (void* p = pool->take(cap, got)) {
+            b.p = p;
+            b.bytes = bytes;
+            b.cap = got;
+            b.pool = pool;
+            return;
+        }
+    }
+    hipError_t e = hipMalloc(&b.p, cap);
+    if (e != hipSuccess && pool) {
+        // what the pool keeps may be what is missing
+        (void)hipGetLastError();
+        pool->clear();
+        e = hipMalloc(&b.p, cap);
+    }
     if (e != hipSuccess) {
         // a failed allocation is not sticky, but it stays the runtime's last error:
         // clear it, or the next launch check (hipGetLastError) would report it
@@ -115,6 +204,8 @@ inline void dalloc(DevBuf& b, size_t bytes, const char* what)
         check(e, what);
     }
     b.bytes = bytes;
+    b.cap = cap;
+    b.pool = pool;
 }
 
 }  // namespace leo2d

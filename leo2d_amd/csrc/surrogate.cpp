@@ -24,6 +24,7 @@ using leo2d::DevBuf;
 using leo2d::HipError;
 
 struct leo2d_mlp {
+    leo2d::DevPool pool;   // first member: the buffers below go back to it
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
@@ -55,6 +56,7 @@ struct ArgError : std::runtime_error {
 template <typename F>
 int guarded(leo2d_mlp* m, F&& f)
 {
+    leo2d::DevPool::Use use(m ? &m->pool : nullptr);
     try {
         if (m) check(hipSetDevice(m->device), "hipSetDevice");
         return f();
@@ -86,6 +88,7 @@ void to_device_f32(DevBuf& b, const std::vector<float>& v, hipStream_t s)
 void ensure_capacity(leo2d_mlp* m, int rows)
 {
     if (rows <= m->cap) return;
+    leo2d::DevPool::Use own(&m->pool);   // the network's buffers, whichever network's call this is
     const int cap = std::max(rows, 256);
     const int hmax = *std::max_element(m->dims.begin() + 1, m->dims.end() - 1);
     dalloc(m->X16, sizeof(uint16_t) * (size_t)cap * m->in(), "mlp inputs");
@@ -107,11 +110,12 @@ void ensure_capacity(leo2d_mlp* m, int rows)
     m->cap = cap;
 }
 
-// Y[rows][out] = MLP(X16[rows][in]) ; Y may point outside the workspace
-void forward(leo2d_mlp* m, int rows, float* Y)
+// Y[rows][out] = MLP(X16[rows][in]) ; Y (and X16, by default the network's own) may
+// point outside the workspace
+void forward(leo2d_mlp* m, int rows, float* Y, const uint16_t* X16 = nullptr)
 {
     hipStream_t s = m->stream;
-    const uint16_t* hin = bf(m->X16);
+    const uint16_t* hin = X16 ? X16 : bf(m->X16);
     for (int l = 0; l < m->layers(); ++l) {
         const int din = m->dims[l], dout = m->dims[l + 1];
         leo2d::GemmArgs g{};
@@ -443,6 +447,7 @@ int leo2d_mlp_train_ensemble(leo2d_mlp* const* nets, int32_t count, const float*
         const int64_t total = steps * (int64_t)p->epochs;
         if (total + 1 > 0x7fffffffLL) throw ArgError("too many training steps");
         if (p->epochs == 0) return LEO2D_OK;
+        leo2d::DevPool::Use none(nullptr);   // buffers several streams use are not pooled
         hipStream_t s0 = m0->stream;
         DevBuf X, T;
         dalloc(X, sizeof(float) * (size_t)n * m0->in(), "training inputs");
@@ -560,32 +565,51 @@ int leo2d_mlp_ensemble(leo2d_mlp* const* nets, int32_t count, const float* x, in
     for (int e = 0; e < count; ++e)
         if (!nets[e] || nets[e]->dims != m0->dims || nets[e]->device != m0->device) return LEO2D_ERR_ARG;
     return guarded(m0, [&]() {
+        // The inputs go up and are rounded once, on the first network's stream; the networks
+        // run side by side on their own streams after it, and the statistics wait for them all.
+        leo2d::DevPool::Use none(nullptr);   // buffers several streams use are not pooled
         const int chunk = 4096;
         const int out = m0->out();
+        hipStream_t s0 = m0->stream;
         DevBuf Ys, dmean, dspread;
         dalloc(Ys, sizeof(float) * (size_t)count * chunk * out, "ensemble outputs");
         dalloc(dmean, sizeof(float) * (size_t)chunk * out, "ensemble mean");
-        dalloc(dspread, sizeof(float) * (size_t)chunk * blocks, "ensemble spread");
+        dalloc(dspread, sizeof(float) * (size_t)std::max<int64_t>(n, 1) * blocks, "ensemble spread");
+        struct Event {
+            hipEvent_t e = nullptr;
+            Event() { check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "ensemble event"); }
+            Event(const Event&) = delete;
+            Event& operator=(const Event&) = delete;
+            ~Event() { (void)hipEventDestroy(e); }
+        };
+        std::vector<Event> done((size_t)count);   // [0]: inputs ready
         for (int e = 0; e < count; ++e) ensure_capacity(nets[e], std::min<int64_t>(n, chunk));
-        for (int64_t r0 = 0; r0 < n; r0 += chunk) {
-            const int rows = (int)std::min<int64_t>(chunk, n - r0);
-            for (int e = 0; e < count; ++e) {
-                leo2d_mlp* m = nets[e];
-                upload_inputs(m, x + (size_t)r0 * m->in(), rows);
-                forward(m, rows, static_cast<float*>(Ys.p) + (size_t)e * chunk * out);
-                check(hipStreamSynchronize(m->stream), "ensemble forward");
+        try {
+            for (int64_t r0 = 0; r0 < n; r0 += chunk) {
+                const int rows = (int)std::min<int64_t>(chunk, n - r0);
+                upload_inputs(m0, x + (size_t)r0 * m0->in(), rows);
+                check(hipEventRecord(done[0].e, s0), "ensemble inputs");
+                for (int e = 0; e < count; ++e) {
+                    leo2d_mlp* m = nets[e];
+                    if (m != m0) check(hipStreamWaitEvent(m->stream, done[0].e, 0), "ensemble inputs");
+                    forward(m, rows, static_cast<float*>(Ys.p) + (size_t)e * chunk * out, bf(m0->X16));
+                    if (m != m0) check(hipEventRecord(done[(size_t)e].e, m->stream), "ensemble forward");
+                }
+                for (int e = 0; e < count; ++e)
+                    if (nets[e] != m0) check(hipStreamWaitEvent(s0, done[(size_t)e].e, 0), "ensemble forward");
+                check(leo2d::launch_ensemble_stats(static_cast<const float*>(Ys.p), count, (int64_t)chunk * out, rows, out,
+                                                   blocks, f32(dmean), f32(dspread, r0 * blocks), s0),
+                      "ensemble stats");
+                if (mean)
+                    check(hipMemcpyAsync(mean + (size_t)r0 * out, dmean.p, sizeof(float) * (size_t)rows * out,
+                                         hipMemcpyDeviceToHost, s0),
+                          "ensemble mean");
             }
-            check(leo2d::launch_ensemble_stats(static_cast<const float*>(Ys.p), count, (int64_t)chunk * out, rows, out,
-                                               blocks, f32(dmean), f32(dspread), m0->stream),
-                  "ensemble stats");
-            if (mean)
-                check(hipMemcpyAsync(mean + (size_t)r0 * out, dmean.p, sizeof(float) * (size_t)rows * out,
-                                     hipMemcpyDeviceToHost, m0->stream),
-                      "ensemble mean");
-            check(hipMemcpyAsync(spread + r0 * blocks, dspread.p, sizeof(float) * rows * blocks, hipMemcpyDeviceToHost,
-                                 m0->stream),
-                  "ensemble spread");
-            check(hipStreamSynchronize(m0->stream), "ensemble");
+            if (n) check(hipMemcpyAsync(spread, dspread.p, sizeof(float) * n * blocks, hipMemcpyDeviceToHost, s0), "ensemble spread");
+            check(hipStreamSynchronize(s0), "ensemble");
+        } catch (...) {
+            (void)hipDeviceSynchronize();   // nothing may still run on the buffers freed here
+            throw;
         }
         return LEO2D_OK;
     });

@@ -1,0 +1,75 @@
+"""Device buffers a handle keeps between calls: calls of other sizes and kinds in
+between, and other handles on other threads, leave every result bit for bit what
+a fresh handle gives."""
+import threading
+
+import numpy as np
+import pytest
+
+import leo2d_amd as L
+from leo2d_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _calls(dev):
+    """Moments and DoS of matrices of several sizes, conductivity and a batch, in one sequence."""
+    out = []
+    for radius, R in ((12.0, 3), (30.0, 16), (12.0, 1), (21.0, 64), (12.0, 3)):
+        geom = L.Geometry(L.Deck(W.tblg_flake_deck(3.0, radius, M=64)))
+        dev.set_geometry(geom)
+        job = geom.jobs()[0]
+        dev.assemble_velocity(job, L.PATTERN_PRUNED)
+        mu = dev.kpm(64, targets=np.arange(R, dtype=np.int32))
+        out += [mu, dev.dos(mu, 10.5, 0.0)[1], dev.kpm(64, random_phase=(R, 5)), dev.cond_moments(24, [0, 1, 2])]
+        dev.batch_append()
+    out.append(dev.batch_kpm(32, 16, seed=3, mode=L.BATCH_ROW_CHUNKS))
+    dev.batch_clear()
+    return out
+
+
+def _fresh():
+    dev = L.Device(0)
+    try:
+        return _calls(dev)
+    finally:
+        dev.close()
+
+
+def test_repeated_calls_on_kept_buffers():
+    ref = _fresh()
+    dev = L.Device(0)
+    for _ in range(3):
+        assert all(np.array_equal(a, b) for a, b in zip(_calls(dev), ref))
+    dev.close()
+
+
+def test_handles_on_threads():
+    ref = _fresh()
+    got = [None] * 3
+
+    def work(k):
+        got[k] = [_fresh(), _fresh()]
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for pair in got:
+        for calls in pair:
+            assert all(np.array_equal(a, b) for a, b in zip(calls, ref))
+
+
+def test_ensemble_members_destroyed_in_any_order():
+    x = np.random.default_rng(0).standard_normal((700, 72)).astype(np.float32)
+    nets = [L.Mlp(0, 72, 64, 2, 96, seed=k) for k in range(3)]
+    one = [m.forward(x) for m in nets]
+    mean, spread = L.mlp_ensemble([nets[1], nets[0], nets[2], nets[0]], x)
+    ref = np.mean([one[1], one[0], one[2], one[0]], axis=0)
+    assert np.max(np.abs(mean - ref)) <= 1e-6 * np.max(np.abs(ref))
+    nets[1].close()
+    assert np.array_equal(nets[0].forward(x), one[0])
+    nets[0].close()
+    assert np.array_equal(nets[2].forward(x), one[2])
+    nets[2].close()
