@@ -27,6 +27,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "assemble.h"
+#include "devbuf.h"
 #include "kernels.h"
 
 namespace leo2d {
@@ -1041,11 +1042,10 @@ hipError_t scan_counts(const int64_t* cnt, int64_t* out, int n, hipStream_t s)
     size_t tmp_bytes = 0;
     hipError_t e = hipcub::DeviceScan::InclusiveSum(nullptr, tmp_bytes, cnt, out + 1, n, s);
     if (e != hipSuccess) return e;
-    void* tmp = nullptr;
-    e = hipMallocAsync(&tmp, tmp_bytes + 16, s);
-    if (e != hipSuccess) return e;
-    e = hipcub::DeviceScan::InclusiveSum(tmp, tmp_bytes, cnt, out + 1, n, s);
-    hipFreeAsync(tmp, s);
+    // from the handle's kept buffers: an allocation on the stream fails while another thread captures a graph
+    DevBuf tmp;
+    dalloc(tmp, tmp_bytes + 16, "scan workspace");
+    e = hipcub::DeviceScan::InclusiveSum(tmp.p, tmp_bytes, cnt, out + 1, n, s);
     if (e != hipSuccess) return e;
     return hipMemsetAsync(out, 0, sizeof(int64_t), s);
 }
