@@ -7,15 +7,25 @@
 // keeps FP32 master weights.  There is no counterpart in the reference; the
 // moments it learns come from the KPM recursion of this library.
 //
-// One GEMM kernel serves every product of training and inference through
-// strides: C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = A[m*sam + k*sak] and
-// B(k, n) = B[k*sbk + n*sbn], so X W^T (forward), dZ^T X (weight gradient)
-// and dZ W (input gradient) need no transposed copies.  The epilogue fuses
-// bias, GELU, its derivative and the bf16 store of the next layer's operand.
+// Both operands of every product have k contiguous in memory, so a lane's eight k of
+// an MFMA operand are one 16-byte load: X W^T reads X and W, the input gradient dZ W
+// reads a transposed copy of W, the weight gradient dZ^T X transposed copies of dZ
+// and X, which the kernels that make these operands write beside them.
 //
-// Tiling: a 256-thread workgroup owns a 64 x 64 tile of C; its 4 wavefronts
-// each own 32 x 32 = 2 x 2 MFMA tiles of 16 x 16.  K advances in steps of 32
-// through LDS (A tile 64 x 32, B tile 32 x 64, bf16), two MFMA k-steps each.
+// What bounds it: the products are small (a training batch of 512 on 256-wide
+// layers), so a launch is a chain of load latencies.  Small products take 32 x 32
+// tiles, a 16 x 16 block per wavefront with sixteen loads straight into registers in
+// flight: 128 to 512 workgroups where 64 x 64 tiles gave 32, and no barrier per k
+// step.  Large products (inference) stage 64 x 64 or 128 x 128 tiles through LDS:
+// read straight from memory, an operand row's 64 bytes per k step come at the 16
+// bytes a clock of a scattered load.  Every output is one chain of k steps of 32 in
+// order in all of them, so the tile does not change a bit of the result.  (k shared
+// by the four wavefronts of a workgroup was as fast and changes the rounding.)
+// The two products of a layer's backward pass (its weight gradient and the input
+// gradient below) go out in one launch, bias gradients and the loss with them: a
+// training step on 512 rows of 72 -> 3 x 256 -> 1024 is 10 launches and about 75 us
+// on the GPU (19 and 177 us with 64 x 64 tiles, operands transposed through LDS two
+// bytes at a time and a kernel each for the loss and the column sums).
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -27,11 +37,11 @@
 namespace leo2d {
 namespace {
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef short bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kT = 256;
-constexpr int kTM = 64, kTN = 64, kTK = 32;
 
 __device__ inline uint16_t f2bf(float f)
 {
@@ -56,326 +66,334 @@ __device__ inline float gelu_grad(float z)
     return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * z * z);
 }
 
+// eight k of an operand row from k on, zero past K
+__device__ inline bf16x8 ld_frag(const uint16_t* row, int k, int K)
+{
+    bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (k < K) {
+        v = *reinterpret_cast<const bf16x8*>(row + k);
+        if (k + 8 > K) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                if (k + t >= K) v[t] = 0;
+        }
+    }
+    return v;
+}
+
+struct GemmBatch {
+    GemmArgs g[2];
+    int tiles[2];       // workgroups of each product
+    SumArgs sums;
+    int sum_blocks;
+    LossArgs loss;
+};
+
+// the epilogue EPI of four rows of one column (rows row .. row + 3, those below M)
 template <int EPI>
-__global__ __launch_bounds__(kT) void gemm_bf16_kernel(GemmArgs g)
+__device__ inline void gemm_store(const GemmArgs& g, const floatx4& v, int row, int col, int lane)
 {
-    __shared__ uint16_t As[kTM][kTK + 4];
-    __shared__ uint16_t Bs[kTK][kTN + 4];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
-
-    floatx4 acc[2][2];
+    const bool in = col < g.N;
+    const int rows = in ? min(4, g.M - row) : 0;
+    const float bias = in && (EPI == EPI_BIAS_F32 || EPI == EPI_BIAS_GELU || EPI == EPI_MSE) ? g.bias[col] : 0.f;
+    uint16_t h[4] = {0, 0, 0, 0};
+    double sq[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        // stage A (64 x 32) and B (32 x 64): 8 elements per thread each, zero outside the matrix
-        for (int e = tid; e < kTM * kTK; e += kT) {
-            const int mm = e / kTK, kk = e % kTK;
-            const int m = m0 + mm, k = k0 + kk;
-            As[mm][kk] = (m < g.M && k < g.K) ? g.A[(int64_t)m * g.sam + (int64_t)k * g.sak] : (uint16_t)0;
-        }
-        for (int e = tid; e < kTK * kTN; e += kT) {
-            const int kk = e / kTN, nn = e % kTN;
-            const int k = k0 + kk, n = n0 + nn;
-            Bs[kk][nn] = (k < g.K && n < g.N) ? g.B[(int64_t)k * g.sbk + (int64_t)n * g.sbn] : (uint16_t)0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < kTK; ks += 16) {
-            bf16x4 af[2], bfr[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int row = wm * 32 + i * 16 + (lane & 15);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) af[i][t] = (short)As[row][ks + 4 * (lane >> 4) + t];
+    for (int t = 0; t < 4; ++t) {
+        if (t < rows) {
+            const int64_t o = (int64_t)(row + t) * g.ldc + col;
+            if (EPI == EPI_STORE_F32) {
+                g.C32[o] = v[t];
+            } else if (EPI == EPI_BIAS_F32) {
+                g.C32[o] = v[t] + bias;
+            } else if (EPI == EPI_BIAS_GELU) {
+                const float z = v[t] + bias;
+                if (g.Z) g.Z[o] = z;
+                h[t] = f2bf(gelu(z));
+            } else if (EPI == EPI_GELU_BWD) {
+                h[t] = f2bf(v[t] * gelu_grad(g.Z[o]));
+            } else {
+                const float d = (v[t] + bias) - g.T[o];
+                h[t] = f2bf(g.scale * d);
+                sq[t] = (double)d * (double)d;
             }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int cc = wn * 32 + j * 16 + (lane & 15);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) bfr[j][t] = (short)Bs[ks + 4 * (lane >> 4) + t][cc];
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af[i], bfr[j], acc[i][j], 0, 0, 0);
+            if (EPI != EPI_STORE_F32 && EPI != EPI_BIAS_F32) g.C16[(int64_t)(row + t) * g.ld16 + col] = h[t];
         }
-        __syncthreads();
     }
-
-    // epilogue: lane holds C[row0 + t][col] for t = 0..3
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn * 32 + j * 16 + (lane & 15);
-            if (col >= g.N) continue;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int row = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + t;
-                if (row >= g.M) continue;
-                const int64_t o = (int64_t)row * g.scm + col;
-                const float v = acc[i][j][t];
-                if (EPI == EPI_STORE_F32) {
-                    g.C32[o] = v;
-                } else if (EPI == EPI_BIAS_F32) {
-                    g.C32[o] = v + g.bias[col];
-                } else if (EPI == EPI_BIAS_GELU) {
-                    const float z = v + g.bias[col];
-                    g.Z[o] = z;
-                    g.C16[o] = f2bf(gelu(z));
-                } else {   // EPI_GELU_BWD: dZ = (dZ_next W) * gelu'(Z)
-                    g.C16[o] = f2bf(v * gelu_grad(g.Z[o]));
-                }
-            }
-        }
-}
-
-// ---- vectorised GEMM (gfx950 16x16x32 bf16 MFMA) -------------------------------
-// Same product and epilogues.  Operands are staged as 16-byte runs of 8 bf16
-// (along k when that is the contiguous direction, else along m / n), A as
-// As[m][k] and B transposed as Bt[n][k] in LDS, so every MFMA operand is one
-// 16-byte LDS read.  The next k-tile is loaded into registers while the
-// current one is multiplied.  Needs K, the contiguous strides and the base
-// addresses to be multiples of 8 elements (checked by the launcher).
-typedef short bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
-constexpr int kPad = 8;
-
-template <bool AK>
-__device__ inline u16x8 load_a(const GemmArgs& g, int m0, int k0, int tid, int& mm, int& kk)
-{
-    // AK: 8 consecutive k of one row m (thread -> (m, k-run)); else 8 consecutive m of one k
-    if (AK) {
-        mm = tid >> 2;
-        kk = (tid & 3) * 8;
-    } else {
-        kk = tid >> 3;
-        mm = (tid & 7) * 8;
-    }
-    const int m = m0 + mm, k = k0 + kk;
-    u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (k < g.K && m < g.M) v = *reinterpret_cast<const u16x8*>(g.A + (int64_t)m * g.sam + (int64_t)k * g.sak);
-    return v;
-}
-template <bool BK>
-__device__ inline u16x8 load_b(const GemmArgs& g, int n0, int k0, int tid, int& nn, int& kk)
-{
-    if (BK) {
-        nn = tid >> 2;
-        kk = (tid & 3) * 8;
-    } else {
-        kk = tid >> 3;
-        nn = (tid & 7) * 8;
-    }
-    const int n = n0 + nn, k = k0 + kk;
-    u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (k < g.K && n < g.N) v = *reinterpret_cast<const u16x8*>(g.B + (int64_t)k * g.sbk + (int64_t)n * g.sbn);
-    return v;
-}
-
-template <int EPI, bool AK, bool BK>
-__global__ __launch_bounds__(kT) void gemm_bf16_v2_kernel(GemmArgs g)
-{
-    __shared__ __align__(16) uint16_t As[kTM][kTK + kPad];
-    __shared__ __align__(16) uint16_t Bt[kTN][kTK + kPad];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
-
-    floatx4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    int am, ak, bn, bk;
-    u16x8 ra = load_a<AK>(g, m0, 0, tid, am, ak);
-    u16x8 rb = load_b<BK>(g, n0, 0, tid, bn, bk);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        __syncthreads();   // previous tile fully read
-        if (AK) {
-            *reinterpret_cast<u16x8*>(&As[am][ak]) = ra;
+    if (EPI == EPI_STORE_F32 || EPI == EPI_BIAS_F32) return;
+    if (g.C16T && rows > 0) {
+        uint16_t* p = g.C16T + (int64_t)col * g.ld16t + row;   // row is a multiple of 4, ld16t of 8
+        if (rows == 4) {
+            *reinterpret_cast<u16x4*>(p) = u16x4{h[0], h[1], h[2], h[3]};
         } else {
 #pragma unroll
-            for (int t = 0; t < 8; ++t) As[am + t][ak] = ra[t];
+            for (int t = 0; t < 4; ++t)
+                if (t < rows) p[t] = h[t];
         }
-        if (BK) {
-            *reinterpret_cast<u16x8*>(&Bt[bn][bk]) = rb;
-        } else {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) Bt[bn + t][bk] = rb[t];
-        }
-        __syncthreads();
-        if (k0 + kTK < g.K) {   // next tile in flight during the products
-            ra = load_a<AK>(g, m0, k0 + kTK, tid, am, ak);
-            rb = load_b<BK>(g, n0, k0 + kTK, tid, bn, bk);
-        }
-        bf16x8 af[2], bfr[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            af[i] = *reinterpret_cast<const bf16x8*>(&As[wm * 32 + i * 16 + (lane & 15)][8 * (lane >> 4)]);
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            bfr[j] = *reinterpret_cast<const bf16x8*>(&Bt[wn * 32 + j * 16 + (lane & 15)][8 * (lane >> 4)]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
     }
-
+    if (EPI == EPI_MSE) {
+        // the 16 columns of this block (their lanes hold the same four rows)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int t = 0; t < 4; ++t) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn * 32 + j * 16 + (lane & 15);
-            if (col >= g.N) continue;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int row = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + t;
-                if (row >= g.M) continue;
-                const int64_t o = (int64_t)row * g.scm + col;
-                const float v = acc[i][j][t];
-                if (EPI == EPI_STORE_F32) {
-                    g.C32[o] = v;
-                } else if (EPI == EPI_BIAS_F32) {
-                    g.C32[o] = v + g.bias[col];
-                } else if (EPI == EPI_BIAS_GELU) {
-                    const float z = v + g.bias[col];
-                    g.Z[o] = z;
-                    g.C16[o] = f2bf(gelu(z));
-                } else {
-                    g.C16[o] = f2bf(v * gelu_grad(g.Z[o]));
-                }
-            }
+            for (int off = 8; off > 0; off >>= 1) sq[t] += __shfl_xor(sq[t], off);
+            if ((lane & 15) == 0 && row + t < g.M && col < g.N)
+                g.loss[(int64_t)(row + t) * ((g.N + 15) / 16) + col / 16] = sq[t];
         }
+    }
+}
+// the same, the epilogue known at run time only
+__device__ inline void gemm_store(const GemmArgs& g, const floatx4& v, int row, int col, int lane)
+{
+    switch (g.epi) {
+    case EPI_STORE_F32: gemm_store<EPI_STORE_F32>(g, v, row, col, lane); break;
+    case EPI_BIAS_F32: gemm_store<EPI_BIAS_F32>(g, v, row, col, lane); break;
+    case EPI_BIAS_GELU: gemm_store<EPI_BIAS_GELU>(g, v, row, col, lane); break;
+    case EPI_GELU_BWD: gemm_store<EPI_GELU_BWD>(g, v, row, col, lane); break;
+    default: gemm_store<EPI_MSE>(g, v, row, col, lane); break;
+    }
 }
 
-// dY = scale (Y - T) as bf16 and per-row squared-error sums (FP64, fixed order)
-__global__ __launch_bounds__(kT) void mse_grad_kernel(const float* Y, const float* T, int rows, int cols, float scale,
-                                                      uint16_t* dY, double* row_loss)
+// out[c] = sum_k A[c][k].  A workgroup owns kSumRows rows of A (outputs c); kSumGroups
+// threads each add a contiguous slice of k in order, and the slices are added in order.
+constexpr int kSumRows = 16;
+constexpr int kSumGroups = kT / kSumRows;
+__device__ inline void row_sums(const SumArgs& a, int block, float (*part)[kSumRows])
 {
-    const int r = blockIdx.x;
-    if (r >= rows) return;
-    __shared__ double s[kT];
-    double acc = 0.0;
-    for (int c = threadIdx.x; c < cols; c += kT) {
-        const int64_t o = (int64_t)r * cols + c;
-        const float d = Y[o] - T[o];
-        dY[o] = f2bf(scale * d);
-        acc += (double)d * (double)d;
-    }
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = kT / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) row_loss[r] = s[0];
-}
-
-// db[n] = sum_m dZ[m][n] (bf16 operand values, FP32 sum in row order)
-// db[c] = sum_r dZ[r][c].  A workgroup owns kColsumCols columns; its kColsumGroups
-// row groups each sum a contiguous slice of rows (8 loads in flight), and the
-// slices are added in group order, so the result does not depend on timing.
-constexpr int kColsumCols = 16;
-constexpr int kColsumGroups = kT / kColsumCols;
-
-__global__ __launch_bounds__(kT) void colsum_kernel(const uint16_t* dZ, int rows, int cols, float* db)
-{
-    __shared__ float part[kColsumGroups][kColsumCols];
-    const int cx = threadIdx.x % kColsumCols, g = threadIdx.x / kColsumCols;
-    const int c = blockIdx.x * kColsumCols + cx;
-    const int per = (rows + kColsumGroups - 1) / kColsumGroups;
-    const int r0 = min(rows, g * per), r1 = min(rows, r0 + per);
+    const int cx = threadIdx.x / kSumGroups, g = threadIdx.x % kSumGroups;
+    const int c = block * kSumRows + cx;
+    const int per = (a.K + kSumGroups - 1) / kSumGroups;
+    const int k0 = min(a.K, g * per), k1 = min(a.K, k0 + per);
     float s = 0.f;
-    if (c < cols) {
-        int r = r0;
-        for (; r + 8 <= r1; r += 8) {
+    if (c < a.rows) {
+        const uint16_t* p = a.A + (int64_t)c * a.lda;
+        int k = k0;
+        for (; k + 8 <= k1; k += 8) {
             float v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = bf2f(dZ[(int64_t)(r + u) * cols + c]);
+            for (int u = 0; u < 8; ++u) v[u] = bf2f(p[k + u]);
 #pragma unroll
             for (int u = 0; u < 8; ++u) s += v[u];
         }
-        for (; r < r1; ++r) s += bf2f(dZ[(int64_t)r * cols + c]);
+        for (; k < k1; ++k) s += bf2f(p[k]);
     }
     part[g][cx] = s;
     __syncthreads();
-    if (g == 0 && c < cols) {
+    if (g == 0 && c < a.rows) {
         float t = part[0][cx];
-        for (int q = 1; q < kColsumGroups; ++q) t += part[q][cx];
-        db[c] = t;
+        for (int q = 1; q < kSumGroups; ++q) t += part[q][cx];
+        a.out[c] = t;
     }
 }
 
-// rows idx[b] of X (FP32) -> bf16 batch; rows idx[b] of T -> FP32 batch
+// the product and tile of a workgroup of a batch; false for the workgroups of the sums
+__device__ inline bool gemm_tile(const GemmBatch& p, int tile, bool& second, int& m0, int& n0)
+{
+    __shared__ float part[kSumGroups][kSumRows];
+    int t = blockIdx.x;
+    const int products = p.tiles[0] + p.tiles[1];
+    if (t >= products + p.sum_blocks) {
+        const int r = (t - products - p.sum_blocks) * kT + threadIdx.x;
+        if (r < p.loss.rows) {
+            const double* q = p.loss.part + (int64_t)r * p.loss.parts;
+            double s = 0.0;
+            for (int c = 0; c < p.loss.parts; ++c) s += q[c];
+            p.loss.row_loss[r] = s;
+        }
+        return false;
+    }
+    if (t >= products) {
+        row_sums(p.sums, t - products, part);
+        return false;
+    }
+    second = t >= p.tiles[0];
+    if (second) t -= p.tiles[0];
+    const int tiles_n = (p.g[second].N + tile - 1) / tile;
+    m0 = t / tiles_n * tile;
+    n0 = t % tiles_n * tile;
+    return true;
+}
+
+// a 32 x 32 tile, a 16 x 16 block per wavefront, operands straight into registers: the
+// next U k steps load while the current U are multiplied
+__global__ __launch_bounds__(kT) void mlp_gemm_small_kernel(GemmBatch p)
+{
+    constexpr int U = 4;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    bool second;
+    int m0, n0;
+    if (!gemm_tile(p, 32, second, m0, n0)) return;
+    const GemmArgs& g = second ? p.g[1] : p.g[0];
+    const int r = lane & 15, kg = lane >> 4;
+    m0 += (wave >> 1) * 16;
+    n0 += (wave & 1) * 16;
+    const uint16_t* a = g.A + (int64_t)min(m0 + r, g.M - 1) * g.lda;
+    const uint16_t* b = g.B + (int64_t)min(n0 + r, g.N - 1) * g.ldb;
+    const int K = g.K;
+    bf16x8 fa[2][U], fb[2][U];
+    auto load = [&](bf16x8 (&va)[U], bf16x8 (&vb)[U], int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            va[u] = ld_frag(a, k + 32 * u + 8 * kg, K);
+            vb[u] = ld_frag(b, k + 32 * u + 8 * kg, K);
+        }
+    };
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto mul = [&](const bf16x8 (&va)[U], const bf16x8 (&vb)[U]) {
+        // steps past K multiply zeros
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[u], vb[u], acc, 0, 0, 0);
+    };
+    load(fa[0], fb[0], 0);
+    for (int k = 0; k < K; k += 64 * U) {
+        load(fa[1], fb[1], k + 32 * U);
+        mul(fa[0], fb[0]);
+        load(fa[0], fb[0], k + 64 * U);
+        mul(fa[1], fb[1]);
+    }
+    // a lane holds C[row0 + t][col], t = 0..3
+    gemm_store(g, acc, m0 + 4 * kg, n0 + r, lane);
+}
+
+// TILE x TILE outputs through LDS, a (TILE / 2)^2 quarter per wavefront; k in steps of
+// 64, the next step's rows in registers during the products of this one
+template <int TILE, int EPI>
+__global__ __launch_bounds__(kT) void mlp_gemm_tile_kernel(GemmBatch p)
+{
+    constexpr int BK = 64, LD = BK + 8;        // padded rows: 16 lanes of a read start in 16 different banks
+    constexpr int NB = TILE / 32;              // 16 x 16 blocks per side of a wavefront's quarter
+    constexpr int NL = TILE * BK / (8 * kT);   // 16-byte runs per thread and operand
+    __shared__ __align__(16) uint16_t As[TILE * LD], Bs[TILE * LD];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    bool second;
+    int m0, n0;
+    if (!gemm_tile(p, TILE, second, m0, n0)) return;
+    const GemmArgs& g = p.g[0];
+    const int r = lane & 15, kg = lane >> 4;
+    const int wm = (wave >> 1) * (TILE / 2), wn = (wave & 1) * (TILE / 2);
+    const int K = g.K;
+    bf16x8 ra[NL], rb[NL];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const int row = (q * kT + tid) / 8, kk = k + (tid & 7) * 8;
+            ra[q] = ld_frag(g.A + (int64_t)min(m0 + row, g.M - 1) * g.lda, kk, K);
+            rb[q] = ld_frag(g.B + (int64_t)min(n0 + row, g.N - 1) * g.ldb, kk, K);
+        }
+    };
+    floatx4 acc[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load(0);
+    for (int k = 0; k < K; k += BK) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const int at = (q * kT + tid) / 8 * LD + (tid & 7) * 8;
+            *reinterpret_cast<bf16x8*>(&As[at]) = ra[q];
+            *reinterpret_cast<bf16x8*>(&Bs[at]) = rb[q];
+        }
+        __syncthreads();
+        if (k + BK < K) load(k + BK);
+#pragma unroll
+        for (int ks = 0; ks < BK; ks += 32) {
+            bf16x8 fa[NB], fb[NB];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                fa[i] = *reinterpret_cast<const bf16x8*>(&As[(wm + 16 * i + r) * LD + ks + 8 * kg]);
+                fb[i] = *reinterpret_cast<const bf16x8*>(&Bs[(wn + 16 * i + r) * LD + ks + 8 * kg]);
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) gemm_store<EPI>(g, acc[i][j], m0 + wm + 16 * i + 4 * kg, n0 + wn + 16 * j + r, lane);
+}
+
+// rows of X (FP32; row b is idx[b], or b without idx) -> bf16 batch and its transpose; rows of T -> FP32 batch
 __global__ __launch_bounds__(kT) void gather_kernel(const float* X, int in, const float* T, int out, const int64_t* idx,
-                                                    int rows, uint16_t* Xb, float* Tb)
+                                                    int rows, uint16_t* Xb, int64_t ldx, uint16_t* XbT, int64_t ldxt,
+                                                    float* Tb, int* ctr)
 {
     const int b = blockIdx.x;
     if (b >= rows) return;
-    const int64_t src = idx[b];
-    for (int c = threadIdx.x; c < in; c += kT) Xb[(int64_t)b * in + c] = f2bf(X[src * in + c]);
+    if (ctr && b == 0 && threadIdx.x == 0) *ctr += 1;
+    const int64_t src = idx ? idx[b] : b;
+    for (int c = threadIdx.x; c < in; c += kT) {
+        const uint16_t h = f2bf(X[src * in + c]);
+        Xb[(int64_t)b * ldx + c] = h;
+        if (XbT) XbT[(int64_t)c * ldxt + b] = h;
+    }
     if (T)
         for (int c = threadIdx.x; c < out; c += kT) Tb[(int64_t)b * out + c] = T[src * out + c];
 }
 
-__global__ __launch_bounds__(kT) void cast_bf16_kernel(const float* x, int64_t n, uint16_t* y)
+// Adam with bias correction on one parameter, and its bf16 rounding
+__device__ inline uint16_t param_step(const ParamArgs& a, float c1, float c2, int64_t i)
 {
-    for (int64_t i = blockIdx.x * (int64_t)kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) y[i] = f2bf(x[i]);
-}
-
-// Adam with bias correction; writes the bf16 copy used by the GEMMs
-__global__ __launch_bounds__(kT) void adam_kernel(float* p, const float* grad, float* m, float* v, int64_t n, float lr,
-                                                  float b1, float b2, float eps, float c1, float c2, uint16_t* p16)
-{
-    for (int64_t i = blockIdx.x * (int64_t)kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) {
-        const float gr = grad[i];
-        const float mi = b1 * m[i] + (1.f - b1) * gr;
-        const float vi = b2 * v[i] + (1.f - b2) * gr * gr;
-        m[i] = mi;
-        v[i] = vi;
-        const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        const float pn = p[i] - upd;
-        p[i] = pn;
-        if (p16) p16[i] = f2bf(pn);
+    float pn = a.p[i];
+    if (a.grad) {
+        const float gr = a.grad[i];
+        const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gr;
+        const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gr * gr;
+        a.m[i] = mi;
+        a.v[i] = vi;
+        const float upd = a.lr * (mi / c1) / (sqrtf(vi / c2) + a.eps);
+        pn = pn - upd;
+        a.p[i] = pn;
     }
+    return f2bf(pn);
 }
 
-// The same update with the bias corrections of step *ctr read from corr[2 *ctr],
-// corr[2 *ctr + 1] (a captured training epoch replays unchanged while the step
-// advances); count_kernel advances *ctr after it.
-__global__ __launch_bounds__(kT) void adam_table_kernel(float* p, const float* grad, float* m, float* v, int64_t n,
-                                                        float lr, float b1, float b2, float eps, const float* corr,
-                                                        const int* ctr, uint16_t* p16)
+// A workgroup owns a 32 x 32 block of one layer's W (or 256 biases): the update runs
+// along the rows of W, the transposed copy leaves through LDS.
+__global__ __launch_bounds__(kT) void params_kernel(ParamArgs a)
 {
-    const int k = *ctr;
-    const float c1 = corr[2 * (int64_t)k], c2 = corr[2 * (int64_t)k + 1];
-    for (int64_t i = blockIdx.x * (int64_t)kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) {
-        const float gr = grad[i];
-        const float mi = b1 * m[i] + (1.f - b1) * gr;
-        const float vi = b2 * v[i] + (1.f - b2) * gr * gr;
-        m[i] = mi;
-        v[i] = vi;
-        const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        const float pn = p[i] - upd;
-        p[i] = pn;
-        if (p16) p16[i] = f2bf(pn);
+    __shared__ uint16_t tile[kParamTile][kParamTile + 1];
+    int l = 0;
+    while (l + 1 < a.nlayers && a.layers[l + 1].tile0 <= (int)blockIdx.x) ++l;
+    const LayerDesc d = a.layers[l];
+    const int t = blockIdx.x - d.tile0;
+    float c1 = a.c1, c2 = a.c2;
+    if (a.corr) {
+        const int64_t k = *a.ctr;
+        c1 = a.corr[2 * k];
+        c2 = a.corr[2 * k + 1];
     }
-}
-
-__global__ void count_kernel(int* ctr)
-{
-    if (threadIdx.x == 0) *ctr += 1;
+    const int tiles_i = (d.din + kParamTile - 1) / kParamTile, tiles_o = (d.dout + kParamTile - 1) / kParamTile;
+    if (t >= tiles_i * tiles_o) {
+        const int o = (t - tiles_i * tiles_o) * kT + threadIdx.x;
+        if (o < d.dout) (void)param_step(a, c1, c2, d.boff + o);
+        return;
+    }
+    const int i0 = t % tiles_i * kParamTile, o0 = t / tiles_i * kParamTile;
+    const int x = threadIdx.x % kParamTile, y = threadIdx.x / kParamTile;
+    constexpr int RY = kT / kParamTile;
+    for (int q = y; q < kParamTile; q += RY) {
+        const int o = o0 + q, i = i0 + x;
+        if (o < d.dout && i < d.din) {
+            const uint16_t h = param_step(a, c1, c2, d.woff + (int64_t)o * d.din + i);
+            a.p16[d.w16 + (int64_t)o * d.ldw + i] = h;
+            tile[q][x] = h;
+        }
+    }
+    __syncthreads();
+    for (int q = y; q < kParamTile; q += RY) {
+        const int i = i0 + q, o = o0 + x;
+        if (o < d.dout && i < d.din) a.pt16[d.wt16 + (int64_t)i * d.ldwt + o] = tile[x][q];
+    }
 }
 
 // per row: mean over the E ensemble members and, for each of nblk equal blocks
@@ -399,7 +417,7 @@ __global__ __launch_bounds__(kT) void ensemble_stats_kernel(const float* Ys, int
             const float d = Ys[e * estride + o] - mu;
             var += d * d;
         }
-        mean[o] = mu;
+        if (mean) mean[o] = mu;
         acc += var / (float)E;
     }
     s[threadIdx.x] = acc;
@@ -411,83 +429,74 @@ __global__ __launch_bounds__(kT) void ensemble_stats_kernel(const float* Ys, int
     if (threadIdx.x == 0) spread[(int64_t)r * nblk + b] = sqrtf(s[0] / (float)bw);
 }
 
-int blocks_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(4096, (n + kT - 1) / kT)); }
+}  // namespace
+
+namespace {
+
+template <int TILE>
+void launch_tile(const GemmBatch& p, dim3 grid, hipStream_t s)
+{
+    switch (p.g[0].epi) {
+    case EPI_STORE_F32: hipLaunchKernelGGL((mlp_gemm_tile_kernel<TILE, EPI_STORE_F32>), grid, dim3(kT), 0, s, p); break;
+    case EPI_BIAS_F32: hipLaunchKernelGGL((mlp_gemm_tile_kernel<TILE, EPI_BIAS_F32>), grid, dim3(kT), 0, s, p); break;
+    case EPI_BIAS_GELU: hipLaunchKernelGGL((mlp_gemm_tile_kernel<TILE, EPI_BIAS_GELU>), grid, dim3(kT), 0, s, p); break;
+    case EPI_GELU_BWD: hipLaunchKernelGGL((mlp_gemm_tile_kernel<TILE, EPI_GELU_BWD>), grid, dim3(kT), 0, s, p); break;
+    default: hipLaunchKernelGGL((mlp_gemm_tile_kernel<TILE, EPI_MSE>), grid, dim3(kT), 0, s, p); break;
+    }
+}
 
 }  // namespace
 
-template <int EPI>
-void launch_v2(const GemmArgs& g, bool ak, bool bk, dim3 grid, hipStream_t s)
+hipError_t launch_gemm_bf16(const GemmArgs& a, const GemmArgs* b, const SumArgs& sums, const LossArgs& loss,
+                            hipStream_t s)
 {
-    if (ak && bk) hipLaunchKernelGGL((gemm_bf16_v2_kernel<EPI, true, true>), grid, dim3(kT), 0, s, g);
-    else if (ak) hipLaunchKernelGGL((gemm_bf16_v2_kernel<EPI, true, false>), grid, dim3(kT), 0, s, g);
-    else if (bk) hipLaunchKernelGGL((gemm_bf16_v2_kernel<EPI, false, true>), grid, dim3(kT), 0, s, g);
-    else hipLaunchKernelGGL((gemm_bf16_v2_kernel<EPI, false, false>), grid, dim3(kT), 0, s, g);
-}
-
-// the 16-byte staging needs: K a multiple of 8; a unit stride along k or along
-// m (A) / n (B) with the other stride a multiple of 8; for m- / n-runs, M / N a
-// multiple of 8; base addresses on 16 bytes
-bool v2_ok(const GemmArgs& g, bool& ak, bool& bk)
-{
-    if (g.K % 8 != 0) return false;
-    if (((uintptr_t)g.A | (uintptr_t)g.B) % 16 != 0) return false;
-    if (g.sak == 1 && g.sam % 8 == 0) ak = true;
-    else if (g.sam == 1 && g.sak % 8 == 0 && g.M % 8 == 0) ak = false;
-    else return false;
-    if (g.sbk == 1 && g.sbn % 8 == 0) bk = true;
-    else if (g.sbn == 1 && g.sbk % 8 == 0 && g.N % 8 == 0) bk = false;
-    else return false;
-    return true;
-}
-
-hipError_t launch_gemm_bf16(const GemmArgs& g, int epi, hipStream_t s)
-{
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return hipErrorInvalidValue;
-    const dim3 grid((g.N + kTN - 1) / kTN, (g.M + kTM - 1) / kTM);
-    bool ak = false, bk = false;
-    if (v2_ok(g, ak, bk)) {
-        switch (epi) {
-        case EPI_STORE_F32: launch_v2<EPI_STORE_F32>(g, ak, bk, grid, s); break;
-        case EPI_BIAS_F32: launch_v2<EPI_BIAS_F32>(g, ak, bk, grid, s); break;
-        case EPI_BIAS_GELU: launch_v2<EPI_BIAS_GELU>(g, ak, bk, grid, s); break;
-        case EPI_GELU_BWD: launch_v2<EPI_GELU_BWD>(g, ak, bk, grid, s); break;
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
+    auto bad = [](const GemmArgs& g) {
+        return g.M <= 0 || g.N <= 0 || g.K <= 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.ld16t % 8 != 0 ||
+               ((uintptr_t)g.A | (uintptr_t)g.B) % 16 != 0 || (uintptr_t)g.C16T % 8 != 0;
+    };
+    if (bad(a) || (b && bad(*b))) return hipErrorInvalidValue;
+    auto tiles = [](const GemmArgs& g, int t) { return (int64_t)((g.M + t - 1) / t) * ((g.N + t - 1) / t); };
+    // the widest tile that still gives each of the 256 CUs a workgroup
+    auto width = [&](const GemmArgs& g) { return tiles(g, 128) >= 256 ? 128 : (tiles(g, 64) >= 256 ? 64 : 32); };
+    if (b && (width(a) != 32 || width(*b) != 32)) {
+        const hipError_t e = launch_gemm_bf16(a, nullptr, sums, loss, s);
+        return e != hipSuccess ? e : launch_gemm_bf16(*b, nullptr, SumArgs{}, LossArgs{}, s);
     }
-    switch (epi) {
-    case EPI_STORE_F32: hipLaunchKernelGGL(gemm_bf16_kernel<EPI_STORE_F32>, grid, dim3(kT), 0, s, g); break;
-    case EPI_BIAS_F32: hipLaunchKernelGGL(gemm_bf16_kernel<EPI_BIAS_F32>, grid, dim3(kT), 0, s, g); break;
-    case EPI_BIAS_GELU: hipLaunchKernelGGL(gemm_bf16_kernel<EPI_BIAS_GELU>, grid, dim3(kT), 0, s, g); break;
-    case EPI_GELU_BWD: hipLaunchKernelGGL(gemm_bf16_kernel<EPI_GELU_BWD>, grid, dim3(kT), 0, s, g); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_mse_grad(const float* Y, const float* T, int rows, int cols, float scale, uint16_t* dY,
-                           double* row_loss, hipStream_t s)
-{
-    hipLaunchKernelGGL(mse_grad_kernel, dim3(rows), dim3(kT), 0, s, Y, T, rows, cols, scale, dY, row_loss);
-    return hipGetLastError();
-}
-
-hipError_t launch_colsum(const uint16_t* dZ, int rows, int cols, float* db, hipStream_t s)
-{
-    hipLaunchKernelGGL(colsum_kernel, dim3((cols + kColsumCols - 1) / kColsumCols), dim3(kT), 0, s, dZ, rows, cols, db);
+    const int t = width(a);
+    GemmBatch p{};
+    p.g[0] = a;
+    if (b) p.g[1] = *b;
+    p.sums = sums;
+    p.sum_blocks = (sums.rows + kSumRows - 1) / kSumRows;
+    p.loss = loss;
+    const int64_t na = tiles(a, t), nb = b ? tiles(*b, t) : 0;
+    const int64_t blocks = na + nb + p.sum_blocks + (loss.rows + kT - 1) / kT;
+    if (blocks > 0x7fffff) return hipErrorInvalidValue;   // grid x block below 2^32
+    p.tiles[0] = (int)na;
+    p.tiles[1] = (int)nb;
+    const dim3 grid((unsigned)blocks);
+    if (t == 128) launch_tile<128>(p, grid, s);
+    else if (t == 64) launch_tile<64>(p, grid, s);
+    else hipLaunchKernelGGL(mlp_gemm_small_kernel, grid, dim3(kT), 0, s, p);
     return hipGetLastError();
 }
 
 hipError_t launch_gather(const float* X, int in, const float* T, int out, const int64_t* idx, int rows, uint16_t* Xb,
-                         float* Tb, hipStream_t s)
+                         int64_t ldx, uint16_t* XbT, int64_t ldxt, float* Tb, int* ctr, hipStream_t s)
 {
-    hipLaunchKernelGGL(gather_kernel, dim3(rows), dim3(kT), 0, s, X, in, T, out, idx, rows, Xb, Tb);
+    hipLaunchKernelGGL(gather_kernel, dim3(rows), dim3(kT), 0, s, X, in, T, out, idx, rows, Xb, ldx, XbT, ldxt, Tb, ctr);
     return hipGetLastError();
 }
 
-hipError_t launch_cast_bf16(const float* x, int64_t n, uint16_t* y, hipStream_t s)
+hipError_t launch_cast_rows(const float* X, int in, int rows, uint16_t* Xb, int64_t ldx, uint16_t* XbT, int64_t ldxt,
+                            hipStream_t s)
 {
-    hipLaunchKernelGGL(cast_bf16_kernel, dim3(blocks_for(n)), dim3(kT), 0, s, x, n, y);
+    return launch_gather(X, in, nullptr, 0, nullptr, rows, Xb, ldx, XbT, ldxt, nullptr, nullptr, s);
+}
+
+hipError_t launch_params(const ParamArgs& a, hipStream_t s)
+{
+    hipLaunchKernelGGL(params_kernel, dim3(a.blocks), dim3(kT), 0, s, a);
     return hipGetLastError();
 }
 
@@ -501,32 +510,10 @@ hipError_t launch_ensemble_stats(const float* Ys, int E, int64_t estride, int ro
     return hipGetLastError();
 }
 
-hipError_t launch_adam(float* p, const float* grad, float* m, float* v, int64_t n, float lr, float b1, float b2,
-                       float eps, int step, uint16_t* p16, hipStream_t s)
-{
-    float c1, c2;
-    adam_corrections(b1, b2, step, &c1, &c2);
-    hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(n)), dim3(kT), 0, s, p, grad, m, v, n, lr, b1, b2, eps, c1, c2,
-                       p16);
-    return hipGetLastError();
-}
-
-hipError_t adam_corrections(float b1, float b2, int step, float* c1, float* c2)
+void adam_corrections(float b1, float b2, int step, float* c1, float* c2)
 {
     *c1 = 1.f - powf(b1, (float)step);
     *c2 = 1.f - powf(b2, (float)step);
-    return hipSuccess;
-}
-
-hipError_t launch_adam_table(float* p, const float* grad, float* m, float* v, int64_t n, float lr, float b1, float b2,
-                             float eps, const float* corr, int* ctr, uint16_t* p16, hipStream_t s)
-{
-    hipLaunchKernelGGL(adam_table_kernel, dim3(blocks_for(n)), dim3(kT), 0, s, p, grad, m, v, n, lr, b1, b2, eps, corr,
-                       ctr, p16);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(count_kernel, dim3(1), dim3(64), 0, s, ctr);
-    return hipGetLastError();
 }
 
 }  // namespace leo2d

@@ -31,12 +31,17 @@ struct leo2d_mlp {
     std::vector<int> dims;                 // in, hidden x layers, out
     std::vector<int64_t> woff, boff;       // offsets of W_l and b_l in the flat parameter vector
     int64_t nparams = 0;
-    DevBuf P32, P16, G, Mom, Var;          // master weights, bf16 copy, gradient, Adam moments
+    DevBuf P32, G, Mom, Var;               // master weights, gradient, Adam moments
+    DevBuf P16, PT16, descs;               // bf16 copies of every W and W^T, their layout (mlp.h)
+    std::vector<leo2d::LayerDesc> layer;
+    int param_blocks = 0;
     int64_t adam_step = 0;
     // batch workspace
     int cap = 0;
-    DevBuf X16, Y, T, dY16, dZa, dZb, rowloss, xin, idx;
-    std::vector<DevBuf> Z, H;              // per hidden layer: pre-activation FP32, activation bf16
+    int64_t ldt = 0;                       // leading dimension of the transposed batch operands
+    DevBuf X16, XT16, Y, T, lossparts, rowloss, xin;
+    std::vector<DevBuf> Z, H, HT;          // per hidden layer: pre-activation FP32, activation bf16 and its transpose
+    DevBuf dZ[2], dZT[2];                  // gradients of two neighbouring layers' inputs, bf16, and their transposes
 
     int layers() const { return (int)dims.size() - 1; }
     int in() const { return dims.front(); }
@@ -85,118 +90,192 @@ void to_device_f32(DevBuf& b, const std::vector<float>& v, hipStream_t s)
     check(hipMemcpyAsync(b.p, v.data(), sizeof(float) * v.size(), hipMemcpyHostToDevice, s), "adam corrections");
 }
 
+// Buffers for batches of up to `rows` rows.  bf16 operands have k contiguous on both
+// sides of a product (mlp.h): activations and gradients in both orders, leading
+// dimensions padded to 8.
 void ensure_capacity(leo2d_mlp* m, int rows)
 {
     if (rows <= m->cap) return;
     leo2d::DevPool::Use own(&m->pool);   // the network's buffers, whichever network's call this is
     const int cap = std::max(rows, 256);
-    const int hmax = *std::max_element(m->dims.begin() + 1, m->dims.end() - 1);
-    dalloc(m->X16, sizeof(uint16_t) * (size_t)cap * m->in(), "mlp inputs");
+    const int64_t ldt = leo2d::pad8(cap);
+    const int64_t widest = leo2d::pad8(*std::max_element(m->dims.begin() + 1, m->dims.end()));
+    auto b16 = [&](DevBuf& b, int64_t elems, const char* what) { dalloc(b, sizeof(uint16_t) * (size_t)elems, what); };
+    b16(m->X16, cap * leo2d::pad8(m->in()), "mlp inputs");
+    b16(m->XT16, ldt * m->in(), "mlp inputs");
     dalloc(m->xin, sizeof(float) * (size_t)cap * m->in(), "mlp inputs");
     dalloc(m->Y, sizeof(float) * (size_t)cap * m->out(), "mlp outputs");
     dalloc(m->T, sizeof(float) * (size_t)cap * m->out(), "mlp targets");
-    dalloc(m->dY16, sizeof(uint16_t) * (size_t)cap * m->out(), "mlp output gradient");
-    dalloc(m->dZa, sizeof(uint16_t) * (size_t)cap * hmax, "mlp gradient");
-    dalloc(m->dZb, sizeof(uint16_t) * (size_t)cap * hmax, "mlp gradient");
+    for (int q = 0; q < 2; ++q) {
+        b16(m->dZ[q], cap * widest, "mlp gradient");
+        b16(m->dZT[q], ldt * widest, "mlp gradient");
+    }
+    dalloc(m->lossparts, sizeof(double) * (size_t)cap * ((m->out() + 15) / 16), "mlp loss");
     dalloc(m->rowloss, sizeof(double) * (size_t)cap, "mlp loss");
     m->Z.clear();
     m->H.clear();
+    m->HT.clear();
     m->Z.resize(m->layers() - 1);
     m->H.resize(m->layers() - 1);
+    m->HT.resize(m->layers() - 1);
     for (int l = 0; l + 1 < m->layers(); ++l) {
         dalloc(m->Z[l], sizeof(float) * (size_t)cap * m->dims[l + 1], "mlp pre-activations");
-        dalloc(m->H[l], sizeof(uint16_t) * (size_t)cap * m->dims[l + 1], "mlp activations");
+        b16(m->H[l], cap * leo2d::pad8(m->dims[l + 1]), "mlp activations");
+        b16(m->HT[l], ldt * m->dims[l + 1], "mlp activations");
     }
     m->cap = cap;
+    m->ldt = ldt;
 }
 
-// Y[rows][out] = MLP(X16[rows][in]) ; Y (and X16, by default the network's own) may
-// point outside the workspace
+const leo2d::SumArgs kNoSums{nullptr, 0, 0, 0, nullptr};
+const leo2d::LossArgs kNoLoss{nullptr, 0, 0, nullptr};
+
+// the product of layer l's inputs with W^T, up to its epilogue
+leo2d::GemmArgs layer_product(leo2d_mlp* m, int l, const uint16_t* hin, int rows)
+{
+    leo2d::GemmArgs g{};
+    g.A = hin;
+    g.lda = leo2d::pad8(m->dims[l]);
+    g.B = bf(m->P16, m->layer[(size_t)l].w16);
+    g.ldb = m->layer[(size_t)l].ldw;
+    g.M = rows;
+    g.N = m->dims[l + 1];
+    g.K = m->dims[l];
+    g.bias = f32(m->P32, m->boff[l]);
+    g.ldc = m->dims[l + 1];
+    return g;
+}
+
+// The hidden layers on X16 (by default the network's own); train: with what the
+// backward pass needs.  Returns the last hidden activations.
+const uint16_t* hidden_layers(leo2d_mlp* m, int rows, const uint16_t* X16, bool train)
+{
+    const uint16_t* hin = X16 ? X16 : bf(m->X16);
+    for (int l = 0; l + 1 < m->layers(); ++l) {
+        leo2d::GemmArgs g = layer_product(m, l, hin, rows);
+        g.epi = leo2d::EPI_BIAS_GELU;
+        g.C16 = bfw(m->H[l]);
+        g.ld16 = leo2d::pad8(g.N);
+        if (train) {
+            g.Z = f32(m->Z[l]);
+            g.C16T = bfw(m->HT[l]);
+            g.ld16t = m->ldt;
+        }
+        check(leo2d::launch_gemm_bf16(g, nullptr, kNoSums, kNoLoss, m->stream), "mlp forward");
+        hin = bf(m->H[l]);
+    }
+    return hin;
+}
+
+// Y[rows][out] = MLP(X16[rows][in]) ; Y and X16 may point outside the workspace
 void forward(leo2d_mlp* m, int rows, float* Y, const uint16_t* X16 = nullptr)
 {
-    hipStream_t s = m->stream;
-    const uint16_t* hin = X16 ? X16 : bf(m->X16);
-    for (int l = 0; l < m->layers(); ++l) {
-        const int din = m->dims[l], dout = m->dims[l + 1];
-        leo2d::GemmArgs g{};
-        g.A = hin;
-        g.sam = din;
-        g.sak = 1;
-        g.B = bf(m->P16, m->woff[l]);   // B(k, n) = W[n][k]
-        g.sbk = 1;
-        g.sbn = din;
-        g.M = rows;
-        g.N = dout;
-        g.K = din;
-        g.bias = f32(m->P32, m->boff[l]);
-        g.scm = dout;
-        if (l + 1 < m->layers()) {
-            g.Z = f32(m->Z[l]);
-            g.C16 = bfw(m->H[l]);
-            check(leo2d::launch_gemm_bf16(g, leo2d::EPI_BIAS_GELU, s), "mlp forward");
-            hin = bf(m->H[l]);
-        } else {
-            g.C32 = Y;
-            check(leo2d::launch_gemm_bf16(g, leo2d::EPI_BIAS_F32, s), "mlp forward");
-        }
-    }
+    const uint16_t* hin = hidden_layers(m, rows, X16, false);
+    leo2d::GemmArgs g = layer_product(m, m->layers() - 1, hin, rows);
+    g.epi = leo2d::EPI_BIAS_F32;
+    g.C32 = Y;
+    check(leo2d::launch_gemm_bf16(g, nullptr, kNoSums, kNoLoss, m->stream), "mlp forward");
 }
 
-// gradient of the mean squared error over rows x out into m->G; row losses in
-// row_loss (m->rowloss when null)
-void backward(leo2d_mlp* m, int rows, double* row_loss = nullptr)
+// gradient of the mean squared error over rows x out into m->G, from X16, XT16 and
+// T; row losses in row_loss (m->rowloss when null)
+void gradients(leo2d_mlp* m, int rows, double* row_loss = nullptr)
 {
     hipStream_t s = m->stream;
     const int L = m->layers();
-    check(leo2d::launch_mse_grad(f32(m->Y), f32(m->T), rows, m->out(), 2.0f / ((float)rows * (float)m->out()),
-                                 bfw(m->dY16), row_loss ? row_loss : static_cast<double*>(m->rowloss.p), s),
-          "mlp loss");
-    const uint16_t* gz = bf(m->dY16);
-    DevBuf* next = &m->dZa;
+    const uint16_t* hin = hidden_layers(m, rows, nullptr, true);
+    leo2d::GemmArgs o = layer_product(m, L - 1, hin, rows);
+    o.epi = leo2d::EPI_MSE;
+    o.T = f32(m->T);
+    o.scale = 2.0f / ((float)rows * (float)m->out());
+    o.C16 = bfw(m->dZ[0]);
+    o.ld16 = leo2d::pad8(o.N);
+    o.C16T = bfw(m->dZT[0]);
+    o.ld16t = m->ldt;
+    o.loss = static_cast<double*>(m->lossparts.p);
+    check(leo2d::launch_gemm_bf16(o, nullptr, kNoSums, kNoLoss, s), "mlp loss");
+    leo2d::LossArgs loss{o.loss, rows, (m->out() + 15) / 16, row_loss ? row_loss : static_cast<double*>(m->rowloss.p)};
+    int cur = 0;
     for (int l = L - 1; l >= 0; --l) {
         const int din = m->dims[l], dout = m->dims[l + 1];
-        const uint16_t* hin = l == 0 ? bf(m->X16) : bf(m->H[l - 1]);
-        // dW_l[o][i] = sum_b dZ[b][o] Hin[b][i]
+        // dW_l[o][i] = sum_b dZ[b][o] Hin[b][i], db_l[o] = sum_b dZ[b][o]
         leo2d::GemmArgs gw{};
-        gw.A = gz;
-        gw.sam = 1;
-        gw.sak = dout;
-        gw.B = hin;
-        gw.sbk = din;
-        gw.sbn = 1;
+        gw.epi = leo2d::EPI_STORE_F32;
+        gw.A = bf(m->dZT[cur]);
+        gw.lda = m->ldt;
+        gw.B = l == 0 ? bf(m->XT16) : bf(m->HT[l - 1]);
+        gw.ldb = m->ldt;
         gw.M = dout;
         gw.N = din;
         gw.K = rows;
         gw.C32 = f32(m->G, m->woff[l]);
-        gw.scm = din;
-        check(leo2d::launch_gemm_bf16(gw, leo2d::EPI_STORE_F32, s), "mlp weight gradient");
-        check(leo2d::launch_colsum(gz, rows, dout, f32(m->G, m->boff[l]), s), "mlp bias gradient");
-        if (l == 0) break;
+        gw.ldc = din;
+        const leo2d::SumArgs db{gw.A, gw.lda, dout, rows, f32(m->G, m->boff[l])};
         // dZ_{l-1} = (dZ_l W_l) * gelu'(Z_{l-1})
         leo2d::GemmArgs gx{};
-        gx.A = gz;
-        gx.sam = dout;
-        gx.sak = 1;
-        gx.B = bf(m->P16, m->woff[l]);   // B(k=o, n=i) = W[o][i]
-        gx.sbk = din;
-        gx.sbn = 1;
-        gx.M = rows;
-        gx.N = din;
-        gx.K = dout;
-        gx.Z = f32(m->Z[l - 1]);
-        gx.C16 = bfw(*next);
-        gx.scm = din;
-        check(leo2d::launch_gemm_bf16(gx, leo2d::EPI_GELU_BWD, s), "mlp input gradient");
-        gz = bf(*next);
-        next = next == &m->dZa ? &m->dZb : &m->dZa;
+        if (l > 0) {
+            gx.epi = leo2d::EPI_GELU_BWD;
+            gx.A = bf(m->dZ[cur]);
+            gx.lda = leo2d::pad8(dout);
+            gx.B = bf(m->PT16, m->layer[(size_t)l].wt16);
+            gx.ldb = m->layer[(size_t)l].ldwt;
+            gx.M = rows;
+            gx.N = din;
+            gx.K = dout;
+            gx.Z = f32(m->Z[l - 1]);
+            gx.ldc = din;
+            gx.C16 = bfw(m->dZ[1 - cur]);
+            gx.ld16 = leo2d::pad8(din);
+            gx.C16T = bfw(m->dZT[1 - cur]);
+            gx.ld16t = m->ldt;
+        }
+        check(leo2d::launch_gemm_bf16(gw, l > 0 ? &gx : nullptr, db, l == L - 1 ? loss : kNoLoss, s), "mlp gradient");
+        cur = 1 - cur;
     }
 }
 
-void upload_inputs(leo2d_mlp* m, const float* x, int rows)
+leo2d::ParamArgs param_args(leo2d_mlp* m)
+{
+    leo2d::ParamArgs a{};
+    a.layers = static_cast<const leo2d::LayerDesc*>(m->descs.p);
+    a.nlayers = m->layers();
+    a.blocks = m->param_blocks;
+    a.p = f32(m->P32);
+    a.p16 = bfw(m->P16);
+    a.pt16 = bfw(m->PT16);
+    return a;
+}
+
+// one Adam step on the gradient in m->G
+leo2d::ParamArgs adam_args(leo2d_mlp* m, const leo2d_mlp_train_params* p)
+{
+    leo2d::ParamArgs a = param_args(m);
+    a.grad = f32(m->G);
+    a.m = f32(m->Mom);
+    a.v = f32(m->Var);
+    a.lr = p->lr;
+    a.b1 = p->beta1;
+    a.b2 = p->beta2;
+    a.eps = p->eps;
+    return a;
+}
+
+// one mini-batch: rows idx[0 .. rows) of the training set, gradient and row losses
+void batch_gradients(leo2d_mlp* m, const float* X, const float* T, const int64_t* idx, int rows, double* row_loss, int* ctr)
+{
+    check(leo2d::launch_gather(X, m->in(), T, m->out(), idx, rows, bfw(m->X16), leo2d::pad8(m->in()), bfw(m->XT16), m->ldt,
+                               f32(m->T), ctr, m->stream),
+          "batch gather");
+    gradients(m, rows, row_loss);
+}
+
+void upload_inputs(leo2d_mlp* m, const float* x, int rows, bool train = false)
 {
     check(hipMemcpyAsync(m->xin.p, x, sizeof(float) * (size_t)rows * m->in(), hipMemcpyHostToDevice, m->stream),
           "mlp inputs");
-    check(leo2d::launch_cast_bf16(f32(m->xin), (int64_t)rows * m->in(), bfw(m->X16), m->stream), "mlp inputs");
+    check(leo2d::launch_cast_rows(f32(m->xin), m->in(), rows, bfw(m->X16), leo2d::pad8(m->in()),
+                                  train ? bfw(m->XT16) : nullptr, m->ldt, m->stream),
+          "mlp inputs");
 }
 
 // Fourier features of one configuration (b1, b2, exx, eyy, exy, theta in degrees):
@@ -267,12 +346,27 @@ int leo2d_mlp_create(int32_t device, const leo2d_mlp_desc* d, leo2d_mlp** out)
         m->dims.push_back(d->in);
         for (int l = 0; l < d->layers; ++l) m->dims.push_back(d->hidden);
         m->dims.push_back(d->out);
-        int64_t off = 0;
+        int64_t off = 0, off16 = 0, offt16 = 0;
         for (int l = 0; l < m->layers(); ++l) {
+            const int din = m->dims[l], dout = m->dims[l + 1];
+            leo2d::LayerDesc d{};
+            d.din = din;
+            d.dout = dout;
+            d.ldw = leo2d::pad8(din);
+            d.ldwt = leo2d::pad8(dout);
+            d.woff = off;
             m->woff.push_back(off);
-            off += (int64_t)m->dims[l + 1] * m->dims[l];
+            off += (int64_t)dout * din;
+            d.boff = off;
             m->boff.push_back(off);
-            off += m->dims[l + 1];
+            off += dout;
+            d.w16 = off16;
+            off16 += dout * d.ldw;
+            d.wt16 = offt16;
+            offt16 += din * d.ldwt;
+            d.tile0 = m->param_blocks;
+            m->param_blocks += leo2d::param_tiles(din, dout);
+            m->layer.push_back(d);
         }
         m->nparams = off;
         // Glorot-uniform weights, zero biases
@@ -284,12 +378,17 @@ int leo2d_mlp_create(int32_t device, const leo2d_mlp_desc* d, leo2d_mlp** out)
             for (int64_t q = 0; q < (int64_t)m->dims[l + 1] * m->dims[l]; ++q) p[m->woff[l] + q] = (float)U(rng);
         }
         dalloc(m->P32, sizeof(float) * off, "mlp weights");
-        dalloc(m->P16, sizeof(uint16_t) * off, "mlp weights");
+        dalloc(m->P16, sizeof(uint16_t) * off16, "mlp weights");
+        dalloc(m->PT16, sizeof(uint16_t) * offt16, "mlp weights");
+        dalloc(m->descs, sizeof(leo2d::LayerDesc) * m->layer.size(), "mlp layers");
+        check(hipMemcpyAsync(m->descs.p, m->layer.data(), sizeof(leo2d::LayerDesc) * m->layer.size(), hipMemcpyHostToDevice,
+                             m->stream),
+              "mlp layers");
         dalloc(m->G, sizeof(float) * off, "mlp gradient");
         dalloc(m->Mom, sizeof(float) * off, "mlp optimiser");
         dalloc(m->Var, sizeof(float) * off, "mlp optimiser");
         check(hipMemcpyAsync(m->P32.p, p.data(), sizeof(float) * off, hipMemcpyHostToDevice, m->stream), "mlp init");
-        check(leo2d::launch_cast_bf16(f32(m->P32), off, bfw(m->P16), m->stream), "mlp init");
+        check(leo2d::launch_params(param_args(m), m->stream), "mlp init");
         check(hipMemsetAsync(m->Mom.p, 0, sizeof(float) * off, m->stream), "mlp init");
         check(hipMemsetAsync(m->Var.p, 0, sizeof(float) * off, m->stream), "mlp init");
         check(hipStreamSynchronize(m->stream), "mlp init");
@@ -329,7 +428,7 @@ int leo2d_mlp_set_params(leo2d_mlp* m, const float* p)
     if (!m || !p) return LEO2D_ERR_ARG;
     return guarded(m, [&]() {
         check(hipMemcpyAsync(m->P32.p, p, sizeof(float) * m->nparams, hipMemcpyHostToDevice, m->stream), "mlp params");
-        check(leo2d::launch_cast_bf16(f32(m->P32), m->nparams, bfw(m->P16), m->stream), "mlp params");
+        check(leo2d::launch_params(param_args(m), m->stream), "mlp params");
         check(hipMemsetAsync(m->Mom.p, 0, sizeof(float) * m->nparams, m->stream), "mlp params");
         check(hipMemsetAsync(m->Var.p, 0, sizeof(float) * m->nparams, m->stream), "mlp params");
         m->adam_step = 0;
@@ -362,11 +461,10 @@ int leo2d_mlp_gradients(leo2d_mlp* m, const float* x, const float* t, int32_t n,
     if (!m || !x || !t || n <= 0) return LEO2D_ERR_ARG;
     return guarded(m, [&]() {
         ensure_capacity(m, n);
-        upload_inputs(m, x, n);
+        upload_inputs(m, x, n, true);
         check(hipMemcpyAsync(m->T.p, t, sizeof(float) * (size_t)n * m->out(), hipMemcpyHostToDevice, m->stream),
               "mlp targets");
-        forward(m, n, f32(m->Y));
-        backward(m, n);
+        gradients(m, n);
         std::vector<double> rl(n);
         check(hipMemcpyAsync(rl.data(), m->rowloss.p, sizeof(double) * n, hipMemcpyDeviceToHost, m->stream), "loss");
         if (grad)
@@ -402,19 +500,12 @@ int leo2d_mlp_train(leo2d_mlp* m, const float* x, const float* t, int64_t n, con
             check(hipMemcpyAsync(idx.p, order.data(), sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, s), "order");
             for (int64_t b0 = 0; b0 < n; b0 += B) {
                 const int rows = (int)std::min<int64_t>(B, n - b0);
-                check(leo2d::launch_gather(static_cast<const float*>(X.p), m->in(), static_cast<const float*>(T.p),
-                                           m->out(), static_cast<const int64_t*>(idx.p) + b0, rows, bfw(m->X16),
-                                           f32(m->T), s),
-                      "batch gather");
-                forward(m, rows, f32(m->Y));
-                backward(m, rows);
-                check(hipMemcpyAsync(static_cast<double*>(losses.p) + b0, m->rowloss.p, sizeof(double) * rows,
-                                     hipMemcpyDeviceToDevice, s),
-                      "loss");
+                batch_gradients(m, static_cast<const float*>(X.p), static_cast<const float*>(T.p),
+                                static_cast<const int64_t*>(idx.p) + b0, rows, static_cast<double*>(losses.p) + b0, nullptr);
                 ++m->adam_step;
-                check(leo2d::launch_adam(f32(m->P32), f32(m->G), f32(m->Mom), f32(m->Var), m->nparams, p->lr, p->beta1,
-                                         p->beta2, p->eps, (int)m->adam_step, bfw(m->P16), s),
-                      "adam");
+                leo2d::ParamArgs pa = adam_args(m, p);
+                leo2d::adam_corrections(p->beta1, p->beta2, (int)m->adam_step, &pa.c1, &pa.c2);
+                check(leo2d::launch_params(pa, s), "adam");
             }
             check(hipMemcpyAsync(rl.data(), losses.p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, s), "loss");
             check(hipStreamSynchronize(s), "epoch");
@@ -483,8 +574,8 @@ int leo2d_mlp_train_ensemble(leo2d_mlp* const* nets, int32_t count, const float*
                     leo2d::adam_corrections(p->beta1, p->beta2, (int)(m->adam_step + 1 + i), &corr[2 * (size_t)i],
                                             &corr[2 * (size_t)i + 1]);
                 to_device_f32(q.corr, corr, s);
-                const int zero = 0;
-                check(hipMemcpyAsync(q.ctr.p, &zero, sizeof(int), hipMemcpyHostToDevice, s), "adam step");
+                const int before = -1;   // the gather of a step advances it
+                check(hipMemcpyAsync(q.ctr.p, &before, sizeof(int), hipMemcpyHostToDevice, s), "adam step");
                 check(hipStreamSynchronize(s), "training setup");
                 q.order.resize((size_t)n);
                 std::iota(q.order.begin(), q.order.end(), (int64_t)0);
@@ -496,17 +587,13 @@ int leo2d_mlp_train_ensemble(leo2d_mlp* const* nets, int32_t count, const float*
                 try {
                     for (int64_t b0 = 0; b0 < n; b0 += B) {
                         const int rows = (int)std::min<int64_t>(B, n - b0);
-                        check(leo2d::launch_gather(static_cast<const float*>(X.p), m->in(),
-                                                   static_cast<const float*>(T.p), m->out(),
-                                                   static_cast<const int64_t*>(q.idx.p) + b0, rows, bfw(m->X16),
-                                                   f32(m->T), s),
-                              "batch gather");
-                        forward(m, rows, f32(m->Y));
-                        backward(m, rows, static_cast<double*>(q.loss.p) + b0);
-                        check(leo2d::launch_adam_table(f32(m->P32), f32(m->G), f32(m->Mom), f32(m->Var), m->nparams,
-                                                       p->lr, p->beta1, p->beta2, p->eps, f32(q.corr),
-                                                       static_cast<int*>(q.ctr.p), bfw(m->P16), s),
-                              "adam");
+                        batch_gradients(m, static_cast<const float*>(X.p), static_cast<const float*>(T.p),
+                                        static_cast<const int64_t*>(q.idx.p) + b0, rows,
+                                        static_cast<double*>(q.loss.p) + b0, static_cast<int*>(q.ctr.p));
+                        leo2d::ParamArgs pa = adam_args(m, p);
+                        pa.corr = f32(q.corr);
+                        pa.ctr = static_cast<const int*>(q.ctr.p);
+                        check(leo2d::launch_params(pa, s), "adam");
                     }
                 } catch (...) {
                     (void)hipStreamEndCapture(s, &graph);
@@ -566,14 +653,14 @@ int leo2d_mlp_ensemble(leo2d_mlp* const* nets, int32_t count, const float* x, in
         if (!nets[e] || nets[e]->dims != m0->dims || nets[e]->device != m0->device) return LEO2D_ERR_ARG;
     return guarded(m0, [&]() {
         // The inputs go up and are rounded once, on the first network's stream; the networks
-        // run side by side on their own streams after it, and the statistics wait for them all.
-        leo2d::DevPool::Use none(nullptr);   // buffers several streams use are not pooled
+        // run side by side on their own streams after it, and the statistics wait for them all:
+        // when the first network's stream has drained, and its buffers go back, all have.
         const int chunk = 4096;
         const int out = m0->out();
         hipStream_t s0 = m0->stream;
         DevBuf Ys, dmean, dspread;
         dalloc(Ys, sizeof(float) * (size_t)count * chunk * out, "ensemble outputs");
-        dalloc(dmean, sizeof(float) * (size_t)chunk * out, "ensemble mean");
+        if (mean) dalloc(dmean, sizeof(float) * (size_t)chunk * out, "ensemble mean");
         dalloc(dspread, sizeof(float) * (size_t)std::max<int64_t>(n, 1) * blocks, "ensemble spread");
         struct Event {
             hipEvent_t e = nullptr;
