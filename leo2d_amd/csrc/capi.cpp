@@ -6,7 +6,6 @@
 // the KPM recursion.  No exception crosses the ABI: every entry point catches
 // and converts to a LEO2D_ERR_* code with a message in leo2d_last_error().
 #include <algorithm>
-#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -14,7 +13,6 @@
 #include <fstream>
 #include <random>
 #include <string>
-#include <thread>
 #include <vector>
 
 
@@ -35,7 +33,6 @@ struct leo2d_geom {
 namespace {
 
 using leo2d::DevBuf;
-using leo2d::HostBuf;
 using leo2d::HipError;
 using leo2d::check;
 using leo2d::dalloc;
@@ -104,11 +101,9 @@ struct SellTiles {
     bool valid = false, failed = false, spatial = false;
     int ucap = 0, tmax = 0, ntiles = 0, ngroups = 0, tile_rows = 0, max_len = 0;
     int64_t entries = 0;
-    double build_ms = 0.0;
-    DevBuf row0, u0, ucols, g0, grow, glen, goff, eu, map, val, val32;
+    DevBuf row0, u0, ucols, g0, grow, glen, goff, eu, val, val32;
     bool val_valid = false, val32_valid = false;
-    std::vector<int32_t> job_tile0;   // first tile of each job when cut at job boundaries
-    DevBuf djob_tile0;
+    DevBuf djob_tile0;   // first tile of each job when cut at job boundaries
 };
 
 }  // namespace
@@ -153,9 +148,8 @@ struct leo2d_handle {
     bool pcsr_valid = false, pval32_valid = false;
     DevBuf prp, pcol_k, pval, pval32;
     // SELL-4-sigma row tiles of the recursion matrix for the LDS-staged step
-    // (sell.hip): pattern built on the host on first use, values gathered on the device
+    // (sell.hip), built on first use
     SellTiles sell;
-    HostBuf sell_stage;   // pinned staging of a pattern for its SELL tile build, kept for the next build
     leo2d_timing timing{};
     std::vector<hipEvent_t> events;
     // batched jobs: stacked block-diagonal CSR of every appended Hamiltonian
@@ -340,285 +334,112 @@ void set_csr_owned(leo2d_handle* h, int n, int64_t nnz, int cpx)
     h->has_dx = false;
 }
 
-// Tiles of the rows [lo, hi), with tile starts forced at lo and at the rows
-// marked in brk.  With `local`, every column lies in [lo, hi) (checked) and the
-// per-column scratch covers only those rows; otherwise it covers all n.  Offsets
-// (u0, g0, goff) are relative to this part's own arrays; rows, columns and CSR
-// positions are global.
-struct SellPart {
-    std::vector<int32_t> row0, ucols, g0, grow, glen;
-    std::vector<int64_t> u0, goff, map;
-    std::vector<uint16_t> eu;
-    int tile_rows = 0, max_len = 0;
-    bool ok = true;
-};
-
-void build_sell_part(SellPart& P, const int64_t* rp, const int32_t* col, const uint8_t* brk, int lo, int hi, int ucap,
-                     int tmax, bool local, int n)
-{
-    const int base = local ? lo : 0;
-    const int m = local ? hi - lo : n;
-    std::vector<int32_t> stamp(m, -1), loc(m, 0), added, halo, order;
-    int r = lo, tile = 0;
-    while (r < hi) {
-        const int start = r;
-        int size = 0;   // distinct columns of the tile so far (own rows included)
-        while (r < hi && r - start < tmax && !(r > start && brk[r])) {
-            if (rp[r + 1] - rp[r] > leo2d::kSellMaxLen) {
-                P.ok = false;
-                return;
-            }
-            added.clear();
-            auto take = [&](int c) {
-                if (stamp[c - base] != tile) {
-                    stamp[c - base] = tile;
-                    added.push_back(c);
-                }
-            };
-            take(r);
-            for (int64_t q = rp[r]; q < rp[r + 1]; ++q) {
-                if (local && (col[q] < lo || col[q] >= hi)) {
-                    P.ok = false;
-                    return;
-                }
-                take(col[q]);
-            }
-            if (size + (int)added.size() > ucap) {
-                for (int c : added) stamp[c - base] = -1;
-                break;
-            }
-            size += (int)added.size();
-            ++r;
-        }
-        if (r == start) {
-            P.ok = false;
-            return;
-        }
-        const int T = r - start;
-        P.tile_rows = std::max(P.tile_rows, T);
-        // union: own rows, then the other columns in increasing order
-        halo.clear();
-        for (int rr = start; rr < r; ++rr)
-            for (int64_t q = rp[rr]; q < rp[rr + 1]; ++q) {
-                const int c = col[q];
-                if ((c < start || c >= r) && stamp[c - base] == tile) {
-                    stamp[c - base] = -2 - tile;   // listed once
-                    halo.push_back(c);
-                }
-            }
-        std::sort(halo.begin(), halo.end());
-        P.row0.push_back(start);
-        P.u0.push_back((int64_t)P.ucols.size());
-        for (int rr = start; rr < r; ++rr) {
-            loc[rr - base] = rr - start;
-            P.ucols.push_back(rr);
-        }
-        for (size_t k = 0; k < halo.size(); ++k) {
-            loc[halo[k] - base] = T + (int)k;
-            P.ucols.push_back(halo[k]);
-        }
-        // SELL-4 groups, rows by decreasing length (sigma = the tile)
-        order.resize(T);
-        for (int k = 0; k < T; ++k) order[k] = start + k;
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int a, int b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
-        P.g0.push_back((int32_t)P.glen.size());
-        for (int k = 0; k < T; k += 4) {
-            int L = 0;
-            for (int j = 0; j < 4; ++j) {
-                const int row = k + j < T ? order[k + j] : -1;
-                P.grow.push_back(row);
-                if (row >= 0) L = std::max(L, (int)(rp[row + 1] - rp[row]));
-            }
-            L = (L + 3) / 4 * 4;
-            P.max_len = std::max(P.max_len, L);
-            P.glen.push_back(L);
-            P.goff.push_back((int64_t)P.eu.size());
-            for (int e = 0; e < L; ++e)
-                for (int j = 0; j < 4; ++j) {
-                    const int row = k + j < T ? order[k + j] : -1;
-                    if (row >= 0 && e < rp[row + 1] - rp[row]) {
-                        const int64_t q = rp[row] + e;
-                        P.eu.push_back((uint16_t)loc[col[q] - base]);
-                        P.map.push_back(q);
-                    } else {
-                        P.eu.push_back(0);
-                        P.map.push_back(-1);
-                    }
-                }
-        }
-        ++tile;
-    }
-}
-
-// SELL-4-sigma row tiles for the LDS-staged step (sell.hip).  Greedy tiles of
-// consecutive rows of the recursion matrix (at most kSellMaxRows) while the
-// tile's distinct columns -- its own rows first, then the other columns in
-// increasing order -- fit `ucap` LDS rows.  Within a tile the rows are sorted by
-// length (longest first, ties by row) and cut into groups of four; a group of
-// longest row L stores round_up(L, 4) entries per slot, entry e of slot s at
-// goff + 4 e + s, padded with (union index 0, value 0).  `map` gives each
-// stored entry's position in the CSR (-1 for padding) so the values can be
-// gathered on the device for every matrix with this pattern.  Returns false
-// when a row has more than kSellMaxLen entries or does not fit `ucap` alone.
+// SELL-4-sigma row tiles for the LDS-staged step (sell.hip), built on the device
+// (sell_build.hip).  Greedy tiles of consecutive rows of the recursion matrix (at
+// most tmax) while the tile's distinct columns -- its own rows first, then the other
+// columns in increasing order -- fit `ucap` LDS rows.  Within a tile the rows are
+// sorted by length (longest first, ties by row) and cut into groups of four; a group
+// of longest row L stores round_up(L, 4) entries per slot, entry e of slot s at
+// goff + 4 e + s, padded with (union index 0, value 0).  Returns false when a row
+// has more than kSellMaxLen entries or does not fit `ucap` alone.
 // With `breaks` (ascending first rows of stacked jobs, ending with n) no tile
-// crosses a job boundary, and job_tile0 lists each job's first tile.
-bool build_sell_tiles(SellTiles& S, HostBuf& stage, hipStream_t s, int n, int64_t nnz, const int64_t* drp,
-                      const int32_t* dcol, int ucap, int tmax, bool spatial, const std::vector<int64_t>* breaks)
+// crosses a job boundary, and djob_tile0 lists each job's first tile.
+bool build_sell_tiles(SellTiles& S, hipStream_t s, int n, const int64_t* drp, const int32_t* dcol, int ucap, int tmax,
+                      bool spatial, const std::vector<int64_t>* breaks)
 {
     if (S.valid && S.ucap == ucap && S.tmax == tmax && S.spatial == spatial) return true;
     if (S.failed && S.ucap == ucap && S.tmax == tmax && S.spatial == spatial) return false;
-    const auto t0 = std::chrono::steady_clock::now();
-    // the pattern comes over into pinned memory the handle keeps: batched jobs
-    // rebuild their tiles for every batch, and a pageable copy of a 271 M-entry
-    // pattern took 0.37 s
-    halloc(stage, sizeof(int64_t) * ((size_t)n + 1) + sizeof(int32_t) * (size_t)nnz, "sell pattern staging");
-    int64_t* const rp = static_cast<int64_t*>(stage.p);
-    int32_t* const col = reinterpret_cast<int32_t*>(rp + n + 1);
-    check(hipMemcpyAsync(rp, drp, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost, s), "sell");
-    if (nnz) check(hipMemcpyAsync(col, dcol, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, s), "sell");
-    check(hipStreamSynchronize(s), "sell");
-    std::vector<uint8_t> brk(n + 1, 0);
-    if (breaks)
-        for (int64_t b : *breaks)
-            if (b >= 0 && b <= n) brk[b] = 1;
     S.ucap = ucap;
     S.tmax = tmax;
     S.spatial = spatial;
-    auto fail = [&]() {
-        S.failed = true;
-        S.valid = false;
-        return false;
-    };
-    // Stacked jobs never share a tile, so contiguous runs of whole jobs are built
-    // on host threads side by side (each job's columns lie in its own rows) and
-    // joined in order: the same tiles as one pass over the rows.  A single matrix
-    // of kSellSplitRows rows or more is cut into 16 fixed row ranges (the same on
-    // every machine) whose first rows start tiles; a smaller one is one part
-    // (LEO2D_SELL_SPLIT_ROWS moves that bound).
-    const int64_t split_rows = std::max<int64_t>(16, env_int("LEO2D_SELL_SPLIT_ROWS", 1 << 20));
-    std::vector<int> cuts{0};
-    bool local = true;
-    if (breaks && breaks->size() > 2) {
-        const int want = (int)std::max<unsigned>(1, std::min<unsigned>(16, std::thread::hardware_concurrency()));
-        const int64_t per = (int64_t)n / want + 1;
-        for (int64_t b : *breaks)
-            if (b > cuts.back() && b < n && b - cuts.back() >= per) cuts.push_back((int)b);
-    } else if (!breaks && n >= split_rows) {
-        local = false;
-        for (int k = 1; k < 16; ++k) cuts.push_back((int)((int64_t)n * k / 16));
-    }
-    cuts.push_back(n);
-    const int nparts = (int)cuts.size() - 1;
-    std::vector<SellPart> parts(nparts);
-    auto run = [&](int p) {
-        build_sell_part(parts[p], rp, col, brk.data(), cuts[p], cuts[p + 1], ucap, tmax, local, n);
-    };
-    if (nparts == 1) {
-        run(0);
-    } else {
-        std::vector<std::thread> pool;
-        for (int p = 0; p < nparts; ++p) pool.emplace_back(run, p);
-        for (auto& t : pool) t.join();
-    }
-    if (!std::all_of(parts.begin(), parts.end(), [](const SellPart& P) { return P.ok; })) {
-        if (nparts == 1) return fail();
-        // a part whose rows reach outside it: build the whole matrix as one part
-        parts.assign(1, SellPart{});
-        build_sell_part(parts[0], rp, col, brk.data(), 0, n, ucap, tmax, true, n);
-        if (!parts[0].ok) return fail();
-    }
-    // Device arrays, filled part by part at each part's offsets; only the tile and
-    // group offsets (u0, g0, goff) are shifted on the host.  row0 is also kept on
-    // the host for the job starts.
-    const int np = (int)parts.size();
-    std::vector<size_t> ot(np + 1, 0), ou(np + 1, 0), og(np + 1, 0), oe(np + 1, 0);
-    int tile_rows = 0, max_len = 0;
-    for (int p = 0; p < np; ++p) {
-        const SellPart& P = parts[p];
-        ot[p + 1] = ot[p] + P.row0.size();
-        ou[p + 1] = ou[p] + P.ucols.size();
-        og[p + 1] = og[p] + P.glen.size();
-        oe[p + 1] = oe[p] + P.eu.size();
-        tile_rows = std::max(tile_rows, P.tile_rows);
-        max_len = std::max(max_len, P.max_len);
-    }
-    const size_t T = ot[np], U = ou[np], G = og[np], E = oe[np];
-    dalloc(S.row0, sizeof(int32_t) * (T + 1), "sell tiles");
-    dalloc(S.u0, sizeof(int64_t) * (T + 1), "sell tiles");
-    dalloc(S.g0, sizeof(int32_t) * (T + 1), "sell tiles");
-    dalloc(S.ucols, sizeof(int32_t) * U, "sell tiles");
-    dalloc(S.grow, sizeof(int32_t) * 4 * G, "sell groups");
-    dalloc(S.glen, sizeof(int32_t) * G, "sell groups");
-    dalloc(S.goff, sizeof(int64_t) * G, "sell groups");
-    dalloc(S.eu, sizeof(uint16_t) * E, "sell entries");
-    dalloc(S.map, sizeof(int64_t) * E, "sell entries");
-    auto put = [&](DevBuf& b, size_t off, const auto& v) {
-        using T_ = typename std::decay_t<decltype(v)>::value_type;
-        if (!v.empty())
-            check(hipMemcpyAsync(static_cast<char*>(b.p) + off * sizeof(T_), v.data(), sizeof(T_) * v.size(),
-                                 hipMemcpyHostToDevice, s),
-                  "sell tiles");
-    };
-    std::vector<int32_t> row0;
-    row0.reserve(T + 1);
-    for (int p = 0; p < np; ++p) {
-        SellPart& P = parts[p];
-        for (auto& x : P.u0) x += (int64_t)ou[p];
-        for (auto& x : P.g0) x += (int32_t)og[p];
-        for (auto& x : P.goff) x += (int64_t)oe[p];
-        row0.insert(row0.end(), P.row0.begin(), P.row0.end());
-        put(S.u0, ot[p], P.u0);
-        put(S.g0, ot[p], P.g0);
-        put(S.ucols, ou[p], P.ucols);
-        put(S.grow, 4 * og[p], P.grow);
-        put(S.glen, og[p], P.glen);
-        put(S.goff, og[p], P.goff);
-        put(S.eu, oe[p], P.eu);
-        put(S.map, oe[p], P.map);
-    }
-    row0.push_back(n);
-    put(S.row0, 0, row0);
-    const std::vector<int64_t> u_end{(int64_t)U};
-    const std::vector<int32_t> g_end{(int32_t)G};
-    put(S.u0, T, u_end);
-    put(S.g0, T, g_end);
-    // the parts' host arrays are read by the copies above
-    check(hipStreamSynchronize(s), "sell");
-    parts.clear();
-    const int tile = (int)T;
-    S.job_tile0.clear();
-    if (breaks) {
-        for (int64_t b : *breaks)
-            S.job_tile0.push_back((int32_t)(std::lower_bound(row0.begin(), row0.end() - 1, (int32_t)b) - row0.begin()));
-        to_device(S.djob_tile0, S.job_tile0.data(), sizeof(int32_t) * S.job_tile0.size(), s, "sell job tiles");
-    }
-    check(hipStreamSynchronize(s), "sell");
-    S.ntiles = tile;
-    S.tile_rows = tile_rows;
-    S.max_len = max_len;
-    S.ngroups = (int)G;
-    S.entries = (int64_t)E;
+    S.valid = false;
     S.val_valid = S.val32_valid = false;
+    // Segments of up to kSegTiles full tiles, fewer while that leaves less than 96: each is walked
+    // by one wavefront, row after row, and ends in a tile cut short, which the steps pay for
+    // (segments of 3 tiles made the step on 190 k rows 5 % slower, of 13 tiles 2.5 %).
+    const int64_t seg = (int64_t)tmax * std::max(1, std::min<int>(leo2d::kSegTiles, n / (tmax * 96)));
+    std::vector<int32_t> seg_row0, job_seg;
+    const std::vector<int64_t> whole{0, n};
+    const std::vector<int64_t>& jobs = breaks ? *breaks : whole;
+    for (size_t j = 0; j + 1 < jobs.size(); ++j) {
+        job_seg.push_back((int32_t)seg_row0.size());
+        for (int64_t r = jobs[j]; r < jobs[j + 1]; r += seg) seg_row0.push_back((int32_t)r);
+    }
+    const int nseg = (int)seg_row0.size();
+    job_seg.push_back(nseg);
+    seg_row0.push_back(n);
+    DevBuf dseg, djob, cut_row, cut_u, counts, offs, state, ucount, gcount, ecount, g0_64, e0_64;
+    to_device(dseg, seg_row0.data(), sizeof(int32_t) * seg_row0.size(), s, "sell segments");
+    to_device(djob, job_seg.data(), sizeof(int32_t) * job_seg.size(), s, "sell segments");
+    dalloc(cut_row, sizeof(int32_t) * (size_t)n, "sell tiles");
+    dalloc(cut_u, sizeof(int32_t) * (size_t)n, "sell tiles");
+    dalloc(counts, sizeof(int64_t) * (size_t)nseg, "sell tiles");
+    dalloc(offs, sizeof(int64_t) * ((size_t)nseg + 1), "sell tiles");
+    dalloc(state, sizeof(int32_t) * 4, "sell tiles");   // most rows, most steps, -, a row that does not fit
+    check(hipMemsetAsync(state.p, 0, sizeof(int32_t) * 4, s), "sell tiles");
+    check(hipMemsetAsync(counts.p, 0, sizeof(int64_t) * (size_t)nseg, s), "sell tiles");
+    int32_t* const dstate = (int32_t*)state.p;
+    check(leo2d::launch_sell_cut(drp, dcol, (const int32_t*)dseg.p, nseg, ucap, tmax, (int32_t*)cut_row.p,
+                                 (int32_t*)cut_u.p, (int64_t*)counts.p, dstate + 3, s),
+          "sell tiles");
+    check(leo2d::scan_exclusive_i64((const int64_t*)counts.p, (int64_t*)offs.p, nseg, s), "sell scan");
+    int64_t ntiles = 0;
+    int32_t hstate[4] = {0, 0, 0, 0};
+    check(hipMemcpyAsync(&ntiles, (const int64_t*)offs.p + nseg, sizeof(int64_t), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipMemcpyAsync(hstate, state.p, sizeof(hstate), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipStreamSynchronize(s), "sell tiles");
+    S.failed = hstate[3] != 0 || ntiles <= 0;
+    if (S.failed) return false;
+    const int T = (int)ntiles;
+    dalloc(S.row0, sizeof(int32_t) * ((size_t)T + 1), "sell tiles");
+    dalloc(S.u0, sizeof(int64_t) * ((size_t)T + 1), "sell tiles");
+    dalloc(S.g0, sizeof(int32_t) * ((size_t)T + 1), "sell tiles");
+    dalloc(S.djob_tile0, sizeof(int32_t) * job_seg.size(), "sell job tiles");
+    for (DevBuf* b : {&ucount, &gcount, &ecount}) dalloc(*b, sizeof(int64_t) * (size_t)T, "sell tiles");
+    for (DevBuf* b : {&g0_64, &e0_64}) dalloc(*b, sizeof(int64_t) * ((size_t)T + 1), "sell tiles");
+    check(leo2d::launch_sell_list(drp, (const int32_t*)dseg.p, (const int64_t*)offs.p, nseg, T, (const int32_t*)cut_row.p,
+                                  (const int32_t*)cut_u.p, (int32_t*)S.row0.p, (int64_t*)ucount.p, (int64_t*)gcount.p,
+                                  (int64_t*)ecount.p, dstate, (const int32_t*)djob.p, (int)job_seg.size(),
+                                  (int32_t*)S.djob_tile0.p, s),
+          "sell tiles");
+    check(leo2d::scan_exclusive_i64((const int64_t*)ucount.p, (int64_t*)S.u0.p, T, s), "sell scan");
+    check(leo2d::scan_exclusive_i64((const int64_t*)gcount.p, (int64_t*)g0_64.p, T, s), "sell scan");
+    check(leo2d::scan_exclusive_i64((const int64_t*)ecount.p, (int64_t*)e0_64.p, T, s), "sell scan");
+    int64_t U = 0, G = 0, E = 0;
+    check(hipMemcpyAsync(&U, (const int64_t*)S.u0.p + T, sizeof(int64_t), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipMemcpyAsync(&G, (const int64_t*)g0_64.p + T, sizeof(int64_t), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipMemcpyAsync(&E, (const int64_t*)e0_64.p + T, sizeof(int64_t), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipMemcpyAsync(hstate, state.p, sizeof(hstate), hipMemcpyDeviceToHost, s), "sell tiles");
+    check(hipStreamSynchronize(s), "sell tiles");
+    dalloc(S.ucols, sizeof(int32_t) * (size_t)U, "sell tiles");
+    dalloc(S.grow, sizeof(int32_t) * 4 * (size_t)G, "sell groups");
+    dalloc(S.glen, sizeof(int32_t) * (size_t)G, "sell groups");
+    dalloc(S.goff, sizeof(int64_t) * (size_t)G, "sell groups");
+    dalloc(S.eu, sizeof(uint16_t) * (size_t)E, "sell entries");
+    check(leo2d::launch_sell_write(drp, dcol, T, (const int32_t*)S.row0.p, (const int64_t*)S.u0.p, (const int64_t*)g0_64.p,
+                                   (const int64_t*)e0_64.p, (int32_t*)S.g0.p, (int32_t*)S.ucols.p, (int32_t*)S.grow.p,
+                                   (int32_t*)S.glen.p, (int64_t*)S.goff.p, (uint16_t*)S.eu.p, s),
+          "sell tiles");
+    check(hipStreamSynchronize(s), "sell tiles");
+    S.ntiles = T;
+    S.tile_rows = hstate[0];
+    S.max_len = hstate[1];
+    S.ngroups = (int)G;
+    S.entries = E;
     S.valid = true;
-    S.failed = false;
-    S.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return true;
 }
 
-bool build_sell(leo2d_handle* h, const int64_t* drp, const int32_t* dcol, int ucap, int tmax, bool spatial)
-{
-    return build_sell_tiles(h->sell, h->sell_stage, h->stream, h->n, h->nnz, drp, dcol, ucap, tmax, spatial, nullptr);
-}
-
-// the SELL values of a matrix (FP64, or FP32 for the mixed recursion)
-const void* sell_values(SellTiles& S, hipStream_t stream, const void* csr_val, int elem_bytes, bool fp32)
+// the SELL values of a matrix with row pointers drp (FP64, or FP32 for the mixed recursion)
+const void* sell_values(SellTiles& S, hipStream_t stream, const int64_t* drp, const void* csr_val, int elem_bytes,
+                        bool fp32)
 {
     DevBuf& buf = fp32 ? S.val32 : S.val;
     bool& ok = fp32 ? S.val32_valid : S.val_valid;
     if (!ok) {
         dalloc(buf, (size_t)elem_bytes * (size_t)S.entries, "sell values");
-        check(leo2d::launch_sell_fill((const int64_t*)S.map.p, csr_val, buf.p, elem_bytes, S.entries, stream),
+        check(leo2d::launch_sell_fill(drp, (const int32_t*)S.grow.p, (const int32_t*)S.glen.p, (const int64_t*)S.goff.p,
+                                      S.ngroups, csr_val, buf.p, elem_bytes, stream),
               "sell values");
         ok = true;
     }
@@ -1561,13 +1382,13 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                 const int tlim = copy_wave ? leo2d::kSellCwRows : leo2d::kSellMaxRows;
                 const int tmax = std::max(4, std::min(tlim, env_int("LEO2D_SELL_TMAX", tlim)));
                 if (!spatial || !leo2d::sell_supported(mat_type, vec_type, B, copy_wave) ||
-                    !build_sell(h, drp, dcol, ucap, tmax, spatial)) {
+                    !build_sell_tiles(h->sell, s, n, drp, dcol, ucap, tmax, spatial, nullptr)) {
                     sa.variant = B == 16 || B == 32 ? 14 : (mixed ? 15 : 1);
                 } else {
                     auto& S = h->sell;
                     const int hb = mat_type == leo2d::MAT_CPX_F64 ? 16
                                    : (mat_type == leo2d::MAT_REAL_F32 ? 4 : 8);
-                    ss.ev = sell_values(S, h->stream, dval, hb, mixed);
+                    ss.ev = sell_values(S, s, drp, dval, hb, mixed);
                     int dev_id = 0, cus = 256;
                     if (hipGetDevice(&dev_id) == hipSuccess)
                         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev_id);
@@ -2132,14 +1953,13 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
         // SELL tiles of the stack (complex vectors, R = 16 or 32; FP32 only at 32): tiles of at most
         // 56 rows for the kernel with a copy wavefront, else 64 rows whose union fits the LDS the
         // eight-wavefront kernel leaves beside its T_{j-1} copies and partials
-        // (built on the host once per stack, so only when mode 3 is asked for or may be tuned in)
+        // (built once per stack, so only when mode 3 is asked for or may be tuned in)
         const bool sell_cw = env_int("LEO2D_SELL_CW", 1) != 0;
         const bool want_sell = p->mode == LEO2D_BATCH_SELL || p->tune;
         // the copy wavefront addresses a vector chunk with 32-bit byte offsets
         const bool sell_fits = !sell_cw || (uint64_t)B.rows * (uint64_t)R * leo2d::vec_bytes(vec_type) < (uint64_t(1) << 32);
         const bool sell_ok = want_sell && leo2d::sell_supported(mat_type, vec_type, R, sell_cw) && R <= 32 && sell_fits &&
-                             build_sell_tiles(B.sell, h->sell_stage, s, (int)B.rows, B.nnz, (const int64_t*)B.rp.p,
-                                              (const int32_t*)B.col.p,
+                             build_sell_tiles(B.sell, s, (int)B.rows, (const int64_t*)B.rp.p, (const int32_t*)B.col.p,
                                               sell_cw ? leo2d::kSellUcap : leo2d::kSellUcapTiled,
                                               sell_cw ? leo2d::kSellCwRows : leo2d::kSellMaxRows, false, &B.job_row0);
         if (!p->tune && p->mode == LEO2D_BATCH_SELL && !sell_ok)
@@ -2174,7 +1994,7 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
         if (sell_ok) {
             auto& S = B.sell;
             const int hb = mat_type == leo2d::MAT_CPX_F64 ? 16 : (mat_type == leo2d::MAT_REAL_F32 ? 4 : 8);
-            ss.ev = sell_values(S, s, dval, hb, mixed);
+            ss.ev = sell_values(S, s, (const int64_t*)B.rp.p, dval, hb, mixed);
             ss.n = (int)B.rows;
             ss.R = R;
             ss.part = (double*)B.part.p;

@@ -92,9 +92,24 @@ struct SellStepArgs {
 // copy_wave: 16 complex FP32 vectors (128-byte row chunks) need the copy-wavefront kernel
 bool sell_supported(int mat_type, int vec_type, int R, bool copy_wave);
 hipError_t launch_kpm_step_sell(int mat_type, int vec_type, const SellStepArgs& a, hipStream_t s);
-// dst[i] = src[map[i]] (zero where map[i] < 0), elements of elem_bytes (4, 8 or 16)
-hipError_t launch_sell_fill(const int64_t* map, const void* src, void* dst, int elem_bytes, int64_t count,
+// Their layout, built on the device (sell_build.hip).  Segments of rows are cut into tiles on
+// their own (a tile never crosses a segment); then the tiles are listed and measured, and after
+// the scans of their union rows, groups and entries written.
+constexpr int kSegTiles = 48;   // full tiles in a segment, at most
+hipError_t launch_sell_cut(const int64_t* rp, const int32_t* col, const int32_t* seg_row0, int nseg, int ucap, int tmax,
+                           int32_t* cut_row, int32_t* cut_u, int64_t* seg_tiles, int32_t* flag, hipStream_t s);
+// most[0], most[1] (zero before): most rows of a tile, most steps of a group; job_tile0[j] = first
+// tile of segment job_seg[j], j < njobs1
+hipError_t launch_sell_list(const int64_t* rp, const int32_t* seg_row0, const int64_t* seg_off, int nseg, int ntiles,
+                            const int32_t* cut_row, const int32_t* cut_u, int32_t* row0, int64_t* ucount, int64_t* gcount,
+                            int64_t* ecount, int32_t* most, const int32_t* job_seg, int njobs1, int32_t* job_tile0,
                             hipStream_t s);
+hipError_t launch_sell_write(const int64_t* rp, const int32_t* col, int ntiles, const int32_t* row0, const int64_t* u0,
+                             const int64_t* g0, const int64_t* e0, int32_t* g0_out, int32_t* ucols, int32_t* grow,
+                             int32_t* glen, int64_t* goff, uint16_t* eu, hipStream_t s);
+// the stored values of every group from the CSR values (elements of 4, 8 or 16 bytes)
+hipError_t launch_sell_fill(const int64_t* rp, const int32_t* grow, const int32_t* glen, const int64_t* goff, int ngroups,
+                            const void* src, void* dst, int elem_bytes, hipStream_t s);
 
 // Deterministic reduction of the partials of `steps` consecutive steps from j0 on
 // into moments (step 0 in a launch of its own: the others read its moments).

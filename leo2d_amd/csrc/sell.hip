@@ -15,7 +15,7 @@
 // row chunks (the tile's "union", about 4 per output row) once into LDS with
 // direct global->LDS loads, and every entry then reads its operand from LDS.
 //
-// Layout of the matrix (built on the host once per sparsity pattern):
+// Layout of the matrix (sell_build.hip, once per sparsity pattern):
 //  * tiles: consecutive rows [tile_row0[t], tile_row0[t+1]) of the spatially
 //    ordered matrix; the tile's union is ucols[tile_u0[t] ...], own rows
 //    first (union index u = row - tile_row0[t]) so T_j of an own row is in LDS;
@@ -1073,20 +1073,6 @@ hipError_t launch_sell_f32x16(const SellStepArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-// dst[i] = src[map[i]] (0 where map[i] < 0): the SELL values from the CSR values
-template <typename E>
-__global__ void sell_fill_kernel(const int64_t* __restrict__ map, const E* __restrict__ src, E* __restrict__ dst,
-                                 int64_t count)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t m = map[i];
-        E e;
-        if (m >= 0) e = src[m];
-        else zero(e);
-        dst[i] = e;
-    }
-}
-
 }  // namespace
 
 bool sell_supported(int mat_type, int vec_type, int R, bool copy_wave)
@@ -1113,28 +1099,6 @@ hipError_t launch_kpm_step_sell(int mat_type, int vec_type, const SellStepArgs& 
     if (mat_type == MAT_REAL_F32)
         return a.R == 16 ? launch_sell_f32x16<float>(a, s) : launch_sell_shape<float, float2, 2>(a, s);
     return hipErrorInvalidValue;
-}
-
-hipError_t launch_sell_fill(const int64_t* map, const void* src, void* dst, int elem_bytes, int64_t count, hipStream_t s)
-{
-    if (count <= 0) return hipSuccess;
-    const int blocks = (int)std::min<int64_t>(4096, (count + 255) / 256);
-    switch (elem_bytes) {
-    case 4:
-        hipLaunchKernelGGL(sell_fill_kernel<float>, dim3(blocks), dim3(256), 0, s, map, (const float*)src, (float*)dst,
-                           count);
-        break;
-    case 8:
-        hipLaunchKernelGGL(sell_fill_kernel<double>, dim3(blocks), dim3(256), 0, s, map, (const double*)src,
-                           (double*)dst, count);
-        break;
-    case 16:
-        hipLaunchKernelGGL(sell_fill_kernel<double2>, dim3(blocks), dim3(256), 0, s, map, (const double2*)src,
-                           (double2*)dst, count);
-        break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
 }
 
 }  // namespace leo2d
