@@ -50,17 +50,32 @@ struct NanError : std::runtime_error {
 // the SELL-4-sigma step with LDS-staged row tiles (sell.hip)
 constexpr int kVariantSell = 20;
 
-// Below this many rows the SELL tiles (at most 56 rows each) are fewer than the
-// GPU's CUs, and a matrix assembled for one short run pays the host-side tile
-// build for little: the vector-chunk kernel runs those.
-constexpr int kSellMinRows = 16384;
+// Fewest rows that run the SELL tiles (sell_tile_rows).  Below, the step is a chain of latencies that
+// the vector-chunk kernel crosses faster; from here on the tiles' staging pays, and so does their
+// build (0.2 ms) within some 200 steps.  Steps in us on commensurate cells, complex FP64, tiles
+// against vector chunks at R = 16 / 32 / 64: 508 rows 7.3 / 6.4 / 9.0 against 6.2 / 6.3 / 6.7,
+// 2,032 rows 5.7 / 7.5 / 10.3 against 6.4 / 6.7 / 10.3, 4,572 rows 6.3 / 8.4 / 11.2 against
+// 8.1 / 11.0 / 19.4, 8,128 rows 7.4 / 9.2 / 13.0 against 8.9 / 15.0 / 27.6.
+constexpr int kSellMinRows = 4096;
+constexpr int kSellMinRows64 = 2048;   // at R = 64
+
+// Rows of a SELL tile (at most `most`): as many as give each workgroup (one per CU) the same number
+// of tiles, with 1/64 to spare for tiles the LDS budget cuts short, in groups of four rows.  Tiles of
+// 56 rows left part of the GPU idle: step on 18,288 rows at R = 64 26.5 us, with 36 or 40 rows
+// (two tiles per CU) 22.8 or 23.4; 8,128 rows at R = 16 7.9 us, with 36 rows 7.4.
+int sell_tile_rows(int n, int most, int cus)
+{
+    const int64_t turns = std::max<int64_t>(1, ((int64_t)n + (int64_t)most * cus - 1) / ((int64_t)most * cus));
+    const int64_t rows = ((int64_t)n + n / 64 + turns * cus - 1) / (turns * cus);
+    return (int)std::max<int64_t>(16, std::min<int64_t>(most, (rows + 3) / 4 * 4));
+}
 
 // step kernel for a block of B vectors on n rows (LEO2D_KPM_VARIANT = 0, 1, 2, 14,
 // 15 or 20 overrides the default).  FP64 blocks of at most 8 vectors run a group of
 // lanes per row (2) in either order.  In the spatial order: B = 16, 32 or 64 run
 // the SELL-4-sigma step with LDS-staged row tiles (20) where its layout applies
-// (complex vectors) and n >= kSellMinRows, else B = 16 or 32 vector chunks split
-// over the XCDs (14).  In the natural order (or where neither applies): B >= 64
+// and n >= kSellMinRows (kSellMinRows64), else vector chunks split over the XCDs
+// (14; at B = 64 only below that).  In the natural order (or where neither applies): B >= 64
 // the wavefront-per-row kernel (1), or for the FP32 recursion at B = 64 two rows
 // per wavefront with 16-byte gathers (15); other B lane per vector (0).
 int kpm_variant(bool mixed, bool spatial, int B, int n)
@@ -71,6 +86,7 @@ int kpm_variant(bool mixed, bool spatial, int B, int n)
     }
     if (!mixed && B <= 8) return 2;
     if (spatial && (B == 16 || B == 32)) return n >= kSellMinRows ? kVariantSell : 14;
+    if (spatial && B == 64 && n < kSellMinRows64) return 14;
     if (spatial && B >= 64) return kVariantSell;
     return mixed && spatial ? 15 : 1;
 }
@@ -1380,7 +1396,10 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                 // eight wavefronts that each issue their share of the copies
                 const bool copy_wave = env_int("LEO2D_SELL_CW", 1) != 0;
                 const int tlim = copy_wave ? leo2d::kSellCwRows : leo2d::kSellMaxRows;
-                const int tmax = std::max(4, std::min(tlim, env_int("LEO2D_SELL_TMAX", tlim)));
+                int dev_id = 0, cus = 256;
+                if (hipGetDevice(&dev_id) == hipSuccess)
+                    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev_id);
+                const int tmax = std::max(4, std::min(tlim, env_int("LEO2D_SELL_TMAX", sell_tile_rows(n, tlim, cus))));
                 if (!spatial || !leo2d::sell_supported(mat_type, vec_type, B, copy_wave) ||
                     !build_sell_tiles(h->sell, s, n, drp, dcol, ucap, tmax, spatial, nullptr)) {
                     sa.variant = B == 16 || B == 32 ? 14 : (mixed ? 15 : 1);
@@ -1389,9 +1408,6 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
                     const int hb = mat_type == leo2d::MAT_CPX_F64 ? 16
                                    : (mat_type == leo2d::MAT_REAL_F32 ? 4 : 8);
                     ss.ev = sell_values(S, s, drp, dval, hb, mixed);
-                    int dev_id = 0, cus = 256;
-                    if (hipGetDevice(&dev_id) == hipSuccess)
-                        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev_id);
                     ss.grid = std::max(8, std::min(G, cus) / 8 * 8);
                     sa.grid = ss.grid;   // the reduce reads this many partials
                     ss.n = n;

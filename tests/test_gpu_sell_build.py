@@ -1,8 +1,9 @@
 """Row tiles of the LDS-staged step where their layout on the device can go
 wrong: matrices smaller than a tile, one row more than whole tiles, segments of
-one tile and of several, tiles cut by the staged-row budget, and rows too long
-for the layout, which the CSR step runs.  FP64 moments within 1e-12 mu_0 of the
-oracle; the same tiles serve the FP32 recursion (2e-5 mu_0)."""
+one tile and of several, tiles cut by the staged-row budget, rows too long for
+the layout, which the CSR step runs, and the least rows it takes.  FP64 moments
+within 1e-12 mu_0 of the oracle; the same tiles serve the FP32 recursion (2e-5
+mu_0)."""
 import numpy as np
 import pytest
 
@@ -60,3 +61,35 @@ def test_long_rows_run_the_csr_step(oracle_mod, monkeypatch, pattern):
         mu = dev.kpm(M, random_phase=(R, 9), scheme=L.SCHEME_DOUBLING)
         assert dev.timing().kernel == (21 if fits else 14)
         assert np.max(np.abs(mu - omu)) <= 1e-12 * geom.n
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 3])
+@pytest.mark.parametrize("R", [16, 32, 64])
+@pytest.mark.parametrize("bloch", [0, 1])
+def test_default_step_by_rows(oracle_mod, monkeypatch, tiles, R, bloch):
+    """508, 2,032 and 4,572 rows: on either side of the least rows of the tiled
+    step, each default against the oracle, and the FP32 recursion against the
+    wavefront-per-row (or lane-per-vector) step, which sums rows alike."""
+    monkeypatch.delenv("LEO2D_KPM_VARIANT", raising=False)
+    dev = L.Device(0)
+    geom = L.Geometry(L.Deck(W.tblg_cell_deck(7, 6, tiles)))
+    dev.set_geometry(geom)
+    dev.pairs_build()
+    job = geom.jobs()[0]
+    job.energy_rescale = 10.5   # the smallest cell's spectrum is the widest
+    job.complex_matrix = bloch
+    if bloch:
+        job.k[0], job.k[1] = 0.011, -0.004
+    dev.assemble(job, L.PATTERN_PRUNED)
+    print("case", geom.n, R, bloch, flush=True)
+    rp, ci, v = dev.csr_copy()
+    M = 24
+    omu = oracle_mod.kpm(rp, ci, v, M, vecs=oracle_mod.random_phase(geom.n, R, 9), doubling_all=True, nthreads=8)
+    tiled = geom.n >= (2048 if R == 64 else 4096)
+    mu = dev.kpm(M, random_phase=(R, 9), scheme=L.SCHEME_DOUBLING)
+    assert dev.timing().kernel == (21 if tiled else 14)
+    assert np.max(np.abs(mu - omu)) <= 1e-12 * geom.n
+    mu32 = dev.kpm(M, random_phase=(R, 9), scheme=L.SCHEME_DOUBLING, precision=L.PREC_MIXED)
+    monkeypatch.setenv("LEO2D_KPM_VARIANT", "1" if R == 64 else "0")
+    ref32 = dev.kpm(M, random_phase=(R, 9), scheme=L.SCHEME_DOUBLING, precision=L.PREC_MIXED)
+    assert np.max(np.abs(mu32 - ref32)) <= 1e-12 * geom.n
