@@ -4,7 +4,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <cstdint>
 #include <map>
+#include <mutex>
+#include <set>
 #include <stdexcept>
 #include <string>
 
@@ -14,44 +18,74 @@ namespace leo2d {
 
 // Device buffers a handle has given back, kept for its next allocations.  A call
 // allocates and frees a dozen small buffers, each some 10-30 us with the device-wide
-// wait of a free; on a 230-orbital deck that was half of the time.  Everything a
-// handle queues runs on its one stream, so a buffer taken again is written only by
-// work queued after its last use.  Bounded: buffers of at most kPoolMost bytes, at
-// most kPoolKeep in all; the rest are freed at once, and all of them when an
-// allocation fails and with the handle.  Not shared between handles (one thread each).
+// wait of a free; on a 230-orbital deck that was half of the time.  Buffers of GBs cost
+// more: a conductivity call that allocated and freed 3 GB of vector sets took 21 ms in
+// one process and 50 to 90 ms in the next, and 20 ms in each with the sets kept.
+// Everything a handle queues runs on its one stream, so a buffer taken again is
+// written only by work queued after its last use.
+// Bounded: buffers of at most kPoolMost bytes, at most kPoolKeep in all handles of the
+// process (a handle's longest unused go first); all of every handle are freed when an
+// allocation fails, a handle's own with it.  A pool serves its handle alone; the lock
+// is for the handle whose allocation failed.
 class DevPool {
 public:
-    static constexpr size_t kPoolMost = size_t(64) << 20;
-    static constexpr size_t kPoolKeep = size_t(256) << 20;
-    DevPool() = default;
+    static constexpr size_t kPoolMost = size_t(2) << 30;
+    static constexpr size_t kPoolKeep = size_t(4) << 30;
+    DevPool()
+    {
+        std::lock_guard<std::mutex> g(all().lock);
+        all().pools.insert(this);
+    }
     DevPool(const DevPool&) = delete;
     DevPool& operator=(const DevPool&) = delete;
-    ~DevPool() { clear(); }
+    ~DevPool()
+    {
+        {
+            std::lock_guard<std::mutex> g(all().lock);
+            all().pools.erase(this);
+        }
+        clear();
+    }
     // a kept buffer of at least `bytes` (and less than twice that), or nullptr; cap: its size
     void* take(size_t bytes, size_t& cap)
     {
+        std::lock_guard<std::mutex> g(lock_);
         auto it = free_.lower_bound(bytes);
         if (it == free_.end() || it->first / 2 > bytes) return nullptr;
-        void* p = it->second;
         cap = it->first;
-        kept_ -= cap;
-        free_.erase(it);
-        return p;
+        return drop(it);
     }
     void give(void* p, size_t cap)
     {
-        if (cap > kPoolMost || kept_ + cap > kPoolKeep) {
-            (void)hipFree(p);
-            return;
+        std::lock_guard<std::mutex> g(lock_);
+        if (cap <= kPoolMost) {
+            // reserve first: two handles must not both take the last room
+            size_t was = all().kept.fetch_add(cap);
+            while (was + cap > kPoolKeep && !free_.empty()) {
+                auto old = free_.begin();
+                for (auto it = free_.begin(); it != free_.end(); ++it)
+                    if (it->second.given < old->second.given) old = it;
+                was -= old->first;
+                (void)hipFree(drop(old));
+            }
+            if (was + cap <= kPoolKeep) {
+                free_.emplace(cap, Kept{p, ++given_});
+                return;
+            }
+            all().kept -= cap;
         }
-        kept_ += cap;
-        free_.emplace(cap, p);
+        (void)hipFree(p);
     }
     void clear()
     {
-        for (auto& f : free_) (void)hipFree(f.second);
-        free_.clear();
-        kept_ = 0;
+        std::lock_guard<std::mutex> g(lock_);
+        while (!free_.empty()) (void)hipFree(drop(free_.begin()));
+    }
+    // every handle's kept buffers (a free waits for the work that may still use them)
+    static void clear_all()
+    {
+        std::lock_guard<std::mutex> g(all().lock);
+        for (DevPool* p : all().pools) p->clear();
     }
     // the pool of the handle whose entry point this thread is in
     static DevPool*& current()
@@ -66,8 +100,31 @@ public:
     };
 
 private:
-    std::multimap<size_t, void*> free_;   // by size
-    size_t kept_ = 0;
+    struct Kept {
+        void* p;
+        uint64_t given;   // order of return
+    };
+    using Free = std::multimap<size_t, Kept>;   // by size
+    struct All {
+        std::mutex lock;
+        std::set<DevPool*> pools;
+        std::atomic<size_t> kept{0};
+    };
+    static All& all()
+    {
+        static All* const a = new All;   // outlives every handle
+        return *a;
+    }
+    void* drop(Free::iterator it)
+    {
+        void* p = it->second.p;
+        all().kept -= it->first;
+        free_.erase(it);
+        return p;
+    }
+    std::mutex lock_;
+    Free free_;
+    uint64_t given_ = 0;
 };
 
 // owning device allocation (given back on release() or destruction; movable, not copyable)
@@ -144,10 +201,10 @@ inline void dalloc(DevBuf& b, size_t bytes, const char* what)
         }
     }
     hipError_t e = hipMalloc(&b.p, cap);
-    if (e != hipSuccess && pool) {
-        // what the pool keeps may be what is missing
+    if (e != hipSuccess) {
+        // what the pools keep may be what is missing
         (void)hipGetLastError();
-        pool->clear();
+        DevPool::clear_all();
         e = hipMalloc(&b.p, cap);
     }
     if (e != hipSuccess) {

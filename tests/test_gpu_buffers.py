@@ -73,3 +73,21 @@ def test_ensemble_members_destroyed_in_any_order():
     nets[0].close()
     assert np.array_equal(nets[2].forward(x), one[2])
     nets[2].close()
+
+
+def test_large_buffers_of_many_handles():
+    """Six handles with vector sets of 0.8 GB each pass the 4 GiB the process keeps: the
+    later ones' sets are freed, or push out what their own handle kept."""
+    geom = L.Geometry(L.Deck(W.tblg_flake_deck(1.05, 100.0, M=64)))
+    devs, ref = [], None
+    for _ in range(6):
+        dev = L.Device(0)
+        devs.append(dev)
+        dev.set_geometry(geom)
+        dev.assemble_velocity(geom.jobs()[0], L.PATTERN_PRUNED)
+        for M in (512, 384, 512):
+            got = dev.cond_moments(M, [0, 100, 1000, 10000])
+        ref = got if ref is None else ref
+        assert np.array_equal(got, ref)
+    for dev in devs:
+        dev.close()
