@@ -2261,11 +2261,16 @@ int leo2d_cond_moments(leo2d_handle* h, const leo2d_cond_params* p, double* C)
         const int64_t* drp = (const int64_t*)h->rp.p;
         const int32_t* dcol = (const int32_t*)h->col.p;
         const size_t nb = (size_t)n * B;
-        DevBuf Bset, Dset, X0, X1, dtg, Cdev;
+        const bool pair = B <= leo2d::kCondPair;
+        DevBuf Bset, Dset, X0, X1, P0, P1, dtg, Cdev;
         dalloc(Bset, sizeof(double) * nb * M, "beta set");
         dalloc(Dset, sizeof(double) * nb * M, "alpha set");
         dalloc(X0, sizeof(double) * nb, "vector block");
         dalloc(X1, sizeof(double) * nb, "vector block");
+        if (pair) {
+            dalloc(P0, sizeof(double) * 2 * nb, "vector block pair");
+            dalloc(P1, sizeof(double) * 2 * nb, "vector block pair");
+        }
         dalloc(dtg, sizeof(int32_t) * B, "targets");
         dalloc(Cdev, sizeof(double) * (size_t)B * M * M, "conductivity moments");
         // split the n-long GEMM reduction into S row chunks so that the M x M outputs of a pass
@@ -2290,9 +2295,6 @@ int leo2d_cond_moments(leo2d_handle* h, const leo2d_cond_params* p, double* C)
             for (int b = 0; b < B; ++b) tg[b] = p->targets[b0 + std::min(b, Bb - 1)];
             check(hipMemcpyAsync(dtg.p, tg.data(), sizeof(int32_t) * B, hipMemcpyHostToDevice, s), "targets");
             check(hipEventRecord(e0, s), "event");
-            // beta_m = T_m(H) e_t, written into the set by the step itself
-            check(leo2d::launch_init_targets(X0.p, leo2d::VEC_REAL_F64, n, B, (const int32_t*)dtg.p, s), "init");
-            scatter(X0.p, 0, Bset);
             auto dual = [&](const void* hv, const void* dv, const void* x, void* prev, void* out, double alpha, int beta,
                             int j, DevBuf* hset, DevBuf* dset) {
                 check(leo2d::launch_cond_dual_step(drp, dcol, (const double*)hv, (const double*)dv, (const double*)x,
@@ -2301,21 +2303,44 @@ int leo2d_cond_moments(leo2d_handle* h, const leo2d_cond_params* p, double* C)
                                                    s),
                       "conductivity step");
             };
-            dual(dH, nullptr, X0.p, nullptr, X1.p, 1.0, 0, 1, &Bset, nullptr);
-            void *cur = X1.p, *prv = X0.p;
-            for (int m = 2; m < M; ++m) {
-                dual(dH, nullptr, cur, prv, prv, 2.0, 1, m, &Bset, nullptr);
-                std::swap(cur, prv);
-            }
-            // alpha_0 = -dxH e_t; a_1 = H a_0, a_j = 2 H a_{j-1} - a_{j-2}.  One pass over a_{j-1}
-            // forms both a_j and D_{j-1} = dxH a_{j-1} (H and dxH share the pattern)
+            // beta_m = T_m(H) e_t and a_j = T_j(H) a_0, a_0 = -dxH e_t, written into the sets by the
+            // steps themselves: beta_j as it is, a_j as D_j = dxH a_j (H and dxH share the pattern)
             check(leo2d::launch_init_targets(X0.p, leo2d::VEC_REAL_F64, n, B, (const int32_t*)dtg.p, s), "init");
-            dual(dX, nullptr, X0.p, nullptr, X1.p, -1.0, 0, 0, nullptr, nullptr);
-            cur = X1.p;      // a_0
-            prv = X0.p;
-            for (int j = 1; j < M; ++j) {
-                dual(dH, dX, cur, j == 1 ? nullptr : prv, prv, j == 1 ? 1.0 : 2.0, j == 1 ? 0 : 1, j - 1, nullptr, &Dset);
-                std::swap(cur, prv);
+            void *cur, *prv;
+            if (pair) {
+                dual(dX, nullptr, X0.p, nullptr, X1.p, -1.0, 0, 0, nullptr, nullptr);
+                check(leo2d::launch_cond_pair_start((const int32_t*)dtg.p, (const double*)X1.p, n, B, M, (double*)P0.p,
+                                                    (double*)Bset.p, s),
+                      "conductivity start");
+                cur = P0.p;
+                prv = P1.p;
+                for (int j = 1; j < M; ++j) {
+                    check(leo2d::launch_cond_pair_step(drp, dcol, (const double*)dH, (const double*)dX, (const double*)cur,
+                                                       (const double*)prv, (double*)prv, j == 1 ? 1.0 : 2.0,
+                                                       j == 1 ? 0 : 1, n, B, j, M, (double*)Bset.p, (double*)Dset.p, s),
+                          "conductivity step");
+                    std::swap(cur, prv);
+                }
+                check(leo2d::launch_cond_pair_alpha((const double*)cur, n, B, (double*)X1.p, s), "conductivity step");
+                cur = X1.p;
+            } else {
+                scatter(X0.p, 0, Bset);
+                dual(dH, nullptr, X0.p, nullptr, X1.p, 1.0, 0, 1, &Bset, nullptr);
+                cur = X1.p;
+                prv = X0.p;
+                for (int m = 2; m < M; ++m) {
+                    dual(dH, nullptr, cur, prv, prv, 2.0, 1, m, &Bset, nullptr);
+                    std::swap(cur, prv);
+                }
+                check(leo2d::launch_init_targets(X0.p, leo2d::VEC_REAL_F64, n, B, (const int32_t*)dtg.p, s), "init");
+                dual(dX, nullptr, X0.p, nullptr, X1.p, -1.0, 0, 0, nullptr, nullptr);
+                cur = X1.p;      // a_0
+                prv = X0.p;
+                for (int j = 1; j < M; ++j) {
+                    dual(dH, dX, cur, j == 1 ? nullptr : prv, prv, j == 1 ? 1.0 : 2.0, j == 1 ? 0 : 1, j - 1, nullptr,
+                         &Dset);
+                    std::swap(cur, prv);
+                }
             }
             dual(nullptr, dX, cur, nullptr, nullptr, 1.0, 0, M - 1, nullptr, &Dset);
             check(hipEventRecord(e1, s), "event");

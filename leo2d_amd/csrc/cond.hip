@@ -200,14 +200,112 @@ __global__ __launch_bounds__(kCondThreads) void dual_step_lanes_kernel(const int
     }
 }
 
+// Both recursions of a block of B <= 4 targets at once: x = [n][2B] holds beta_{j-1}
+// and then a_{j-1} of every target, H x gives both next vectors, dxH x the D_{j-1} of
+// the alpha half; the new betas go straight into their set (vector j), D into its own
+// (vector j - 1).  Each matrix entry and each row's latencies serve both recursions:
+// microseconds per index on 95 k rows with 4 targets, H on the betas and both products
+// on the alphas one after the other 16.2 + 18.2, together 27.9.  Wider blocks keep
+// the recursions apart: from 8 vectors on the gathers bound the step either way.
+template <int B>
+__global__ __launch_bounds__(kCondThreads) void pair_step_kernel(const int64_t* __restrict__ rp,
+                                                                 const int32_t* __restrict__ col,
+                                                                 const double* __restrict__ hv,
+                                                                 const double* __restrict__ dv,
+                                                                 const double* __restrict__ x, const double* prev,
+                                                                 double* out, double alpha, int beta, int n, int j, int M,
+                                                                 double* __restrict__ hset, double* __restrict__ dset)
+{
+    constexpr int V = 2 * B;
+    constexpr int RPI = kCondThreads / 16;
+    const int lane = threadIdx.x & 63;
+    const int l = lane & 15;
+    const int v = l / (16 / V), b = l / (16 / B);
+    // consecutive rows per workgroup, the same at every index
+    const int G = gridDim.x;
+    const int blk = blockIdx.x;
+    const int lb = (blk & 7) * (G >> 3) + (blk >> 3);
+    const int iters = (n + RPI - 1) / RPI;
+    const int it0 = (int)((int64_t)iters * lb / G), it1 = (int)((int64_t)iters * (lb + 1) / G);
+    for (int it = it0; it < it1; ++it) {
+        const int row = it * RPI + (int)(threadIdx.x >> 4);
+        const bool live = row < n;
+        RowExtent e = {0, 0};
+        if (live) e = row_extent(rp, row);
+        const size_t idx = (size_t)(live ? row : 0) * V + v;
+        const double p = beta && live ? prev[idx] : 0.0;
+        double ah[V], ad[B];
+#pragma unroll
+        for (int u = 0; u < V; ++u) ah[u] = 0.0;
+#pragma unroll
+        for (int u = 0; u < B; ++u) ad[u] = 0.0;
+        for (int64_t q = e.q0 + kLaneEntries * l; q < e.q1; q += kLaneEntries * 16) {
+            // entries past the row's end are loaded with these and not used
+            const LaneCols lc = *reinterpret_cast<const LaneCols*>(col + q);
+            const LaneVals<double> lh = *reinterpret_cast<const LaneVals<double>*>(hv + q);
+            const LaneVals<double> ld = *reinterpret_cast<const LaneVals<double>*>(dv + q);
+            const int m = (int)min((int64_t)kLaneEntries, e.q1 - q);
+            double xv[kLaneEntries][V];
+#pragma unroll
+            for (int k = 0; k < kLaneEntries; ++k)
+                if (k < m) ld_vecs<double, V>(xv[k], x + (size_t)lc.c[k] * V);
+#pragma unroll
+            for (int k = 0; k < kLaneEntries; ++k)
+                if (k < m) {
+#pragma unroll
+                    for (int u = 0; u < V; ++u) ah[u] = fma(lh.h[k], xv[k][u], ah[u]);
+#pragma unroll
+                    for (int u = 0; u < B; ++u) ad[u] = fma(ld.h[k], xv[k][B + u], ad[u]);
+                }
+        }
+        const double y = alpha * fold_row<16>(ah, lane) - p;
+        const double d = fold_row<16>(ad, lane);
+        if (live && l % (16 / V) == 0) {
+            out[idx] = y;
+            if (v < B) hset[((size_t)v * M + j) * n + row] = y;
+        }
+        if (live && l % (16 / B) == 0) dset[((size_t)b * M + j - 1) * n + row] = d;
+    }
+}
+
+// x = [n][2B] and the betas' set at index 0: beta_0 = e_t, a_0 as given ([n][B])
+__global__ __launch_bounds__(kCondThreads) void pair_start_kernel(const int32_t* __restrict__ targets,
+                                                                  const double* __restrict__ a0, int n, int B, int M,
+                                                                  double* __restrict__ x, double* __restrict__ hset)
+{
+    const size_t total = (size_t)n * B;
+    for (size_t t = blockIdx.x * (size_t)kCondThreads + threadIdx.x; t < total; t += (size_t)gridDim.x * kCondThreads) {
+        const size_t i = t / B;
+        const int b = (int)(t % B);
+        const double e = (size_t)targets[b] == i ? 1.0 : 0.0;
+        x[i * 2 * B + b] = e;
+        x[i * 2 * B + B + b] = a0[t];
+        hset[(size_t)b * M * n + i] = e;
+    }
+}
+
+// the alpha half of x = [n][2B] as a block of its own
+__global__ __launch_bounds__(kCondThreads) void pair_alpha_kernel(const double* __restrict__ x, int n, int B,
+                                                                  double* __restrict__ a)
+{
+    const size_t total = (size_t)n * B;
+    for (size_t t = blockIdx.x * (size_t)kCondThreads + threadIdx.x; t < total; t += (size_t)gridDim.x * kCondThreads)
+        a[t] = x[t / B * 2 * B + B + t % B];
+}
+
+// 16 rows per workgroup and iteration, at most four workgroups a CU
+dim3 lanes_grid(int n)
+{
+    constexpr int rpi = kCondThreads / 16;
+    return dim3((unsigned)std::min(1024, std::max(8, ((n + rpi - 1) / rpi + 7) / 8 * 8)));
+}
+
 template <int B>
 hipError_t launch_dual_lanes(const int64_t* rp, const int32_t* col, const double* hv, const double* dv, const double* x,
                              const double* prev, double* out, double alpha, int beta, int n, int j, int M, double* hset,
                              double* dset, hipStream_t s)
 {
-    constexpr int rpi = kCondThreads / 16;
-    const int want = (n + rpi - 1) / rpi;
-    const dim3 g((unsigned)std::min(1024, std::max(8, (want + 7) / 8 * 8)));
+    const dim3 g = lanes_grid(n);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, g, dim3(kCondThreads), 0, s, rp, col, hv, dv, x, prev, out, alpha, beta, n, j, M, hset,
                            dset);
@@ -260,6 +358,37 @@ hipError_t launch_cond_dual_step(const int64_t* rp, const int32_t* col, const do
                            alpha, beta, n, B, j, M, hset, dset);
     else
         return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t launch_cond_pair_step(const int64_t* rp, const int32_t* col, const double* hv, const double* dv,
+                                 const double* x, const double* prev, double* out, double alpha, int beta, int n, int B,
+                                 int j, int M, double* hset, double* dset, hipStream_t s)
+{
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, lanes_grid(n), dim3(kCondThreads), 0, s, rp, col, hv, dv, x, prev, out, alpha, beta, n,
+                           j, M, hset, dset);
+        return hipGetLastError();
+    };
+    if (j < 1) return hipErrorInvalidValue;
+    switch (B) {
+    case 1: return launch(pair_step_kernel<1>);
+    case 2: return launch(pair_step_kernel<2>);
+    case 4: return launch(pair_step_kernel<4>);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_cond_pair_start(const int32_t* targets, const double* a0, int n, int B, int M, double* x, double* hset,
+                                  hipStream_t s)
+{
+    hipLaunchKernelGGL(pair_start_kernel, grid_for((size_t)n * B), dim3(kCondThreads), 0, s, targets, a0, n, B, M, x, hset);
+    return hipGetLastError();
+}
+
+hipError_t launch_cond_pair_alpha(const double* x, int n, int B, double* a, hipStream_t s)
+{
+    hipLaunchKernelGGL(pair_alpha_kernel, grid_for((size_t)n * B), dim3(kCondThreads), 0, s, x, n, B, a);
     return hipGetLastError();
 }
 

@@ -202,6 +202,16 @@ hipError_t launch_cond_scatter(const double* blk, int n, int B, int m, int M, do
 hipError_t launch_cond_dual_step(const int64_t* rp, const int32_t* col, const double* hv, const double* dv,
                                  const double* x, const double* prev, double* out, double alpha, int beta, int n, int B,
                                  int j, int M, double* hset, double* dset, hipStream_t s);
+// both recursions of up to kCondPair targets on x = [n][2B], betas first: x_j = alpha H x - (beta ? prev : 0),
+// its beta half into hset as vector j >= 1, dxH times the alpha half of x into dset as vector j - 1
+constexpr int kCondPair = 4;
+hipError_t launch_cond_pair_step(const int64_t* rp, const int32_t* col, const double* hv, const double* dv,
+                                 const double* x, const double* prev, double* out, double alpha, int beta, int n, int B,
+                                 int j, int M, double* hset, double* dset, hipStream_t s);
+// x_0 from the targets' unit vectors (also into hset as vector 0) and a0 = [n][B]; the alpha half of x
+hipError_t launch_cond_pair_start(const int32_t* targets, const double* a0, int n, int B, int M, double* x, double* hset,
+                                  hipStream_t s);
+hipError_t launch_cond_pair_alpha(const double* x, int n, int B, double* a, hipStream_t s);
 hipError_t launch_cond_weight(const double* C, int M, int T, double* X, hipStream_t s);
 // C[b] = sum_c part[b][c] (c = 0 .. S-1, fixed order), blocks of mm values
 hipError_t launch_cond_chunk_sum(const double* part, int S, size_t mm, int B, double* C, hipStream_t s);
