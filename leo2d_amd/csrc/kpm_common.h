@@ -130,13 +130,16 @@ __device__ inline float2 bc16(float2 v) { return make_float2(bc16<K>(v.x), bc16<
 // Blocks of few vectors put 16 lanes (64 where rows are long) on a matrix row.  A lane
 // takes three neighbouring entries, columns and values each in one wide load, gathers
 // all B vectors of each, and the lanes' sums are folded with DPP.  A pruned bilayer
-// row of 32 entries is one round of 48.  What bounds it: up to 4 real vectors the
-// matrix (12 B an entry, 3-4 TB/s), beyond that the gathers, which a CU's data path
-// returns at about 16 bytes a clock whatever the lane layout (TD 71 % busy while the
-// L1 hits 91 %; neighbouring lanes on one entry, or the next row's entries loaded
-// ahead, measured the same).  Microseconds per step on 95 k rows of 32 entries, lane
-// per vector before and this now: 4 real vectors 19.5 -> 15.9; on
-// 230 rows of 154 entries 17.1 -> 4.2.
+// row of 32 entries is one round of 48.  What bounds it: each row's chain of loads
+// (extent, entries, gathers: wavefronts wait three quarters of the time, and one vector
+// takes 11.5 us on 95 k rows where the matrix alone streams in 5) and, from 4 real
+// vectors on, the gathers, which a CU's data path returns at about 16 bytes a clock
+// whatever the lane layout (TD 71 % busy while the L1 hits 91 %).  Measured no faster:
+// neighbouring lanes on one entry, one entry a lane per load, the next row's entries
+// loaded ahead, a tile's neighbour rows staged in LDS (17.3 to 22.7 us), rows in
+// alternate directions.  Microseconds per step on 95 k rows of 32 entries, lane per
+// vector before and this now: 4 real vectors 19.5 -> 15.9; on 230 rows of 154 entries
+// 17.1 -> 4.2.
 constexpr int kLaneEntries = 3;
 // entries that may be loaded (and not used) past the end of a matrix's arrays
 static_assert(kLaneEntries <= kCsrPad, "padding of the CSR arrays");
