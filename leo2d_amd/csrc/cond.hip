@@ -205,8 +205,10 @@ __global__ __launch_bounds__(kCondThreads) void dual_step_lanes_kernel(const int
 // the alpha half; the new betas go straight into their set (vector j), D into its own
 // (vector j - 1).  Each matrix entry and each row's latencies serve both recursions:
 // microseconds per index on 95 k rows with 4 targets, H on the betas and both products
-// on the alphas one after the other 16.2 + 18.2, together 27.9.  Wider blocks keep
-// the recursions apart: from 8 vectors on the gathers bound the step either way.
+// on the alphas one after the other 16.2 + 18.2, together 27.9.  The line lies at four
+// targets: apart and together 25.3 and 14.9 with one, 27.0 and 18.6 with two, 52.9 and
+// 58.9 with eight, where 16 gathered values a row no longer leave several rounds in
+// flight (23.6 k rows: 11.1 and 5.8, 13.9 and 9.7 with four, 18.7 and 21.8 with eight).
 template <int B>
 __global__ __launch_bounds__(kCondThreads) void pair_step_kernel(const int64_t* __restrict__ rp,
                                                                  const int32_t* __restrict__ col,
