@@ -117,6 +117,7 @@ struct SellTiles {
     bool valid = false, failed = false, spatial = false;
     int ucap = 0, tmax = 0, ntiles = 0, ngroups = 0, tile_rows = 0, max_len = 0;
     int64_t entries = 0;
+    int builds = 0;      // layouts built so far: a captured graph reads the arrays of one of them
     DevBuf row0, u0, ucols, g0, grow, glen, goff, eu, val, val32;
     bool val_valid = false, val32_valid = false;
     DevBuf djob_tile0;   // first tile of each job when cut at job boundaries
@@ -196,12 +197,13 @@ struct leo2d_handle {
             int M, R, precision, mode, tile_rows, grid;
             uint64_t seed;
             const void *A, *B, *part, *mu, *val, *targets;
-            int copy_wave;
+            int copy_wave, sell_build;
             bool operator==(const GraphKey& o) const
             {
                 return M == o.M && R == o.R && precision == o.precision && mode == o.mode && tile_rows == o.tile_rows &&
                        grid == o.grid && seed == o.seed && A == o.A && B == o.B && part == o.part && mu == o.mu &&
-                       val == o.val && targets == o.targets && copy_wave == o.copy_wave;
+                       val == o.val && targets == o.targets && copy_wave == o.copy_wave &&
+                       sell_build == o.sell_build;
             }
         } key{};
         DevBuf A, B, part, mu, tgt;
@@ -369,6 +371,7 @@ bool build_sell_tiles(SellTiles& S, hipStream_t s, int n, const int64_t* drp, co
     S.tmax = tmax;
     S.spatial = spatial;
     S.valid = false;
+    ++S.builds;
     S.val_valid = S.val32_valid = false;
     // Segments of up to kSegTiles full tiles, fewer while that leaves less than 96: each is walked
     // by one wavefront, row after row, and ends in a tile cut short, which the steps pay for
@@ -2164,7 +2167,8 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
             const leo2d_handle::Batch::GraphKey key{M, R, p->precision, mode, T, grid, p->seed,
                                                      B.A.p, B.B.p, B.part.p, B.mu.p,
                                                      mode == LEO2D_BATCH_SELL ? ss.ev : dval, dtargets,
-                                                     mode == LEO2D_BATCH_SELL ? ss.copy_wave : 0};
+                                                     mode == LEO2D_BATCH_SELL ? ss.copy_wave : 0,
+                                                     mode == LEO2D_BATCH_SELL ? B.sell.builds : 0};
             if (!B.exec || !(key == B.key)) {
                 B.drop_graph();
                 hipGraph_t graph = nullptr;
