@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <set>
@@ -179,10 +180,21 @@ inline void check(hipError_t e, const char* what)
     }
 }
 
+// LEO2D_ALLOC_LIMIT: bytes above which an allocation fails as on a full device, so that what
+// a call leaves behind after a failed allocation can be tested on an empty one
+inline size_t alloc_limit()
+{
+    const char* e = std::getenv("LEO2D_ALLOC_LIMIT");
+    return e ? (size_t)std::strtoull(e, nullptr, 10) : SIZE_MAX;
+}
+
+// The old buffer goes first: where the allocation fails b is empty, so what describes b's
+// contents is cleared before the call, or the new buffer is a local one moved in when whole.
 inline void dalloc(DevBuf& b, size_t bytes, const char* what)
 {
     b.release();
     if (bytes == 0) bytes = 16;
+    if (bytes > alloc_limit()) check(hipErrorOutOfMemory, what);
     DevPool* const pool = DevPool::current();
     // a pooled buffer's size is rounded up (to an eighth of its power of two), so that calls on
     // slightly different sizes find each other's buffers

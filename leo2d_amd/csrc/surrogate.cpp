@@ -97,6 +97,7 @@ void ensure_capacity(leo2d_mlp* m, int rows)
 {
     if (rows <= m->cap) return;
     leo2d::DevPool::Use own(&m->pool);   // the network's buffers, whichever network's call this is
+    m->cap = 0;   // until every buffer is there
     const int cap = std::max(rows, 256);
     const int64_t ldt = leo2d::pad8(cap);
     const int64_t widest = leo2d::pad8(*std::max_element(m->dims.begin() + 1, m->dims.end()));

@@ -1,0 +1,50 @@
+"""A call whose device allocation fails returns LEO2D_ERR_ALLOC and leaves the handle as it
+was, or without what it could not replace: the next calls either give what a fresh handle
+gives, bit for bit, or refuse.  Failures are forced from the host: allocations above
+LEO2D_ALLOC_LIMIT bytes fail, at limits that stop a call at its first and at later buffers."""
+import numpy as np
+import pytest
+
+import leo2d_amd as L
+
+pytestmark = pytest.mark.gpu
+
+
+class _Limit:
+    """Allocations above `most` bytes fail inside the block, which has to end in ERR_ALLOC."""
+
+    def __init__(self, monkeypatch, most):
+        self.mp, self.most = monkeypatch, most
+
+    def __enter__(self):
+        self.mp.setenv("LEO2D_ALLOC_LIMIT", str(self.most))
+
+    def __exit__(self, kind, err, tb):
+        self.mp.delenv("LEO2D_ALLOC_LIMIT")
+        assert kind is L.Leo2dError and err.code == L.ERR_ALLOC, (kind, err)
+        return True
+
+
+# 600 rows of 40 -> 2 x 96 -> 200: bf16 inputs 48,000 bytes, FP32 inputs 96,000, outputs 480,000,
+# pre-activations 230,400
+@pytest.mark.parametrize("most", [1000, 50_000, 100_000, 300_000])
+def test_network_after_a_failed_allocation(monkeypatch, most):
+    rng = np.random.default_rng(0)
+    x = rng.standard_normal((600, 40)).astype(np.float32)
+    t = rng.standard_normal((600, 200)).astype(np.float32)
+    fresh = L.Mlp(0, 40, 96, 2, 200, seed=1)
+    loss, grad = fresh.gradients(x, t)
+    few = fresh.forward(x[:100])
+    fresh.close()
+    net = L.Mlp(0, 40, 96, 2, 200, seed=1)
+    assert np.array_equal(net.forward(x[:100]), few)
+    for _ in range(2):
+        with _Limit(monkeypatch, most):
+            net.gradients(x, t)
+        assert np.array_equal(net.forward(x[:100]), few)
+        with _Limit(monkeypatch, most):
+            L.mlp_ensemble([net], x)
+        got = net.gradients(x[:100], t[:100])
+        assert np.isfinite(got[0])
+    assert net.gradients(x, t)[0] == loss and np.array_equal(net.gradients(x, t)[1], grad)
+    net.close()
