@@ -1122,6 +1122,7 @@ int leo2d_csr_upload(leo2d_handle* h, int32_t n, int64_t nnz, const int64_t* row
         for (size_t q = 0; q < w * (size_t)nnz; ++q)
             if (!std::isfinite(val[q])) throw NanError("non-finite matrix value at entry " + std::to_string(q / w));
         hipStream_t s = h->stream;
+        h->has_csr = false;   // until the new one is whole (it takes the old one's room)
         to_device(h->rp, row_ptr, sizeof(int64_t) * (n + 1), s, "row pointers");
         to_device(h->col, col, sizeof(int32_t) * (size_t)nnz, s, "columns", sizeof(int32_t) * leo2d::kCsrPad);
         to_device(h->val, val, sizeof(double) * w * (size_t)nnz, s, "values", sizeof(double) * w * leo2d::kCsrPad);

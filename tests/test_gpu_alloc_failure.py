@@ -48,3 +48,44 @@ def test_network_after_a_failed_allocation(monkeypatch, most):
         assert np.isfinite(got[0])
     assert net.gradients(x, t)[0] == loss and np.array_equal(net.gradients(x, t)[1], grad)
     net.close()
+
+
+def _matrix(n, seed, half=3):
+    """Symmetric band of 2 half + 1 entries a row, spectrum inside [-1, 1]."""
+    rng = np.random.default_rng(seed)
+    A = np.zeros((n, n))
+    for k in range(1, half + 1):
+        i = np.arange(n - k)
+        A[i, i + k] = A[i + k, i] = rng.uniform(-1, 1, n - k)
+    A /= 1.01 * np.max(np.abs(A).sum(axis=1))
+    mask = A != 0
+    rp = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    return rp, np.nonzero(mask)[1].astype(np.int32), A[mask]
+
+
+# 900 rows of 6 entries: row pointers 7,208 bytes, columns 21,612, values 43,224
+@pytest.mark.parametrize("most", [1000, 10_000, 30_000])
+def test_upload_after_a_failed_allocation(monkeypatch, most):
+    """The handle holds no Hamiltonian (300 rows with other rows' pointers would read past
+    it) until the next upload; a batch keeps the one appended before."""
+    dev = L.Device(0)
+    small, large = _matrix(300, 1), _matrix(900, 2)
+    t = np.array([0, 5, 299])
+    dev.csr_upload(*small)
+    ref = dev.kpm(32, targets=t)
+    dev.batch_append()
+    bref = dev.batch_kpm(32, 4, seed=1)
+    for _ in range(2):
+        with _Limit(monkeypatch, most):
+            dev.csr_upload(*large)
+        for call in (dev.csr_info, dev.csr_copy, dev.spectral_bounds, dev.batch_append, lambda: dev.kpm(32, targets=t),
+                     lambda: dev.kpm(32, targets=t, noalloc=True)):
+            with pytest.raises(L.Leo2dError) as e:
+                call()
+            assert e.value.code == L.ERR_STATE
+        assert np.array_equal(dev.batch_kpm(32, 4, seed=1), bref)
+        dev.csr_upload(*small)
+        assert np.array_equal(dev.kpm(32, targets=t), ref)
+    dev.csr_upload(*large)
+    assert dev.csr_info()[0] == 900
+    dev.close()
