@@ -545,34 +545,39 @@ void batch_stack(leo2d_handle* h)
     }
     if (rows > 0x7fffffffLL) throw ArgError("batch exceeds 2^31 rows");
     const size_t vb = B.is_complex ? 16 : 8;
-    DevBuf rp, col, val;
+    std::vector<int64_t> row0 = B.job_row0;
+    for (auto& q : B.pending) row0.push_back(row0.back() + q.n);
+    DevBuf rp, col, val, drow0;   // the batch keeps its stack until the new one is whole
     dalloc(rp, sizeof(int64_t) * (size_t)(rows + 1), "batch row pointers");
     dalloc(col, sizeof(int32_t) * ((size_t)nnz + leo2d::kCsrPad), "batch columns");
     dalloc(val, vb * ((size_t)nnz + leo2d::kCsrPad), "batch values");
+    to_device(drow0, row0.data(), sizeof(int64_t) * row0.size(), s, "batch job rows");
     if (B.rows > 0) {
         check(hipMemcpyAsync(rp.p, B.rp.p, sizeof(int64_t) * (size_t)(B.rows + 1), hipMemcpyDeviceToDevice, s), "batch");
         check(hipMemcpyAsync(col.p, B.col.p, sizeof(int32_t) * (size_t)B.nnz, hipMemcpyDeviceToDevice, s), "batch");
         check(hipMemcpyAsync(val.p, B.val.p, vb * (size_t)B.nnz, hipMemcpyDeviceToDevice, s), "batch");
     }
+    int64_t r = B.rows, z = B.nnz;
     for (auto& q : B.pending) {
-        check(leo2d::launch_batch_offset((const int32_t*)q.col.p, q.nnz, (int32_t)B.rows, (int32_t*)col.p + B.nnz,
-                                         (const int64_t*)q.rp.p, q.n, B.nnz, (int64_t*)rp.p + B.rows, s),
+        check(leo2d::launch_batch_offset((const int32_t*)q.col.p, q.nnz, (int32_t)r, (int32_t*)col.p + z,
+                                         (const int64_t*)q.rp.p, q.n, z, (int64_t*)rp.p + r, s),
               "batch offsets");
         if (q.nnz)
-            check(hipMemcpyAsync((char*)val.p + vb * (size_t)B.nnz, q.val.p, vb * (size_t)q.nnz, hipMemcpyDeviceToDevice, s),
+            check(hipMemcpyAsync((char*)val.p + vb * (size_t)z, q.val.p, vb * (size_t)q.nnz, hipMemcpyDeviceToDevice, s),
                   "batch values");
-        B.rows += q.n;
-        B.nnz += q.nnz;
-        B.job_row0.push_back(B.rows);
+        r += q.n;
+        z += q.nnz;
     }
     check(hipStreamSynchronize(s), "batch stack");
     B.pending.clear();
+    B.rows = rows;
+    B.nnz = nnz;
+    B.job_row0 = std::move(row0);
     B.rp = std::move(rp);
     B.col = std::move(col);
     B.val = std::move(val);
+    B.drow0 = std::move(drow0);
     B.val32_valid = false;
-    to_device(B.drow0, B.job_row0.data(), sizeof(int64_t) * B.job_row0.size(), s, "batch job rows");
-    check(hipStreamSynchronize(s), "batch job rows");
     B.tile_rows = 0;
     B.sell.valid = B.sell.failed = false;
     B.sell.val_valid = B.sell.val32_valid = false;
@@ -588,6 +593,7 @@ void batch_tiles(leo2d_handle* h, int T)
     // the old tile arrays may still be read by queued steps or a captured graph
     check(hipStreamSynchronize(h->stream), "batch tiles");
     B.drop_graph();
+    B.tile_rows = 0;   // until both arrays are there
     const int P = (int)B.job_row0.size() - 1;
     B.tile_row0.clear();
     B.job_tile0.assign(1, 0);

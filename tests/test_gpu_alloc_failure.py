@@ -89,3 +89,47 @@ def test_upload_after_a_failed_allocation(monkeypatch, most):
     dev.csr_upload(*large)
     assert dev.csr_info()[0] == 900
     dev.close()
+
+
+def _jobs(dev, sizes):
+    for k, n in enumerate(sizes):
+        dev.csr_upload(*_matrix(n, 10 + k))
+        dev.batch_append()
+
+
+# stacked: 5,000 rows, 40,008 bytes of row pointers, 29,976 entries, 119,968 bytes of columns, 239,872 of values
+@pytest.mark.parametrize("most", [1000, 50_000, 150_000])
+def test_stack_after_a_failed_allocation(monkeypatch, most):
+    """Jobs appended after a run stay pending until their stack is whole."""
+    fresh = L.Device(0)
+    _jobs(fresh, (2000, 3000))
+    ref = fresh.batch_kpm(32, 4, seed=1)
+    fresh.close()
+    dev = L.Device(0)
+    _jobs(dev, (2000,))
+    for graph in (False, True):
+        first = dev.batch_kpm(32, 4, seed=1, graph=graph)
+        assert np.array_equal(first[0], ref[0])
+    dev.csr_upload(*_matrix(3000, 11))
+    dev.batch_append()
+    info = dev.batch_info()
+    for _ in range(2):
+        with _Limit(monkeypatch, most):
+            dev.batch_kpm(32, 4, seed=1)
+        assert dev.batch_info() == info == (2, 5000, info[2])
+    for graph in (False, True, True):
+        assert np.array_equal(dev.batch_kpm(32, 4, seed=1, graph=graph), ref)
+    dev.close()
+
+
+@pytest.mark.parametrize("mode", [L.BATCH_ROW_GROUPS, L.BATCH_ENTRY_SLOTS])
+def test_batch_tiles_after_a_failed_allocation(monkeypatch, mode):
+    """125 tiles of 16 rows are 504 bytes of first rows, 16 of 128 rows 68."""
+    dev = L.Device(0)
+    _jobs(dev, (2000,))
+    ref = dev.batch_kpm(32, 4, seed=1, mode=mode, tile_rows=128)
+    for graph in (False, True):
+        with _Limit(monkeypatch, 400):
+            dev.batch_kpm(32, 4, seed=1, mode=mode, tile_rows=16, graph=graph)
+        assert np.array_equal(dev.batch_kpm(32, 4, seed=1, mode=mode, tile_rows=128, graph=graph), ref)
+    dev.close()
