@@ -777,6 +777,7 @@ int leo2d_set_geometry(leo2d_handle* h, const leo2d_geom* gin)
         int mat0 = g.sheets[0].mat;
         for (const auto& sd : g.sheets)
             if (sd.mat != mat0) throw ArgError("sheets with different coupling models are not supported");
+        h->has_geom = false;   // until every array is there
         h->geom = g;
         h->has_pairs = false;
         h->has_csr = false;
@@ -858,6 +859,7 @@ int leo2d_pairs_build(leo2d_handle* h, int64_t* n_intra, int64_t* n_inter, int64
         if (!h->has_geom) throw StateError("leo2d_pairs_build before leo2d_set_geometry");
         const int n = h->gdev.n;
         hipStream_t s = h->stream;
+        h->has_pairs = false;   // until the new lists are whole
         dalloc(h->cnt_intra, sizeof(int32_t) * n, "pair counts");
         dalloc(h->cnt_tmp, sizeof(int64_t) * n, "pair counts");
         dalloc(h->pair_rp, sizeof(int64_t) * (n + 1), "pair offsets");
@@ -1077,6 +1079,7 @@ int leo2d_set_relaxation(leo2d_handle* h, int32_t max_k, const double* coeffs)
         for (size_t q = 0; q < count; ++q)
             if (!std::isfinite(coeffs[q])) throw NanError("relaxation coefficient is not finite");
         check(hipStreamSynchronize(h->stream), "relaxation");
+        h->relax_max_k = -1;   // until the new coefficients are there
         dalloc(h->relax, sizeof(double) * count, "relaxation coefficients");
         check(hipMemcpy(h->relax.p, coeffs, sizeof(double) * count, hipMemcpyHostToDevice), "relaxation upload");
         h->relax_max_k = max_k;

@@ -2,10 +2,15 @@
 was, or without what it could not replace: the next calls either give what a fresh handle
 gives, bit for bit, or refuse.  Failures are forced from the host: allocations above
 LEO2D_ALLOC_LIMIT bytes fail, at limits that stop a call at its first and at later buffers."""
+import os
+
 import numpy as np
 import pytest
 
+from conftest import ROOT
+
 import leo2d_amd as L
+from leo2d_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -132,4 +137,68 @@ def test_batch_tiles_after_a_failed_allocation(monkeypatch, mode):
         with _Limit(monkeypatch, 400):
             dev.batch_kpm(32, 4, seed=1, mode=mode, tile_rows=16, graph=graph)
         assert np.array_equal(dev.batch_kpm(32, 4, seed=1, mode=mode, tile_rows=128, graph=graph), ref)
+    dev.close()
+
+
+def _state_error(*calls):
+    for call in calls:
+        with pytest.raises(L.Leo2dError) as e:
+            call()
+        assert e.value.code == L.ERR_STATE
+
+
+# 944 orbitals: grid indices 15,104 bytes, positions 22,656, orders 3,776
+@pytest.mark.parametrize("most", [100, 10_000, 20_000])
+def test_geometry_after_a_failed_allocation(monkeypatch, most):
+    """No geometry until every array is there: another one's pairs would be searched on
+    arrays that are gone."""
+    old, new = (L.Geometry(L.Deck(W.tblg_flake_deck(3.0, r, M=16))) for r in (8.0, 20.0))
+    dev = L.Device(0)
+    dev.set_geometry(new)
+    dev.assemble(new.jobs()[0], L.PATTERN_PRUNED)
+    ref = dev.csr_copy()
+    dev.set_geometry(old)
+    dev.assemble(old.jobs()[0], L.PATTERN_PRUNED)
+    with _Limit(monkeypatch, most):
+        dev.set_geometry(new)
+    _state_error(dev.pairs_build, lambda: dev.assemble(new.jobs()[0], L.PATTERN_PRUNED), dev.csr_info)
+    dev.set_geometry(new)
+    dev.assemble(new.jobs()[0], L.PATTERN_PRUNED)
+    assert all(np.array_equal(a, b) for a, b in zip(dev.csr_copy(), ref))
+    dev.close()
+
+
+@pytest.mark.parametrize("most", [100, 5_000, 10_000])
+def test_pairs_after_a_failed_allocation(monkeypatch, most):
+    """944 orbitals: counts of 3,776 and 7,552 bytes, lists above; the next assembly searches
+    the pairs again."""
+    geom = L.Geometry(L.Deck(W.tblg_flake_deck(3.0, 20.0, M=16)))
+    dev = L.Device(0)
+    dev.set_geometry(geom)
+    dev.assemble(geom.jobs()[0], L.PATTERN_PRUNED)
+    ref = dev.csr_copy()
+    with _Limit(monkeypatch, most):
+        dev.pairs_build()
+    _state_error(dev.pairs_method)
+    dev.assemble(geom.jobs()[0], L.PATTERN_PRUNED)
+    assert all(np.array_equal(a, b) for a, b in zip(dev.csr_copy(), ref))
+    dev.close()
+
+
+def test_relaxation_after_a_failed_allocation(monkeypatch):
+    geom = L.Geometry(L.Deck(open(os.path.join(ROOT, "tests", "decks", "tblg_relax_cell.in")).read()))
+    job = geom.jobs()[0]
+    job.strain_type = 1
+    c = 1e-3 * np.random.default_rng(0).standard_normal((3, 4))   # max_k = 2: four coefficients a component
+    dev = L.Device(0)
+    dev.set_geometry(geom)
+    dev.set_relaxation(2, c)
+    dev.assemble(job, L.PATTERN_PRUNED)
+    ref = dev.csr_copy()
+    with _Limit(monkeypatch, 50):
+        dev.set_relaxation(2, c)
+    _state_error(lambda: dev.assemble(job, L.PATTERN_PRUNED))
+    dev.set_relaxation(2, c)
+    dev.assemble(job, L.PATTERN_PRUNED)
+    assert all(np.array_equal(a, b) for a, b in zip(dev.csr_copy(), ref))
     dev.close()
