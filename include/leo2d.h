@@ -235,7 +235,7 @@ int leo2d_batch_clear(leo2d_handle* h);
 int leo2d_batch_append(leo2d_handle* h, int32_t* job);
 int leo2d_batch_info(const leo2d_handle* h, int32_t* jobs, int64_t* rows, int64_t* nnz);
 
-#define LEO2D_BATCH_ROW_GROUPS 0    /* 64/R rows per wavefront (4 and 8 FP64 vectors: 16 lanes per row) */
+#define LEO2D_BATCH_ROW_GROUPS 0    /* 64/R rows per wavefront (4 and 8 real FP64 vectors: 16 lanes per row) */
 #define LEO2D_BATCH_ENTRY_SLOTS 1   /* one row per wavefront, 64/R entries in flight */
 #define LEO2D_BATCH_ROW_CHUNKS 2    /* R = 16, 32: 64/R rows per wavefront, 16-entry chunks broadcast in 16-lane rows */
 #define LEO2D_BATCH_SELL 3          /* complex vectors, R = 16 or 32 (FP32: 32): SELL-4-sigma row tiles cut at job

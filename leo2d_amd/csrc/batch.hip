@@ -16,8 +16,8 @@
 //
 // Two lane layouts for R < 64 vectors (both parity-tested):
 //   mode 0 ("row groups"):  64/R rows per wavefront, R lanes per row, entries
-//                           of a row walked sequentially by its lanes (4 and 8 FP64
-//                           vectors: a group of lanes per row);
+//                           of a row walked sequentially by its lanes (4 and 8 real
+//                           FP64 vectors: 16 lanes per row);
 //   mode 1 ("entry slots"): one row per wavefront, 64/R entries of the row in
 //                           flight at once (lanes e, e+R, ...), folded with
 //                           cross-lane shuffles at the end of the row;
@@ -264,15 +264,19 @@ __global__ __launch_bounds__(kThreads) void batch_step_chunk_kernel(BatchStepArg
     }
 }
 
-// Mode 0 with 4 or 8 FP64 vectors: 16 lanes per matrix row (kpm_common.h), sixteen
+// Mode 0 with 4 or 8 real FP64 vectors: 16 lanes per matrix row (kpm_common.h), sixteen
 // wavefronts per tile, so a tile of 128 rows is two rounds of 64 rows; with a lane per
-// vector it was sixteen, each a chain of eight rounds of gathers (eight cells of 1-3
-// degrees, 4 real vectors: 13.7 -> 12.6 us a step).
+// vector it is sixteen, each a chain of eight rounds of gathers.  Microseconds a step, a
+// lane per vector and this: eight cells of 1-3 degrees, 4 vectors 13.7 and 12.6; 8,128 /
+// 35,724 / 95,264 rows in cells, 4 vectors 7.9 and 6.7 / 12.9 and 12.3 / 19.1 and 18.6,
+// 8 vectors 13.6 and 9.4 / 23.2 and 18.3 / 31.1 and 27.3.  Complex vectors keep a lane per
+// vector: eight of them need more registers than 1,024 threads leave a lane (35,724 rows
+// 25.2 against 75.7 here), and four gather rows as wide as eight real ones (8.1 against
+// 9.4, 13.6 against 18.4, 21.1 against 27.4).
 constexpr int kLaneWaves = 16;
-template <typename HT, typename XT, int R>
+template <int R>
 __global__ __launch_bounds__(64 * kLaneWaves) void batch_step_lanes_kernel(BatchStepArgs a)
 {
-    using AT = typename acc_of<XT>::type;
     constexpr int DUP = 16 / R;          // lanes that end with the same vector
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -283,10 +287,10 @@ __global__ __launch_bounds__(64 * kLaneWaves) void batch_step_lanes_kernel(Batch
     const int b = blockIdx.x;
     const int lb = (b & 7) * (G >> 3) + (b >> 3);
 
-    const HT* __restrict__ val = static_cast<const HT*>(a.val);
+    const double* __restrict__ val = static_cast<const double*>(a.val);
     const int32_t* __restrict__ col = a.col;
-    const XT* __restrict__ cur = static_cast<const XT*>(a.cur);
-    XT* out = static_cast<XT*>(a.out);   // holds T_{j-1} on entry, T_{j+1} on exit
+    const double* __restrict__ cur = static_cast<const double*>(a.cur);
+    double* out = static_cast<double*>(a.out);   // holds T_{j-1} on entry, T_{j+1} on exit
     const bool beta = a.beta != 0;
 
     __shared__ double red[kLaneWaves][R][2];
@@ -300,22 +304,20 @@ __global__ __launch_bounds__(64 * kLaneWaves) void batch_step_lanes_kernel(Batch
             RowExtent e = {0, 0};
             if (live) e = row_extent(a.row_ptr, row);
             const size_t idx = (size_t)(live ? row : row0) * R + r;
-            const XT cv = cur[idx];
-            XT p;
-            zero(p);
-            if (beta && live) p = out[idx];
-            AT acc[R];
+            const double cv = cur[idx];
+            const double p = beta && live ? out[idx] : 0.0;
+            double acc[R];
 #pragma unroll
-            for (int v = 0; v < R; ++v) zero(acc[v]);
+            for (int v = 0; v < R; ++v) acc[v] = 0.0;
             for (int64_t q = e.q0 + kLaneEntries * l; q < e.q1; q += kLaneEntries * 16) {
                 // entries past the row's end are loaded with these and not used
                 const LaneCols lc = *reinterpret_cast<const LaneCols*>(col + q);
-                const LaneVals<HT> lv = *reinterpret_cast<const LaneVals<HT>*>(val + q);
+                const LaneVals<double> lv = *reinterpret_cast<const LaneVals<double>*>(val + q);
                 const int m = (int)min((int64_t)kLaneEntries, e.q1 - q);
-                XT x[kLaneEntries][R];
+                double x[kLaneEntries][R];
 #pragma unroll
                 for (int k = 0; k < kLaneEntries; ++k)
-                    if (k < m) ld_vecs<XT, R>(x[k], cur + (size_t)lc.c[k] * R);
+                    if (k < m) ld_vecs<double, R>(x[k], cur + (size_t)lc.c[k] * R);
 #pragma unroll
                 for (int k = 0; k < kLaneEntries; ++k)
                     if (k < m) {
@@ -323,9 +325,9 @@ __global__ __launch_bounds__(64 * kLaneWaves) void batch_step_lanes_kernel(Batch
                         for (int v = 0; v < R; ++v) mac(acc[v], lv.h[k], x[k][v]);
                     }
             }
-            const AT s = fold_row<16>(acc, lane);
+            const double s = fold_row<16>(acc, lane);
             if (live && writer) {
-                const XT o = comb(a.alpha, s, p);
+                const double o = comb(a.alpha, s, p);
                 out[idx] = o;
                 d1 += nrm2(cv);
                 d2 += redot(o, cv);
@@ -451,14 +453,10 @@ hipError_t launch_mode(const BatchStepArgs& a, hipStream_t s)
     } else {
         if (a.mode == 2) return hipErrorInvalidValue;
     }
-    if constexpr (R <= 8 && (std::is_same<XT, double>::value || std::is_same<XT, double2>::value)) {
-        if (a.mode == 0) {
-            hipLaunchKernelGGL((batch_step_lanes_kernel<HT, XT, R>), dim3(a.grid), dim3(64 * kLaneWaves), 0, s, a);
-            return hipGetLastError();
-        }
-    }
     if (a.mode == 1)
         hipLaunchKernelGGL((batch_step_kernel<HT, XT, R, 1>), dim3(a.grid), dim3(kThreads), 0, s, a);
+    else if constexpr (R <= 8 && std::is_same<XT, double>::value)
+        hipLaunchKernelGGL(batch_step_lanes_kernel<R>, dim3(a.grid), dim3(64 * kLaneWaves), 0, s, a);
     else
         hipLaunchKernelGGL((batch_step_kernel<HT, XT, R, 0>), dim3(a.grid), dim3(kThreads), 0, s, a);
     return hipGetLastError();
