@@ -70,21 +70,49 @@ int sell_tile_rows(int n, int most, int cus)
     return (int)std::max<int64_t>(16, std::min<int64_t>(most, (rows + 3) / 4 * 4));
 }
 
-// step kernel for a block of B vectors on n rows (LEO2D_KPM_VARIANT = 0, 1, 2, 14,
-// 15 or 20 overrides the default).  FP64 blocks of at most 8 vectors run a group of
-// lanes per row (2) in either order.  In the spatial order: B = 16, 32 or 64 run
+// The lanes-per-row kernel takes a wavefront per row instead of 16 lanes where rows are long: the
+// rows of a bilayer's pruned pattern hold about 32 entries, those of the reference pattern 150 to
+// 300.  Where few rows leave the GPU idle a row's own chain of loads is the time and 64 lanes win
+// early; where rows fill it, they have to be kept busy.  us a step with 16 and 64 lanes, 4 real
+// vectors, rows of 41 / 65 / 97 / 129 entries: 500 rows 3.6 and 3.5 / 4.3 and 3.5 / 4.8 and 3.5 /
+// 4.9 and 3.5, 20,000 rows 7.2 and 11.8 / 10.1 and 12.2 / 12.4 and 12.9 / 15.0 and 14.5.
+constexpr int kFewRows = 8192;
+bool long_rows(int n, int64_t nnz) { return nnz > (n < kFewRows ? 64 : 96) * (int64_t)n; }
+
+// FP64 blocks of at most 8 vectors: 16 or 64 lanes per row (2) or a lane per vector (0).  The first
+// crosses a row's chain of loads faster; the second gathers a wide row of vectors in fewer loads, and
+// wins where the rows fill the GPU.  us a step, lane per vector against lanes per row, complex vectors:
+//   8 (128 bytes a row) on 2,114 / 4,784 / 14,378 / 94,676 / 190,528 rows of 32: 6.4 against 5.5, 6.6
+//   against 7.6, 8.0 against 13.0, 38.6 against 57.3, 73 against 111; rows of 290 of a complex H: 4,572
+//   rows 41 against 36, 8,128 rows 47 against 44, 11,908 rows 54 against 63;
+//   4 (64 bytes) on 11,908 / 20,176 / 64,412 / 130,622 rows: 6.8 against 6.1, 8.2 against 9.2, 13.9
+//   against 18.0, 28.3 against 33.4; past the 131,072 rows that one round of a lane per vector covers
+//   48 against 38 on 147,782, 64 against 50 on 190,528; rows of 290: 59 against 51 on 20,176.
+// Narrower rows (real vectors up to 8, complex up to 2) run lanes per row throughout (8 real on 2,114
+// / 23,642 / 94,676 rows 6.4 against 4.2, 9.3 against 9.8, 36.6 against 26.1).
+int few_vectors_variant(bool cpx_vec, bool cpx_h, int B, int n, int64_t nnz)
+{
+    const bool lr = long_rows(n, nnz);
+    if (cpx_vec && B == 8) return n < (cpx_h && lr ? kFewRows : 4096) ? 2 : 0;
+    if (cpx_vec && B == 4 && !lr && n >= 16384 && n <= 131072) return 0;
+    return 2;
+}
+
+// step kernel for a block of B vectors on n rows of nnz entries (LEO2D_KPM_VARIANT =
+// 0, 1, 2, 14, 15 or 20 overrides the default).  FP64 blocks of at most 8 vectors:
+// few_vectors_variant, in either order.  In the spatial order: B = 16, 32 or 64 run
 // the SELL-4-sigma step with LDS-staged row tiles (20) where its layout applies
 // and n >= kSellMinRows (kSellMinRows64), else vector chunks split over the XCDs
 // (14; at B = 64 only below that).  In the natural order (or where neither applies): B >= 64
 // the wavefront-per-row kernel (1), or for the FP32 recursion at B = 64 two rows
 // per wavefront with 16-byte gathers (15); other B lane per vector (0).
-int kpm_variant(bool mixed, bool spatial, int B, int n)
+int kpm_variant(bool mixed, bool spatial, bool cpx_vec, bool cpx_h, int B, int n, int64_t nnz)
 {
     if (const char* e = std::getenv("LEO2D_KPM_VARIANT")) {
         const int v = std::atoi(e);
         if (v == 0 || v == 1 || v == 2 || v == 14 || v == 15 || v == kVariantSell) return v;
     }
-    if (!mixed && B <= 8) return 2;
+    if (!mixed && B <= 8) return few_vectors_variant(cpx_vec, cpx_h, B, n, nnz);
     if (spatial && (B == 16 || B == 32)) return n >= kSellMinRows ? kVariantSell : 14;
     if (spatial && B == 64 && n < kSellMinRows64) return 14;
     if (spatial && B >= 64) return kVariantSell;
@@ -1199,10 +1227,6 @@ int leo2d_spectral_bounds(leo2d_handle* h, double* lo, double* hi)
 // ---- KPM --------------------------------------------------------------------
 namespace {
 
-// the lanes-per-row kernel takes a whole wavefront per row: the rows of a bilayer's pruned
-// pattern hold about 32 entries, those of the reference pattern 150 to 300
-bool long_rows(int n, int64_t nnz) { return nnz > 64 * (int64_t)n; }
-
 // workgroups of a step launch when the caller leaves the grid to the library.
 // R >= 64: four workgroups per CU (one wavefront per row); fewer rows in flight
 // keep each XCD's gathered rows in its L2 (measured best on the 1.05 deg 8x8
@@ -1344,7 +1368,7 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
         if (p->scheme == LEO2D_SCHEME_DOUBLING) dev_scheme = 1;
         else dev_scheme = p->start == LEO2D_START_TARGETS ? 0 : 2;
         const bool keep_v = dev_scheme == 2;
-        const int wanted = kpm_variant(mixed, spatial, B, n);
+        const int wanted = kpm_variant(mixed, spatial, !real_vec, h->is_complex, B, n, h->nnz);
         const int G = p->grid > 0 ? p->grid : auto_grid(wanted, n, h->nnz, B);
         if (G % 8 != 0) throw ArgError("grid must be a multiple of 8");
         const size_t vb = leo2d::vec_bytes(vec_type);
@@ -1531,10 +1555,10 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
         if (!base) throw StateError("static device scratch not initialised on this device");
         const int M = p->M, R = p->R, n = h->n;
         const int B = p->block ? p->block : std::min(64, next_pow2(R));
-        // the kernel leo2d_kpm_moments picks for the reference row order in FP64
-        int variant = kpm_variant(false, false, B, n);
         const bool real_vec = !h->is_complex && (p->start == LEO2D_START_TARGETS ||
-                                                   (p->start == LEO2D_START_VECTORS && !p->vectors_complex));
+                                                 (p->start == LEO2D_START_VECTORS && !p->vectors_complex));
+        // the kernel leo2d_kpm_moments picks for the reference row order in FP64
+        int variant = kpm_variant(false, false, !real_vec, h->is_complex, B, n, h->nnz);
         int G = p->grid > 0 ? p->grid : auto_grid(variant, n, h->nnz, B);
         if (variant == kVariantSell) variant = B == 16 || B == 32 ? 14 : 1;
         if (variant == 14 && B != 16 && B != 32 && B != 64 && B != 128) variant = 1;
@@ -1568,7 +1592,7 @@ int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double
         // a request that only just fits takes fewer workgroups (and partials) than leo2d_kpm_moments
         // would, down to the eight of a small matrix's lane-per-vector launch
         auto part_bytes = [&]() { return (sizeof(double) * 3 * (size_t)G * B + 255) / 256 * 256; };
-        while (p->grid == 0 && variant == 2 && G > 8 && off + part_bytes() > leo2d::kScratchBytes) G = G / 16 * 8;
+        while (p->grid == 0 && B <= 8 && G > 8 && off + part_bytes() > leo2d::kScratchBytes) G = G / 16 * 8;
         const size_t part_step = sizeof(double) * 3 * (size_t)G * B;
         const size_t oPart = take(part_step);
         if (off > leo2d::kScratchBytes)

@@ -6,6 +6,7 @@ Against a dense FP64 recursion; 1e-12 mu_0 as in test_gpu_parity.py (the sums
 run in another order)."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import leo2d_amd as L
 
@@ -85,4 +86,41 @@ def test_small_batch_blocks(R, cpx):
             E = np.zeros((A.shape[0], R))
             E[t, np.arange(R)] = 1.0
             assert np.max(np.abs(m - _moments(A, E, 48))) <= 1e-12
+    dev.close()
+
+
+def _band(n, half, cpx, rng):
+    """Hermitian band of 2 half + 1 entries a row (fewer at its ends), spectrum inside [-1, 1]."""
+    d = {0: rng.standard_normal(n)}
+    for k in range(1, half + 1):
+        v = rng.standard_normal(n - k) + (1j * rng.standard_normal(n - k) if cpx else 0)
+        d[k], d[-k] = v, np.conj(v)
+    A = sp.diags(list(d.values()), list(d.keys()), format="csr")
+    A = A / (1.01 * np.max(abs(A).sum(axis=1)))
+    A.sort_indices()
+    return A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data, A
+
+
+# either side of each line of the choice between lanes per row (2) and a lane per vector (0), and of
+# 16 against 64 lanes per row: rows, half band, complex H, vectors, kernel
+@pytest.mark.parametrize("n,half,cpx,R,kernel", [
+    (4095, 15, False, 8, 2), (4096, 15, False, 8, 0), (4097, 15, True, 5, 0), (8191, 40, True, 8, 2),
+    (8191, 40, False, 8, 0), (8192, 50, True, 8, 0), (16383, 15, True, 4, 2), (16384, 15, True, 3, 0),
+    (16384, 50, False, 4, 2), (131072, 2, False, 4, 0), (131073, 2, True, 4, 2), (131073, 2, False, 2, 2),
+    (8191, 33, False, 2, 2), (8192, 33, True, 1, 2), (8193, 50, False, 2, 2)])
+def test_few_vectors_on_many_rows(n, half, cpx, R, kernel):
+    """Complex vectors, FP64, against the same recursion in numpy; 1e-12 mu_0 as above."""
+    rng = np.random.default_rng(n + half)
+    rp, ci, v, A = _band(n, half, cpx, rng)
+    X = rng.standard_normal((R, n)) + 1j * rng.standard_normal((R, n))
+    dev = L.Device(0)
+    dev.csr_upload(rp, ci, v)
+    M = 16
+    ref = _moments(A, X.T, M)
+    print("case", n, half, cpx, R, flush=True)
+    mu = dev.kpm(M, vectors=X)
+    assert dev.timing().kernel == kernel
+    assert np.max(np.abs(mu - ref)) <= 1e-12 * np.max(ref[:, 0])
+    if 2 * n * 16 * 8 < 30_000_000:
+        assert np.array_equal(mu, dev.kpm(M, vectors=X, noalloc=True))
     dev.close()
