@@ -132,7 +132,8 @@ __global__ __launch_bounds__(kCondThreads) void dual_step_kernel(const int64_t* 
 // entries and then its gathers are in flight together, where the kernel above walks
 // them eight at a time and reads every column and value once per vector.  The
 // gathers serve both products (95 k rows, 4 targets: 34.9 -> 18.2 us with both
-// products, 20.4 -> 16.2 us with one).
+// products, 20.4 -> 16.2 us with one; both recursions, us an index: 8 targets on 2.1 k /
+// 23.6 k / 94.7 k rows 14.9 -> 8.3 / 24.4 -> 18.8 / 74.4 -> 52.9, 16 targets lanes_grid).
 template <bool HAS_H, bool HAS_D, int B>
 __global__ __launch_bounds__(kCondThreads) void dual_step_lanes_kernel(const int64_t* __restrict__ rp,
                                                                        const int32_t* __restrict__ col,
@@ -295,11 +296,13 @@ __global__ __launch_bounds__(kCondThreads) void pair_alpha_kernel(const double* 
         a[t] = x[t / B * 2 * B + B + t % B];
 }
 
-// 16 rows per workgroup and iteration, at most four workgroups a CU
-dim3 lanes_grid(int n)
+// 16 rows per workgroup and iteration, at most four workgroups a CU; with 16 vectors two, as many as
+// their registers leave room for at a time (23.6 k rows, both recursions: 43.4 us an index with four,
+// 34.7 with two, 39.6 with a thread per row and vector; 94.7 k rows 117, 114 and 123).
+dim3 lanes_grid(int n, int B)
 {
     constexpr int rpi = kCondThreads / 16;
-    return dim3((unsigned)std::min(1024, std::max(8, ((n + rpi - 1) / rpi + 7) / 8 * 8)));
+    return dim3((unsigned)std::min(B < 16 ? 1024 : 512, std::max(8, ((n + rpi - 1) / rpi + 7) / 8 * 8)));
 }
 
 template <int B>
@@ -307,7 +310,7 @@ hipError_t launch_dual_lanes(const int64_t* rp, const int32_t* col, const double
                              const double* prev, double* out, double alpha, int beta, int n, int j, int M, double* hset,
                              double* dset, hipStream_t s)
 {
-    const dim3 g = lanes_grid(n);
+    const dim3 g = lanes_grid(n, B);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, g, dim3(kCondThreads), 0, s, rp, col, hv, dv, x, prev, out, alpha, beta, n, j, M, hset,
                            dset);
@@ -368,7 +371,7 @@ hipError_t launch_cond_pair_step(const int64_t* rp, const int32_t* col, const do
                                  int j, int M, double* hset, double* dset, hipStream_t s)
 {
     const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, lanes_grid(n), dim3(kCondThreads), 0, s, rp, col, hv, dv, x, prev, out, alpha, beta, n,
+        hipLaunchKernelGGL(kernel, lanes_grid(n, B), dim3(kCondThreads), 0, s, rp, col, hv, dv, x, prev, out, alpha, beta, n,
                            j, M, hset, dset);
         return hipGetLastError();
     };

@@ -25,3 +25,18 @@ def test_pair_matches_separate(radius, M):
         got = dev.cond_moments(M, targets, block=block)
         assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(ref)), block
     dev.close()
+
+
+@pytest.mark.parametrize("radius", [13.0, 60.0])
+def test_sixteen_targets(radius):
+    """Blocks of 16 on fewer and on more rows than their launch covers in one round."""
+    dev = L.Device(0)
+    geom = L.Geometry(L.Deck(W.tblg_flake_deck(3.0, radius, M=64)))
+    dev.set_geometry(geom)
+    dev.assemble_velocity(geom.jobs()[0], L.PATTERN_PRUNED)
+    targets = [int(t) for t in np.linspace(0, geom.n - 1, 17)]
+    print("case", geom.n, flush=True)
+    ref = dev.cond_moments(12, targets, block=4)
+    got = dev.cond_moments(12, targets, block=16)
+    assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(ref))
+    dev.close()
