@@ -227,7 +227,8 @@ int leo2d_last_timing(const leo2d_handle* h, leo2d_timing* t);
  * vector p*R + r of the LEO2D_START_RANDOM_PHASE generator, orbital index
  * local to the job) or unit vectors on R of its orbitals (local DoS, as
  * computeDosKPM's targets), and its moments by the doubling identity from the
- * first step. */
+ * first step.  leo2d_batch_clear drops the jobs and gives the device memory the
+ * handle keeps for its next calls back, down to 256 MiB. */
 int leo2d_batch_clear(leo2d_handle* h);
 /* Append the current device Hamiltonian (from leo2d_assemble or
  * leo2d_csr_upload, in its own row order) as the next job; *job (may be NULL)

@@ -1890,6 +1890,7 @@ int leo2d_batch_clear(leo2d_handle* h)
         check(hipStreamSynchronize(h->stream), "batch clear");
         h->batch.drop_graph();
         h->batch = leo2d_handle::Batch();
+        h->pool.trim(leo2d::DevPool::kPoolCleared);   // a large stack's memory goes back to the device
         return LEO2D_OK;
     });
 }

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <set>
@@ -26,12 +27,14 @@ namespace leo2d {
 // written only by work queued after its last use.
 // Bounded: buffers of at most kPoolMost bytes, at most kPoolKeep in all handles of the
 // process (a handle's longest unused go first); all of every handle are freed when an
-// allocation fails, a handle's own with it.  A pool serves its handle alone; the lock
+// allocation fails, a handle's own with it, and leo2d_batch_clear leaves its handle at most
+// kPoolCleared.  A pool serves its handle alone; the lock
 // is for the handle whose allocation failed.
 class DevPool {
 public:
     static constexpr size_t kPoolMost = size_t(2) << 30;
     static constexpr size_t kPoolKeep = size_t(4) << 30;
+    static constexpr size_t kPoolCleared = size_t(256) << 20;   // the buffers of small calls
     DevPool()
     {
         std::lock_guard<std::mutex> g(all().lock);
@@ -77,10 +80,18 @@ public:
         }
         (void)hipFree(p);
     }
-    void clear()
+    void clear() { trim(0); }
+    // frees the largest kept buffers until at most `most` bytes are left
+    void trim(size_t most)
     {
         std::lock_guard<std::mutex> g(lock_);
-        while (!free_.empty()) (void)hipFree(drop(free_.begin()));
+        size_t kept = 0;
+        for (const auto& f : free_) kept += f.first;
+        while (kept > most) {
+            const auto it = std::prev(free_.end());
+            kept -= it->first;
+            (void)hipFree(drop(it));
+        }
     }
     // every handle's kept buffers (a free waits for the work that may still use them)
     static void clear_all()

@@ -1,6 +1,7 @@
 """Device buffers a handle keeps between calls: calls of other sizes and kinds in
 between, and other handles on other threads, leave every result bit for bit what
 a fresh handle gives."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -91,3 +92,32 @@ def test_large_buffers_of_many_handles():
         assert np.array_equal(got, ref)
     for dev in devs:
         dev.close()
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert L.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0   # the runtime the library runs on
+    return free.value
+
+
+def test_batch_clear_gives_memory_back():
+    """A stack of 571,584 rows with blocks of 32 vectors takes some 1.2 GB; after the clear
+    the device has all but 256 MiB of it again."""
+    dev = L.Device(0)
+    geom = L.Geometry(L.Deck(W.tblg_cell_deck(32, 31, 4, M=8)))
+    dev.set_geometry(geom)
+    W.assemble_rescaled(dev, geom, (0.2, 0.1))
+    dev.batch_clear()
+    before = _free_bytes()
+    for _ in range(3):
+        dev.batch_append()
+    mu = dev.batch_kpm(8, 32, seed=1)
+    during = _free_bytes()
+    assert before - during > 900 << 20
+    dev.batch_clear()
+    after = _free_bytes()
+    assert before - after <= 320 << 20   # and what the runtime rounds up
+    for _ in range(3):
+        dev.batch_append()
+    assert np.array_equal(dev.batch_kpm(8, 32, seed=1), mu)
+    dev.close()
