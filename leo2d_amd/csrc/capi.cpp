@@ -125,6 +125,14 @@ int env_int(const char* k, int d)
     return e ? std::atoi(e) : d;
 }
 
+// bytes of step partials collected before a reduction (LEO2D_PARTIAL_SPACE overrides the default,
+// so that a short recursion reduces several times as a long one does)
+size_t partial_space(size_t d)
+{
+    const char* e = std::getenv("LEO2D_PARTIAL_SPACE");
+    return e ? (size_t)std::strtoull(e, nullptr, 10) : d;
+}
+
 // row schedule of the wavefront-per-row kernels: 1 = one contiguous slice of
 // rows per XCD (LEO2D_KPM_SCHED overrides the default)
 int kpm_sched()
@@ -1376,7 +1384,7 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
         dalloc(A, vb * (size_t)n * B, "vector block");
         dalloc(Bf, vb * (size_t)n * B, "vector block");
         if (keep_v) dalloc(V, vb * (size_t)n * B, "start vectors");
-        dalloc(part, std::max(sizeof(double) * 3 * (size_t)G * B, leo2d::kPartialSpace), "partials");
+        dalloc(part, std::max(sizeof(double) * 3 * (size_t)G * B, partial_space(leo2d::kPartialSpace)), "partials");
         dalloc(dmu, sizeof(double) * (size_t)M * B, "moments");
         dalloc(dtg, sizeof(int32_t) * B, "targets");
         double rec_ms = 0.0, step_ms = 0.0;
@@ -2027,7 +2035,7 @@ int leo2d_batch_kpm(leo2d_handle* h, const leo2d_batch_params* p, double* mu)
         ensure(B.B, vbytes, "batch vectors");
         // partials of one step under any tiling, or of as many steps as kBatchPartialSpace holds
         const size_t part_max = sizeof(double) * 2 * (size_t)std::max<int64_t>(max_tiles, 1) * R;
-        const size_t part_space = part_max * (size_t)leo2d::reduce_every(part_max, leo2d::kBatchPartialSpace, M);
+        const size_t part_space = part_max * (size_t)leo2d::reduce_every(part_max, partial_space(leo2d::kBatchPartialSpace), M);
         ensure(B.part, part_space, "batch partials");
         ensure(B.mu, sizeof(double) * (size_t)P * R * M, "batch moments");
 
