@@ -925,15 +925,16 @@ __device__ inline void add_pair(const GeomDev& g, const JobDev& j, const double*
 // The whole pattern of a 230-orbital flake: 706 us then, 18 us now.
 constexpr int kFillWaves = 4;   // rows (wavefronts) per workgroup
 
-// lane l looks at pair b + l of the row's list [q0, q1): the end of its run when it heads one, else 0
+// a row's pairs and their runs of equal columns inside either list
 struct RowLists {
     int64_t q0, qi, q1;   // intralayer pairs [q0, qi), interlayer pairs [qi, q1)
     const int32_t* pcol;
+    // pair q is the first of its run
     __device__ inline bool head(int64_t q) const
     {
         return q < q1 && (q == q0 || q == qi || pcol[q] != pcol[q - 1]);
     }
-    // pairs of the run that starts at q: q .. end(q) - 1
+    // pair p >= q still belongs to the run that starts at q
     __device__ inline bool more(int64_t q, int64_t p) const
     {
         return p < (q < qi ? qi : q1) && pcol[p] == pcol[q];

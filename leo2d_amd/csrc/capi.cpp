@@ -1550,7 +1550,8 @@ int leo2d_kpm_moments(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
 // memory is allocated or freed.  Layout of one block of B vectors, each region
 // 256-byte aligned: T_j and T_{j+1} blocks [n][B], the start vectors (reference
 // scheme with caller vectors), the upload staging of caller vectors [B][w n],
-// the step partials [grid][B][3], the moments [B][M] and the targets [B].
+// the moments [B][M], the targets [B], and the step partials [grid][B][3] of as
+// many steps as the rest of the scratch holds.
 int leo2d_kpm_moments_noalloc(leo2d_handle* h, const leo2d_kpm_params* p, double* mu)
 {
     if (!h || !p || !mu) return LEO2D_ERR_ARG;

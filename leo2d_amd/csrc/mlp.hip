@@ -3,7 +3,7 @@
 // The surrogate is a small multilayer perceptron (64 Fourier features of a
 // local stacking configuration -> hidden GELU layers -> local Chebyshev
 // moments).  Weights and activations are bfloat16, every product accumulates
-// in FP32 on the matrix cores (v_mfma_f32_16x16x16_bf16), and the optimiser
+// in FP32 on the matrix cores (v_mfma_f32_16x16x32_bf16), and the optimiser
 // keeps FP32 master weights.  There is no counterpart in the reference; the
 // moments it learns come from the KPM recursion of this library.
 //
