@@ -316,11 +316,10 @@ hipError_t launch_dual_lanes(const int64_t* rp, const int32_t* col, const double
                            dset);
         return hipGetLastError();
     };
-    // up to kCondPair vectors take H in pair_step_kernel; here only dxH alone (a_0, the last D)
-    if constexpr (B > kCondPair) {
+    // both products of up to kCondPair vectors are pair_step_kernel's
+    if constexpr (B > kCondPair)
         if (hv && dv) return launch(dual_step_lanes_kernel<true, true, B>);
-        if (hv) return launch(dual_step_lanes_kernel<true, false, B>);
-    }
+    if (hv && !dv) return launch(dual_step_lanes_kernel<true, false, B>);
     if (!hv && dv) return launch(dual_step_lanes_kernel<false, true, B>);
     return hipErrorInvalidValue;
 }
