@@ -14,7 +14,7 @@
 // vector, so the per-job reduction is a fixed-order sum over that job's
 // contiguous tile range: deterministic, no atomics.
 //
-// Two lane layouts for R < 64 vectors (both parity-tested):
+// Three lane layouts for R < 64 vectors (all parity-tested):
 //   mode 0 ("row groups"):  64/R rows per wavefront, R lanes per row, entries
 //                           of a row walked sequentially by its lanes (4 and 8 real
 //                           FP64 vectors: 16 lanes per row);

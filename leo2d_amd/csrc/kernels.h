@@ -40,7 +40,7 @@ struct StepArgs {
                     // (FP64, R <= 8), 14 = vector chunks split
                     // over the XCDs (R = 16, 32, 64, 128), 15 = two rows per wavefront, 16-byte FP32 gathers
                     // (complex FP32, R = 64)
-    int long_rows;  // variant 2: 1 = a wavefront per row (rows of more than 64 entries on average)
+    int long_rows;  // variant 2: 1 = a wavefront per row instead of 16 lanes
     int xcd_rows;   // variant 1: rows per XCD slice (0 = interleave rows over the grid)
 };
 
